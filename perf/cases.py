@@ -1,5 +1,5 @@
 """The workloads this framework's speed is measured on: dense LU solves, re-solves with resident
-factors, mixed-precision solves, batches of small systems, SimpleGMRES and the serving loop, each
+factors, mixed-precision solves, batches of small systems and SimpleGMRES, each
 called as a program calls it (the LinearProblem / init / solve_ interface, or the C entry points
 of include/lsx.h on device arrays) with the handles such a program keeps.
 
@@ -59,8 +59,6 @@ def listed():
         dict(name="gmres_1024", kind="gmres", m=1024, pe=5.0, memory=30, restart=True, maxiters=300),
         # one GMRES per diagonal block
         dict(name="gmres_batched_4096", kind="gmres_batched", blocks=4096, m=16, memory=20),
-        # the serving loop on a burst of mixed requests
-        dict(name="serve_burst", kind="serve", dense=40, gmres=6, nmin=16, nmax=2048, mmin=64, mmax=128),
     ]
 
 
@@ -69,8 +67,7 @@ def _logint(rng, lo, hi):
 
 
 def draw(rng):
-    kind = rng.choice(["lu", "lu", "lu", "resolve", "mixed", "batch", "batch", "gmres", "gmres", "gmres_batched",
-                       "serve"])
+    kind = rng.choice(["lu", "lu", "lu", "resolve", "mixed", "batch", "batch", "gmres", "gmres", "gmres_batched"])
     if kind == "lu":
         return dict(kind=kind, n=_logint(rng, 16, 12000), nrhs=rng.choice([1, 1, 3, 16, 37]), order=rng.choice("CF"))
     if kind == "resolve":
@@ -86,10 +83,7 @@ def draw(rng):
         m = _logint(rng, 16, 900 if restart else 300)
         return dict(kind=kind, m=m, pe=round(rng.uniform(0.0, 10.0), 2), memory=rng.choice([10, 20, 30, 50]),
                     restart=restart, maxiters=rng.choice([60, 150, 300] if restart else [40, 100, 150]))
-    if kind == "gmres_batched":
-        return dict(kind=kind, blocks=_logint(rng, 50, 5000), m=rng.randint(4, 20), memory=rng.choice([10, 20, 30]))
-    return dict(kind=kind, dense=rng.randint(8, 48), gmres=rng.randint(0, 6), nmin=16, nmax=rng.choice([512, 2048]),
-                mmin=32, mmax=100)
+    return dict(kind=kind, blocks=_logint(rng, 50, 5000), m=rng.randint(4, 20), memory=rng.choice([10, 20, 30]))
 
 
 # ---- inputs --------------------------------------------------------------------------------------
@@ -178,22 +172,6 @@ def _blocks_csr(case):
     return rowptr, col, vals
 
 
-def _serve_requests(case, seed):
-    shape = np.random.default_rng([case["dense"], case["gmres"], case["nmax"], case["mmax"]])
-    g = np.random.default_rng([seed, 7])
-    reqs = []
-    for _ in range(case["dense"]):
-        n = int(round(math.exp(shape.uniform(math.log(case["nmin"]), math.log(case["nmax"])))))
-        A = g.standard_normal((n, n)) / math.sqrt(n)
-        A[g.permutation(n), np.arange(n)] += 1.25
-        reqs.append(("dense", np.asfortranarray(A), g.standard_normal(n)))
-    for _ in range(case["gmres"]):
-        m, pe = int(shape.integers(case["mmin"], case["mmax"] + 1)), float(round(shape.uniform(0.0, 10.0), 2))
-        reqs.append(("gmres", (m, pe), g.standard_normal(m * m)))
-    order = shape.permutation(len(reqs))
-    return [reqs[i] for i in order]
-
-
 # ---- the framework's handles ---------------------------------------------------------------------
 
 class _Csr:
@@ -234,16 +212,6 @@ class _Batch:
             self.L.lsx_batch_destroy(self.h)
 
 
-class _Served:
-    """A running server; closed with the state."""
-
-    def __init__(self):
-        self.server = _package().Server(hbm_budget=4 << 30)
-
-    def __del__(self):
-        self.server.close()
-
-
 def prepare(case, seed):
     lsx, kind = _package(), case["kind"]
     if kind in ("lu", "mixed", "resolve"):
@@ -270,19 +238,10 @@ def prepare(case, seed):
         return dict(kind=kind, case=case, h=_Csr(rowptr, col, vals), b=_rhs(N, 1, seed),
                     x=torch.empty(N, dtype=torch.float64, device=DEV),
                     pl=torch.full((N,), 4.0, dtype=torch.float64, device=DEV), st=lsx._abi.GmresStats())
-    if kind == "gmres_batched":
-        N = case["m"] ** 2 * case["blocks"]
-        return dict(kind=kind, case=case, h=_Csr(*_blocks_csr(case)), b=_rhs(N, 1, seed),
-                    x=torch.empty(N, dtype=torch.float64, device=DEV),
-                    pl=torch.full((N,), 4.0, dtype=torch.float64, device=DEV), st=lsx._abi.GmresStats())
-    reqs = []
-    for what, data, b in _serve_requests(case, seed):
-        if what == "gmres":
-            m, pe = data
-            rp, ci, v = (t.cpu().numpy() for t in _stencil(m, pe))
-            data = lsx.CSRMatrix(rp, ci, v, (m * m, m * m))
-        reqs.append((what, data, b))
-    return dict(kind=kind, server=_Served(), reqs=reqs)
+    N = case["m"] ** 2 * case["blocks"]
+    return dict(kind=kind, case=case, h=_Csr(*_blocks_csr(case)), b=_rhs(N, 1, seed),
+                x=torch.empty(N, dtype=torch.float64, device=DEV),
+                pl=torch.full((N,), 4.0, dtype=torch.float64, device=DEV), st=lsx._abi.GmresStats())
 
 
 def run(s):
@@ -312,24 +271,12 @@ def run(s):
                                         ABSTOL, 1e-8, c["maxiters"], s["pl"].data_ptr(), None,
                                         ctypes.byref(s["st"])), "lsx_gmres_solve")
         return {"x": s["x"], "iters": int(s["st"].iters), "retcode": int(s["st"].retcode)}
-    if kind == "gmres_batched":
-        c = s["case"]
-        torch.cuda.current_stream().synchronize()
-        h.ctx.check(h.L.lsx_gmres_solve_batched(h.h, c["m"] ** 2, s["b"].data_ptr(), s["x"].data_ptr(), c["memory"], 1,
-                                                ABSTOL, 1e-8, 1000, s["pl"].data_ptr(), None, ctypes.byref(s["st"])),
-                    "lsx_gmres_solve_batched")
-        return {"x": s["x"], "iters": int(s["st"].iters), "retcode": int(s["st"].retcode)}
-    srv = s["server"].server
-    tickets = []
-    for what, data, b in s["reqs"]:
-        if what == "dense":
-            tickets.append(srv.submit_dense(data, b))
-        else:
-            tickets.append(srv.submit_gmres(data, b, pl=np.full(b.shape, 4.0), memory=30, reltol=1e-8))
-    srv.drain()
-    got = [srv.poll(t) for t in tickets]
-    return {"x": np.concatenate([r["x"] for r in got]), "retcode": np.array([int(r["retcode"]) for r in got]),
-            "iters": np.array([int(r["iters"]) for r in got])}
+    c = s["case"]
+    torch.cuda.current_stream().synchronize()
+    h.ctx.check(h.L.lsx_gmres_solve_batched(h.h, c["m"] ** 2, s["b"].data_ptr(), s["x"].data_ptr(), c["memory"], 1,
+                                            ABSTOL, 1e-8, 1000, s["pl"].data_ptr(), None, ctypes.byref(s["st"])),
+                "lsx_gmres_solve_batched")
+    return {"x": s["x"], "iters": int(s["st"].iters), "retcode": int(s["st"].retcode)}
 
 
 # ---- what a pass cannot do without ---------------------------------------------------------------
@@ -361,22 +308,9 @@ def work(case):
         steps = min(case["maxiters"], 8 * case["m"])  # small grids stop at their tolerance
         b, f = _gmres_work(N, 5 * N, steps, memory)
         return {"bytes": b, "flops": f}
-    if kind == "gmres_batched":
-        N = case["m"] ** 2 * case["blocks"]
-        b, f = _gmres_work(N, 5 * N, 4 * case["m"], case["memory"])
-        return {"bytes": b, "flops": f}
-    by = fl = 0.0
-    for what, data, _ in _serve_shapes(case):
-        if what == "dense":
-            by, fl = by + 8 * (data * data + 2 * data), fl + _luflop(data) + 2.0 * data * data
-        else:
-            b, f = _gmres_work(data * data, 5 * data * data, 8 * data, 30)
-            by, fl = by + b, fl + f
-    return {"bytes": by, "flops": fl}
-
-
-def _serve_shapes(case):
-    return [(w, d.shape[0] if w == "dense" else d[0], len(b)) for w, d, b in _serve_requests(case, 0)]
+    N = case["m"] ** 2 * case["blocks"]
+    b, f = _gmres_work(N, 5 * N, 4 * case["m"], case["memory"])
+    return {"bytes": b, "flops": f}
 
 
 # ---- the same results in 64 bits by plain torch and numpy ----------------------------------------
@@ -476,17 +410,8 @@ def exact(case, seed):
         b = _rhs(case["m"] ** 2, 1, seed)
         x = _plain_gmres(b[None, :], case["m"], [case["pe"]], case["memory"], case["restart"], case["maxiters"])
         return {"x": x[0], "iters": None, "retcode": None}
-    if kind == "gmres_batched":
-        n, nb = case["m"] ** 2, case["blocks"]
-        b = _rhs(n * nb, 1, seed)
-        eps = ABSTOL + 1e-8 * float((b / 4.0).norm())
-        x = _plain_gmres(b.reshape(nb, n), case["m"], _block_pe(case), case["memory"], True, 1000, eps)
-        return {"x": x.reshape(-1), "iters": None, "retcode": None}
-    out = []
-    for what, data, b in _serve_requests(case, seed):
-        if what == "dense":
-            out.append(np.linalg.solve(data, b))
-        else:
-            t = torch.from_numpy(b).to(DEV)
-            out.append(_plain_gmres(t[None, :], data[0], [data[1]], 30, True, b.shape[0])[0].cpu().numpy())
-    return {"x": np.concatenate(out), "retcode": None, "iters": None}
+    n, nb = case["m"] ** 2, case["blocks"]
+    b = _rhs(n * nb, 1, seed)
+    eps = ABSTOL + 1e-8 * float((b / 4.0).norm())
+    x = _plain_gmres(b.reshape(nb, n), case["m"], _block_pe(case), case["memory"], True, 1000, eps)
+    return {"x": x.reshape(-1), "iters": None, "retcode": None}

@@ -1,460 +1,20 @@
-// gmres.hip — SimpleGMRES (restarted GMRES, modified Gram-Schmidt Arnoldi, symmetric Givens)
-// on a CSR matrix, one persistent kernel per solve.
-//
-// Follows src/simplegmres.jl (scalar layout) step for step:
-//   reinit / _init_cacheval (:110-129, :420-462): x = 0, r0 = Pl \ b, beta = ||r0||,
-//     eps = abstol + reltol * beta;
-//   outer restart loop (:500-601): on passes >= 2, w = b - A x, r0 = Pl \ w;
-//   Arnoldi step (:521-574): q = Pl \ (A (Pr \ v_k)); MGS h_i = <v_i, q>, q -= h_i v_i (i = 1..k);
-//     Hbis = ||q||; previous Givens applied to the new column, new Givens (_sym_givens
-//     :140-162); zeta update; stopping tests rNorm <= eps, rNorm + 1 <= 1, Hbis <= eps^(3/4);
-//     v_{k+1} = q / Hbis;
-//   back-substitution R y = z with zero for |R_ii| <= btol (:576-585), x_r += sum y_i v_i,
-//     x_r = Pr \ x_r, x += x_r (:587-595); retcodes (:603-606).
-//
-// Layout: workgroup w of P owns rows [w R, (w+1) R), R = GBS * RPT (GBS = 512 threads); thread
-// t holds rows w R + t + i GBS (i < RPT) of q and of the current basis vector in LDS.  Every
-// workgroup keeps its own copy of the Hessenberg/Givens scalars (R, c, s, z) in LDS and
-// computes them identically from all-reduced values, so all workgroups take the same branches.
-// All-reduces combine per-workgroup partial sums in a fixed order (deterministic, the same
-// result in every workgroup) through flag-in-word messages; basis vectors written by one
-// workgroup and read by the SpMV of another are ordered by a counter barrier with agent-scope
-// release/acquire fences.
+// gmres.hip — SimpleGMRES (restarted GMRES, modified Gram-Schmidt Arnoldi, symmetric Givens) on a
+// CSR matrix: the launches of the persistent kernel (gmres_kernel.hpp) for one solve, for several
+// solves at once and for block-diagonal matrices, and their C entry points.
 #include <algorithm>
-#include <cfloat>
 #include <new>
 #include <vector>
-#include <cmath>
 
-#include "gmres.hpp"
+#include "gmres_kernel.hpp"
 
 namespace lsx {
 
-constexpr int GBS = 512;            // threads per workgroup
-constexpr int GNW = GBS / 64;
-constexpr int GLEAD = 16;           // from this many workgroups on, all-reduces go through workgroup 0
-
-struct GShared {
-    double wsum[2][GNW];
-    double lsum[2][GNW];        // workgroup 0 from GLEAD workgroups on: wave sums of the partials
-    uint32_t rbuf[2][2 * 256];  // 2 words per workgroup, up to 256 workgroups
-    int abort;                  // a wait of this solve gave up: leave the solve
-};
-
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
-}
-
-template <int RPT>
-struct GmresCtx {
-    const GmresArgs& a;
-    GShared& sh;
-    int tid, lane, wave, w;
-    int64_t row0;     // first row of this workgroup
-    uint32_t nred = 0, nbar = 0;
-    bool dead = false;  // a wait of this solve gave up (uniform in the workgroup): its results
-                        // are invalid and every loop of the solve ends
-
-    __device__ GmresCtx(const GmresArgs& a_, GShared& sh_, int w_) : a(a_), sh(sh_) {
-        tid = threadIdx.x;
-        lane = tid & 63;
-        wave = tid >> 6;
-        w = w_;
-        row0 = (int64_t)w * GBS * RPT;
-    }
-    __device__ int64_t row(int i) const { return row0 + tid + (int64_t)i * GBS; }
-
-    // Sum of v over all threads of all workgroups, identical in every thread.
-    __device__ double allreduce(double v) {
-        const int par = (int)(nred & 1);
-        ++nred;
-        v = wave_sum(v);
-        if (lane == 0) sh.wsum[par][wave] = v;
-        __syncthreads();
-        double s = 0.0;
-#pragma unroll
-        for (int i = 0; i < GNW; ++i) s += sh.wsum[par][i];
-        if (a.P == 1) return s;
-        const uint32_t seq = nred;
-        uint64_t* slot = a.red + (size_t)par * a.P * 2;
-        if (tid == 0) {
-            st_relaxed_u64(slot + 2 * w, ll_pack((uint32_t)__double2loint(s), seq));
-            st_relaxed_u64(slot + 2 * w + 1, ll_pack((uint32_t)__double2hiint(s), seq));
-        }
-        // Small P: every workgroup reads all P partials and sums them in order.  From GLEAD
-        // workgroups on, workgroup 0 alone reads them (thread p reads partial p), sums them by a
-        // fixed tree (wave sums, then the waves in order) and publishes the total, so the others
-        // poll two words instead of 2P (the polling traffic grows as P^2 otherwise).
-        const bool lead = a.P >= GLEAD;
-        if (!lead) {
-            if (tid < 2 * a.P) sh.rbuf[par][tid] = poll(slot + tid, seq);
-            __syncthreads();
-            dead = sh.abort != 0;
-            double tot = 0.0;
-            for (int p = 0; p < a.P; ++p)
-                tot += __hiloint2double((int)sh.rbuf[par][2 * p + 1], (int)sh.rbuf[par][2 * p]);
-            return tot;
-        }
-        if (w == 0) {
-            double pv = 0.0;
-            if (tid < a.P) {
-                const uint32_t lo = poll(slot + 2 * tid, seq), hi = poll(slot + 2 * tid + 1, seq);
-                pv = __hiloint2double((int)hi, (int)lo);
-            }
-            pv = wave_sum(pv);
-            if (lane == 0) sh.lsum[par][wave] = pv;
-            __syncthreads();
-            dead = sh.abort != 0;
-            double tot = 0.0;
-#pragma unroll
-            for (int i = 0; i < GNW; ++i) tot += sh.lsum[par][i];
-            if (tid == 0) {
-                uint64_t* res = a.red + 4 * (int64_t)a.P + 8 + 2 * par;
-                st_relaxed_u64(res, ll_pack((uint32_t)__double2loint(tot), seq));
-                st_relaxed_u64(res + 1, ll_pack((uint32_t)__double2hiint(tot), seq));
-            }
-            return tot;
-        }
-        if (tid < 2) sh.rbuf[par][tid] = poll(a.red + 4 * (int64_t)a.P + 8 + 2 * par + tid, seq);
-        __syncthreads();
-        dead = sh.abort != 0;
-        return __hiloint2double((int)sh.rbuf[par][1], (int)sh.rbuf[par][0]);
-    }
-
-    // Payload of a flag-in-word message once it carries sequence number seq.  The wait ends at
-    // the bound, or at once when any wait of this solve has given up (the solve's error word is
-    // set); either way the workgroup's abort flag is raised, read after the caller's barrier.
-    __device__ uint32_t poll(const uint64_t* word, uint32_t seq) const {
-        uint64_t x = ld_relaxed_u64(word);
-        if ((uint32_t)(x >> 32) != seq) {
-            const int64_t t0 = wall_clock64();
-            while (true) {
-                x = ld_relaxed_u64(word);
-                if ((uint32_t)(x >> 32) == seq) break;
-                if (wall_clock64() - t0 > a.timeout) {
-                    atomicOr((unsigned long long*)&a.out->err, 1ull);
-                    sh.abort = 1;
-                    break;
-                }
-                if (ld_relaxed_u64(&a.out->err) != 0) {
-                    sh.abort = 1;
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(1);  // back off: many workgroups poll the same words
-            }
-        }
-        return (uint32_t)x;
-    }
-
-    // Orders this workgroup's global writes before every workgroup's later reads.
-    __device__ void barrier() {
-        if (a.P == 1) {
-            __syncthreads();
-            return;
-        }
-        ++nbar;
-        __threadfence();
-        __syncthreads();
-        if (tid == 0) {
-            __hip_atomic_fetch_add(a.bar, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-            const uint32_t target = nbar * (uint32_t)a.P;
-            if (__hip_atomic_load(a.bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-                const int64_t t0 = wall_clock64();
-                while (__hip_atomic_load(a.bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-                    if (wall_clock64() - t0 > a.timeout) {
-                        atomicOr((unsigned long long*)&a.out->err, 2ull);
-                        sh.abort = 1;
-                        break;
-                    }
-                    if (ld_relaxed_u64(&a.out->err) != 0) {
-                        sh.abort = 1;
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(1);
-                }
-            }
-            __atomic_thread_fence(__ATOMIC_ACQUIRE);
-        }
-        __syncthreads();
-        dead = sh.abort != 0;
-    }
-
-    // y_r = (A (v ./ pr))_r, terms summed in ascending column order without fusion (the order
-    // in which SparseArrays' CSC mul! accumulates a row).
-    __device__ double spmv_row(int64_t r, const double* v) const {
-        const int32_t k0 = a.rowptr[r], k1 = a.rowptr[r + 1];
-        double s = 0.0;
-        for (int32_t k = k0; k < k1; ++k) {
-            const int32_t j = a.col[k];
-            double xv = v[j];
-            if (a.pr) xv = xv / a.pr[j];
-            s = __dadd_rn(s, __dmul_rn(a.val[k], xv));
-        }
-        return s;
-    }
-};
-
-__device__ void sym_givens(double a, double b, double& c, double& s, double& rho) {
-    auto sgn = [](double t) { return t > 0.0 ? 1.0 : (t < 0.0 ? -1.0 : 0.0); };
-    if (b == 0.0) {
-        c = (a == 0.0) ? 1.0 : sgn(a);
-        s = 0.0;
-        rho = fabs(a);
-    } else if (a == 0.0) {
-        c = 0.0;
-        s = sgn(b);
-        rho = fabs(b);
-    } else if (fabs(b) > fabs(a)) {
-        const double t = a / b;
-        s = sgn(b) / sqrt(1.0 + t * t);
-        c = s * t;
-        rho = b / s;
-    } else {
-        const double t = b / a;
-        c = sgn(a) / sqrt(1.0 + t * t);
-        s = c * t;
-        rho = a / c;
-    }
-}
-
-// The solve on workgroup w of a.P (sh, dyn: the workgroup's static and dynamic LDS).  RG: the
-// bookkeeping is in HBM (a.Rg) instead of LDS; a compile-time choice, so that each pointer below
-// is known to be LDS or global memory and gets that memory's instructions.
-template <int RPT, bool RG>
-__device__ __forceinline__ void gmres_body(const GmresArgs& a, int w, GShared& sh, double* dyn) {
-    const int cap = a.cap;
-    // the bookkeeping, read and written by thread 0 (z also by every thread after a barrier): in
-    // LDS, or in this workgroup's HBM area when the Krylov dimension is too large for the LDS
-    double* R = RG ? a.Rg + (size_t)w * (size_t)gmres_book_words(cap) : dyn;  // cap (cap + 1) / 2
-    double* cs = R + ((size_t)cap * (cap + 1)) / 2;  // cap
-    double* sn = cs + cap;                    // cap
-    double* z = sn + cap;                     // cap + 1
-    // q and the current basis slice, one LDS column per thread (each thread touches only its own
-    // slots, so no synchronization is needed for them)
-    double* qs = dyn + (RG ? 0 : gmres_book_words(cap));  // RPT x GBS
-    double* vs = qs + RPT * GBS;              // RPT x GBS
-    __shared__ int s_flags[4];
-    GmresCtx<RPT> g(a, sh, w);
-    if (g.tid == 0) sh.abort = 0;  // ordered before any poll by the first all-reduce's barrier
-    const int64_t N = a.N;
-    const int tid = g.tid;
-    double* x = a.x;
-    double* xr = a.restart ? a.xr : a.x;
-#define q(i) qs[(i) * GBS + tid]
-#define vk(i) vs[(i) * GBS + tid]
-
-    // x = 0; r0 = Pl \ b
-    double part = 0.0;
-#pragma unroll 2
-    for (int i = 0; i < RPT; ++i) {
-        const int64_t r = g.row(i);
-        q(i) = 0.0;
-        if (r < N) {
-            x[r] = 0.0;
-            q(i) = a.pl ? a.b[r] / a.pl[r] : a.b[r];
-            part += q(i) * q(i);
-        }
-    }
-    const double beta0 = sqrt(g.allreduce(part));
-    const double eps_ = a.abstol + a.reltol * beta0;
-    double rNorm = beta0;
-    int64_t iter = 0;
-    int status = LSX_RET_DEFAULT;
-    if (g.dead) {
-        // a wait gave up: the error word tells the host, nothing else is computed
-    } else if (beta0 == 0.0) {
-        status = LSX_RET_SUCCESS;
-    } else {
-        int npass = 0;
-        const double btol = pow(DBL_EPSILON, 0.75);
-        bool breakdown = false, inconsistent = false;
-        bool solved = rNorm <= eps_;
-        int64_t inner_maxiters = a.maxiters;
-        bool tired = iter >= a.maxiters;
-        while (!(solved || tired || breakdown || g.dead)) {
-            int64_t nr = 0;
-            if (a.restart) {
-#pragma unroll 2
-                for (int i = 0; i < RPT; ++i) {
-                    const int64_t r = g.row(i);
-                    if (r < N) xr[r] = 0.0;
-                }
-                if (npass >= 1) {
-                    g.barrier();  // x complete in every workgroup before the SpMV reads it
-#pragma unroll 2
-                    for (int i = 0; i < RPT; ++i) {
-                        const int64_t r = g.row(i);
-                        if (r < N) {
-                            double Ax = 0.0;
-                            const int32_t k0 = a.rowptr[r], k1 = a.rowptr[r + 1];
-                            for (int32_t k = k0; k < k1; ++k) Ax = __dadd_rn(Ax, __dmul_rn(a.val[k], x[a.col[k]]));
-                            const double wv = a.b[r] - Ax;
-                            q(i) = a.pl ? wv / a.pl[r] : wv;
-                        }
-                    }
-                }
-            }
-            // zeta_1 = ||r0||, v_1 = r0 / ||r0||
-            part = 0.0;
-#pragma unroll 2
-            for (int i = 0; i < RPT; ++i) part += (g.row(i) < N) ? q(i) * q(i) : 0.0;
-            const double b0 = sqrt(g.allreduce(part));
-            if (tid == 0) z[0] = b0;
-#pragma unroll 2
-            for (int i = 0; i < RPT; ++i) {
-                const int64_t r = g.row(i);
-                if (r < N) a.V[r] = q(i) / b0;
-            }
-            g.barrier();
-            ++npass;
-            int k = 0;
-            bool inner_tired = false;
-            while (!(solved || inner_tired || breakdown || g.dead)) {
-                ++k;
-                const double* vcur = a.V + (int64_t)(k - 1) * N;
-                // q = Pl \ (A (Pr \ v_k))
-#pragma unroll 2
-                for (int i = 0; i < RPT; ++i) {
-                    const int64_t r = g.row(i);
-                    q(i) = 0.0;
-                    if (r < N) {
-                        const double wv = g.spmv_row(r, vcur);
-                        q(i) = a.pl ? wv / a.pl[r] : wv;
-                    }
-                }
-                // modified Gram-Schmidt, the axpy of basis vector i fused with the dot of i + 1;
-                // the rows of the next basis vector are loaded while the all-reduce travels
-                double h = 0.0;
-                double pre[RPT];
-#pragma unroll
-                for (int i = 0; i < RPT; ++i) {
-                    const int64_t r = g.row(i);
-                    pre[i] = (r < N) ? a.V[r] : 0.0;
-                }
-                for (int ii = 1; ii <= k + 1; ++ii) {
-                    part = 0.0;
-#pragma unroll
-                    for (int i = 0; i < RPT; ++i) {
-                        const int64_t r = g.row(i);
-                        if (r < N) {
-                            if (ii > 1) q(i) = q(i) - h * vk(i);
-                            if (ii <= k) {
-                                vk(i) = pre[i];
-                                part += vk(i) * q(i);
-                            } else {
-                                part += q(i) * q(i);
-                            }
-                        }
-                    }
-                    if (ii < k) {
-                        const double* vn = a.V + (int64_t)ii * N;
-#pragma unroll
-                        for (int i = 0; i < RPT; ++i) {
-                            const int64_t r = g.row(i);
-                            pre[i] = (r < N) ? vn[r] : 0.0;
-                        }
-                    }
-                    const double red = g.allreduce(part);
-                    if (g.dead) break;
-                    if (ii <= k) {
-                        h = red;
-                        if (tid == 0) R[nr + ii - 1] = h;
-                    } else {
-                        h = sqrt(red);  // Hbis
-                    }
-                }
-                const double Hbis = h;
-                if (tid == 0) {
-                    for (int i = 1; i <= k - 1; ++i) {
-                        const double Rtmp = cs[i - 1] * R[nr + i - 1] + sn[i - 1] * R[nr + i];
-                        R[nr + i] = sn[i - 1] * R[nr + i - 1] - cs[i - 1] * R[nr + i];
-                        R[nr + i - 1] = Rtmp;
-                    }
-                    double c_, s_, rho;
-                    sym_givens(R[nr + k - 1], Hbis, c_, s_, rho);
-                    cs[k - 1] = c_;
-                    sn[k - 1] = s_;
-                    R[nr + k - 1] = rho;
-                    const double zeta = s_ * z[k - 1];
-                    z[k - 1] = c_ * z[k - 1];
-                    z[k] = zeta;  // consumed only if the iteration continues
-                }
-                __syncthreads();
-                rNorm = fabs(z[k]);
-                nr += k;
-                const bool mach = (rNorm + 1.0 <= 1.0);
-                const bool lim = rNorm <= eps_;
-                breakdown = Hbis <= btol;
-                solved = lim || mach;
-                inner_tired = a.restart ? (k >= (int64_t)min((int64_t)a.memory, inner_maxiters))
-                                        : (k >= inner_maxiters);
-                if (!(solved || inner_tired || breakdown)) {
-                    double* vn = a.V + (int64_t)k * N;
-#pragma unroll 2
-                    for (int i = 0; i < RPT; ++i) {
-                        const int64_t r = g.row(i);
-                        if (r < N) vn[r] = q(i) / Hbis;
-                    }
-                    g.barrier();
-                }
-            }
-            // back-substitution R y = z (y overwrites z)
-            if (tid == 0) {
-                int inc = 0;
-                for (int i = k; i >= 1; --i) {
-                    int64_t pos = nr + i - k;
-                    for (int j = k; j >= i + 1; --j) {
-                        z[i - 1] = z[i - 1] - R[pos - 1] * z[j - 1];
-                        pos = pos - j + 1;
-                    }
-                    if (fabs(R[pos - 1]) <= btol) {
-                        z[i - 1] = 0.0;
-                        inc = 1;
-                    } else {
-                        z[i - 1] = z[i - 1] / R[pos - 1];
-                    }
-                }
-                s_flags[0] = inc;
-            }
-            __syncthreads();
-            inconsistent = inconsistent || s_flags[0];
-            // x_r += sum_i y_i v_i; x_r = Pr \ x_r; x += x_r
-#pragma unroll 2
-            for (int i = 0; i < RPT; ++i) {
-                const int64_t r = g.row(i);
-                if (r < N) {
-                    double acc = xr[r];
-                    for (int ii = 0; ii < k; ++ii) acc = acc + z[ii] * a.V[(int64_t)ii * N + r];
-                    if (a.pr) acc = acc / a.pr[r];
-                    if (a.restart) x[r] = x[r] + acc;
-                    else xr[r] = acc;
-                }
-            }
-            inner_maxiters -= k;
-            iter += k;
-            tired = iter >= a.maxiters;
-            __syncthreads();
-        }
-        if (tired) status = LSX_RET_MAXITERS;
-        if (solved) status = LSX_RET_SUCCESS;
-        if (inconsistent) status = LSX_RET_INFEASIBLE;
-    }
-#undef q
-#undef vk
-    if (g.w == 0 && tid == 0) {
-        a.out->retcode = status;
-        a.out->iters = iter;
-        a.out->resid = rNorm;
-    }
-}
-
-template <int RPT, bool RG>
-__global__ __launch_bounds__(GBS) void k_gmres(GmresArgs a) {
-    __shared__ GShared sh;
-    extern __shared__ double dyn[];
-    gmres_body<RPT, RG>(a, (int)blockIdx.x, sh, dyn);
+template <int NT, int RPT, bool RG>
+__global__ __launch_bounds__(NT, NT == 1024 ? 4 : (NT == 256 ? 3 : 2)) void k_gmres(GmresArgs a) {
+    __shared__ GShared<NT> sh;
+    extern __shared__ __align__(16) double dyn[];
+    GmresWg<NT, RPT, RG> g(a, sh, (int)blockIdx.x, dyn);
+    g.run();
 }
 
 // Several solves in one launch (gmres_launch_multi), on a pool of workgroups that may be smaller
@@ -463,12 +23,13 @@ __global__ __launch_bounds__(GBS) void k_gmres(GmresArgs a) {
 // every solve but the one holding the highest number handed out so far has all its ranks
 // running and finishes by itself; with at least as many workgroups as the widest solve, that
 // last one fills up as the others end.
-template <int RPT>
-__global__ __launch_bounds__(GBS) void k_gmres_multi(const GmresArgs* __restrict items, const int* __restrict first,
-                                                     int nitems, uint32_t* ticket) {
-    __shared__ GShared sh;
+template <int NT, int RPT>
+__global__ __launch_bounds__(NT, NT == 1024 ? 4 : (NT == 256 ? 3 : 2)) void k_gmres_multi(const GmresArgs* __restrict items,
+                                                                       const int* __restrict first, int nitems,
+                                                                       uint32_t* ticket) {
+    __shared__ GShared<NT> sh;
     __shared__ int s_id;
-    extern __shared__ double dyn[];
+    extern __shared__ __align__(16) double dyn[];
     const int total = first[nitems];
     while (true) {
         __syncthreads();  // the previous solve's LDS is no longer read
@@ -484,16 +45,19 @@ __global__ __launch_bounds__(GBS) void k_gmres_multi(const GmresArgs* __restrict
         }
         const int item = __builtin_amdgcn_readfirstlane(lo);
         const GmresArgs a = items[item];
-        gmres_body<RPT, false>(a, id - first[item], sh, dyn);
+        GmresWg<NT, RPT, false> g(a, sh, id - first[item], dyn);
+        g.run();
     }
 }
 
 // Zeroes the exchange area and result of every solve of a multi launch, and its ticket counter.
+// (grid.x: the solves, grid.y: shares of an exchange area)
 __global__ void k_gmres_clear(const GmresArgs* __restrict items, uint32_t* ticket) {
     const GmresArgs& a = items[blockIdx.x];
-    const int64_t words = gmres_red_words(a.P);
-    for (int64_t i = threadIdx.x; i < words; i += blockDim.x) a.red[i] = 0ull;
-    if (threadIdx.x == 0) {
+    const int64_t words = gmres_red_words(a.P, a.cap);
+    for (int64_t i = (int64_t)blockIdx.y * blockDim.x + threadIdx.x; i < words; i += (int64_t)gridDim.y * blockDim.x)
+        a.red[i] = 0ull;
+    if (threadIdx.x == 0 && blockIdx.y == 0) {
         a.out->retcode = 0;
         a.out->pad = 0;
         a.out->iters = 0;
@@ -513,29 +77,24 @@ __global__ void k_spmv(int64_t N, const int32_t* __restrict rowptr, const int32_
     y[r] = s;
 }
 
-// Rows per thread for a matrix of N rows: a single workgroup up to 8192 rows, then 16 rows per
-// thread over ceil(N / 8192) workgroups.
-// Rows per thread and workgroups of a solve of N rows: beyond 8192 rows, the smallest of 4, 8, 16
-// rows per thread that keeps the solve within GMRES_WIDE workgroups, so that more CUs stream each
-// basis vector (measured: a 256^2 grid 105 -> 69 us per Arnoldi step with 32 workgroups of 2048
-// rows instead of 8 of 8192).  The bound keeps every solve inside the serving lanes' share of the
-// CUs, so a solve has the same shape, and the same bits, in every launch form.
+// Threads, rows per thread and workgroups of a solve of N rows.  A step's two exchanges cost about
+// the same from a few workgroups to GMRES_WIDE of them, while everything else shrinks with the rows
+// of a workgroup, so a solve takes the fewest rows per thread that keep it within a bound of
+// workgroups.  The bounds grow with the rows: up to GALL workgroups the products take one message
+// round instead of two.  GMRES_WIDE keeps every solve inside the serving lanes' share of the CUs, so
+// a solve has the same shape, and the same bits, in every launch form.
 constexpr int GMRES_WIDE = 128;
-static int pick_rpt(int64_t N, int& P) {
-    if (N > 16 * GBS) {
-        for (int r : {4, 8}) {
-            const int64_t p = cdiv(N, (int64_t)r * GBS);
-            if (p <= GMRES_WIDE) {
-                P = (int)p;
-                return r;
-            }
+static void pick_shape(int64_t N, bool one_wg, GmresPlan* out) {
+    out->nt = N <= 256 ? 256 : 1024;
+    out->rpt = N <= 256 ? 1 : 8;
+    const int bound[4] = {32, 64, GMRES_WIDE, GMRES_WIDE};
+    for (int i = 0; i < 4 && N > 256; ++i)
+        if (cdiv(N, 512 << i) <= (one_wg ? 1 : bound[i])) {
+            out->nt = 512;
+            out->rpt = 1 << i;
+            break;
         }
-    }
-    if (N <= GBS) { P = 1; return 1; }
-    if (N <= 4 * GBS) { P = 1; return 4; }
-    if (N <= 16 * GBS) { P = 1; return 16; }
-    P = (int)cdiv(N, 16 * GBS);
-    return 16;
+    out->P = (int)cdiv(N, (int64_t)out->nt * out->rpt);
 }
 
 int csr_spmv_dev(lsx_csr* A, const double* dx, double* dy, hipStream_t st) {
@@ -544,55 +103,87 @@ int csr_spmv_dev(lsx_csr* A, const double* dx, double* dy, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? LSX_OK : LSX_EHIP;
 }
 
-// Dynamic LDS of a solve: q and the basis slice, and (rglob false) the packed triangle R, the
-// Givens pairs and z.
-static size_t gmres_dynlds(int64_t cap, int rpt, bool rglob) {
-    return sizeof(double) * ((rglob ? 0 : (size_t)gmres_book_words(cap)) + 2 * (size_t)rpt * GBS);
-}
-constexpr size_t GMRES_LDS_MAX = 150 * 1024;
+constexpr size_t GMRES_LDS_MAX = 149 * 1024;  // dynamic LDS of a workgroup (160 KB less the static part)
 
-// The largest Krylov dimension of one solve: GMRES_MAX_CAP_G (bookkeeping in HBM from the LDS
-// bound on); with hbm false (the multi-solve launches) the largest whose bookkeeping fits the LDS
-// of a workgroup of a matrix of N rows.
+// The largest Krylov dimension of one solve: GMRES_MAX_CAP_G (bookkeeping in HBM where the LDS does
+// not hold it); with hbm false (the multi-solve launches) 128, and less for matrices whose
+// workgroups have many rows.
 int gmres_cap_limit(int64_t N, bool hbm) {
     if (hbm) return GMRES_MAX_CAP_G;
-    int P = 1;
-    const int rpt = pick_rpt(N, P);
-    int cap = GMRES_MAX_CAP;
-    while (cap > 1 && gmres_dynlds(cap, rpt, false) > GMRES_LDS_MAX) --cap;
-    return cap;
+    int64_t rows = 8192;  // LDS rows (two doubles each) set aside beside R, the Givens pairs and z
+    if (N <= 512) rows = 512;
+    else if (N <= 2048 || (N > 8192 && cdiv(N, 2048) <= GMRES_WIDE)) rows = 2048;
+    else if (N > 8192 && cdiv(N, 4096) <= GMRES_WIDE) rows = 4096;
+    int64_t cap = GMRES_MAX_CAP;
+    while (cap > 1 && 8 * (cap * (cap + 1) / 2 + 3 * cap + 1 + 2 * rows) > 150 * 1024) --cap;
+    return (int)cap;
 }
 
-int gmres_plan(lsx_ctx* ctx, int64_t N, const GmresParams& p, GmresPlan* out, bool hbm) {
-    int P = 1;
-    const int rpt = pick_rpt(N, P);
-    if (P > PMAX_G) return fail(ctx, LSX_EINVAL, "gmres: N = %lld exceeds %d rows", (long long)N, PMAX_G * 16 * GBS);
+int gmres_plan(lsx_ctx* ctx, int64_t N, const GmresParams& p, GmresPlan* out, bool hbm, bool one_wg) {
+    pick_shape(N, one_wg, out);
+    if (out->P > PMAX_G) return fail(ctx, LSX_EINVAL, "gmres: N = %lld exceeds %d rows", (long long)N, PMAX_G * 8192);
     const int64_t memory = std::max<int64_t>(1, std::min<int64_t>(p.memory, p.maxiters));
     const int64_t cap = p.restart ? memory : std::max<int64_t>(memory, p.maxiters);
     const int lim = gmres_cap_limit(N, hbm);
     if (cap > lim)
         return fail(ctx, LSX_EINVAL, "gmres: Krylov dimension %lld exceeds %d (restart = %d, N = %lld)", (long long)cap,
                     lim, p.restart, (long long)N);
-    const bool rglob = gmres_dynlds(cap, rpt, false) > GMRES_LDS_MAX;
-    out->P = P;
-    out->rpt = rpt;
     out->cap = (int)cap;
-    out->rglob = rglob;
-    out->dynlds = gmres_dynlds(cap, rpt, rglob);
+    // LDS: the bookkeeping and the receive buffer first, then the current vector's own rows, then as
+    // many basis vectors as fit.  The receive buffer holds the products of a 32-vector group from
+    // all workgroups when there is room.
+    const int64_t R = (int64_t)out->nt * out->rpt, words = (int64_t)(GMRES_LDS_MAX / sizeof(double));
+    int64_t left = words - gmres_book_words(cap);
+    const int64_t rmin = out->P == 1 ? 0 : 512;
+    out->rglob = left < rmin;
+    if (out->rglob) left = words;
+    out->own_lds = left - rmin >= R;
+    const int64_t rwant = out->P == 1 || out->P > GALL ? rmin : 64 * (int64_t)GALL;
+    out->rbuf_len = (int)std::max(rmin, std::min(rwant, left - (out->own_lds ? R : 0)) & ~(int64_t)1);
+    left -= out->rbuf_len + (out->own_lds ? R : 0);
+    out->ncache = (int)std::min<int64_t>(cap + 1, left / R);
+    out->dynlds = sizeof(double) * (size_t)((out->rglob ? 0 : gmres_book_words(cap)) + out->rbuf_len +
+                                            (out->own_lds ? R : 0) + out->ncache * R);
     return LSX_OK;
 }
 
+void gmres_plan_args(const GmresPlan& plan, GmresArgs* a) {
+    a->cap = plan.cap;
+    a->P = plan.P;
+    a->ncache = plan.ncache;
+    a->own_lds = plan.own_lds;
+    a->rbuf_len = plan.rbuf_len;
+    a->allread = plan.P > 1 && plan.P <= GALL;
+}
+
 int gmres_launch_multi(lsx_ctx* ctx, hipStream_t st, const GmresArgs* items, const int* first, int nitems,
-                       int pool, int rpt, size_t dynlds, uint32_t* ticket) {
+                       int pool, int cls, size_t dynlds, uint32_t* ticket) {
     if (nitems < 1 || pool < 1) return fail(ctx, LSX_EINVAL, "gmres: empty multi launch");
-    hipLaunchKernelGGL(k_gmres_clear, dim3((unsigned)nitems), dim3(256), 0, st, items, ticket);
-    switch (rpt) {
-        case 1: hipLaunchKernelGGL(k_gmres_multi<1>, dim3(pool), dim3(GBS), dynlds, st, items, first, nitems, ticket); break;
-        case 4: hipLaunchKernelGGL(k_gmres_multi<4>, dim3(pool), dim3(GBS), dynlds, st, items, first, nitems, ticket); break;
-        case 8: hipLaunchKernelGGL(k_gmres_multi<8>, dim3(pool), dim3(GBS), dynlds, st, items, first, nitems, ticket); break;
-        default: hipLaunchKernelGGL(k_gmres_multi<16>, dim3(pool), dim3(GBS), dynlds, st, items, first, nitems, ticket); break;
+    hipLaunchKernelGGL(k_gmres_clear, dim3((unsigned)nitems, nitems <= 64 ? 16 : 1), dim3(256), 0, st, items, ticket);
+    auto go = [&](auto kern, int nt) {
+        hipLaunchKernelGGL(kern, dim3(pool), dim3(nt), dynlds, st, items, first, nitems, ticket);
+    };
+    switch (cls) {
+        case 0: go(k_gmres_multi<256, 1>, 256); break;
+        case 1: go(k_gmres_multi<512, 1>, 512); break;
+        case 2: go(k_gmres_multi<512, 2>, 512); break;
+        case 4: go(k_gmres_multi<512, 4>, 512); break;
+        case 8: go(k_gmres_multi<512, 8>, 512); break;
+        default: go(k_gmres_multi<1024, 8>, 1024); break;
     }
     LSX_HIP(ctx, hipGetLastError());
+    return LSX_OK;
+}
+
+// A device buffer of at least `need` bytes in *p (*have: its size), reallocated when it is smaller.
+static int grow(lsx_ctx* ctx, void** p, size_t* have, size_t need, const char* what) {
+    if (need <= *have) return LSX_OK;
+    (void)hipFree(*p);
+    *p = nullptr;
+    *have = 0;
+    if (hipMalloc(p, need) != hipSuccess)
+        return fail(ctx, LSX_ENOMEM, "gmres: cannot allocate %zu bytes of %s", need, what);
+    *have = need;
     return LSX_OK;
 }
 
@@ -603,31 +194,16 @@ int gmres_launch(lsx_csr* A, const GmresParams& p, const double* db, double* dx,
     GmresPlan plan;
     int rc = gmres_plan(ctx, N, p, &plan, true);
     if (rc) return rc;
-    const int P = plan.P, rpt = plan.rpt;
-    const int64_t memory = std::max<int64_t>(1, std::min<int64_t>(p.memory, p.maxiters));
-    const int64_t cap = plan.cap;
-    // workspace: basis (cap + 1) x N, correction N
-    const size_t need = sizeof(double) * (size_t)N * (size_t)(cap + 2);
-    if (need > A->ws_bytes) {
-        (void)hipFree(A->ws);
-        A->ws = nullptr;
-        A->ws_bytes = 0;
-        if (hipMalloc(&A->ws, need) != hipSuccess)
-            return fail(ctx, LSX_ENOMEM, "gmres: cannot allocate %zu bytes of Krylov workspace", need);
-        A->ws_bytes = need;
-    }
-    if (plan.rglob) {
-        const size_t rneed = sizeof(double) * (size_t)P * (size_t)gmres_book_words(cap);
-        if (rneed > A->rg_bytes) {
-            (void)hipFree(A->rg);
-            A->rg = nullptr;
-            A->rg_bytes = 0;
-            if (hipMalloc(&A->rg, rneed) != hipSuccess)
-                return fail(ctx, LSX_ENOMEM, "gmres: cannot allocate %zu bytes of Krylov bookkeeping", rneed);
-            A->rg_bytes = rneed;
-        }
-    }
-    LSX_HIP(ctx, hipMemsetAsync(A->red, 0, sizeof(uint64_t) * 4 * PMAX_G + 256, st));
+    const int P = plan.P;
+    const int64_t cap = plan.cap, ldv = gmres_ldv(N);
+    if ((rc = grow(ctx, (void**)&A->ws, &A->ws_bytes, sizeof(double) * (size_t)ldv * (size_t)(cap + 2), "Krylov workspace")))
+        return rc;
+    if (plan.rglob && (rc = grow(ctx, (void**)&A->rg, &A->rg_bytes, sizeof(double) * (size_t)P * (size_t)gmres_book_words(cap),
+                                 "Krylov bookkeeping")))
+        return rc;
+    const size_t rb = sizeof(uint64_t) * (size_t)gmres_red_words(P, cap);
+    if ((rc = grow(ctx, (void**)&A->red, &A->red_bytes, rb, "exchange words"))) return rc;
+    if (rb) LSX_HIP(ctx, hipMemsetAsync(A->red, 0, rb, st));
     LSX_HIP(ctx, hipMemsetAsync(A->out, 0, sizeof(GmresOut), st));
     GmresArgs g;
     g.N = N;
@@ -639,37 +215,29 @@ int gmres_launch(lsx_csr* A, const GmresParams& p, const double* db, double* dx,
     g.pl = dpl;
     g.pr = dpr;
     g.V = A->ws;
-    g.xr = A->ws + (size_t)N * (size_t)(cap + 1);
-    g.memory = (int)memory;
+    g.ldv = ldv;
+    g.xp = A->ws + ldv * (cap + 1);
+    g.memory = (int)std::max<int64_t>(1, std::min<int64_t>(p.memory, p.maxiters));
     g.restart = p.restart;
-    g.cap = (int)cap;
+    gmres_plan_args(plan, &g);
     g.Rg = plan.rglob ? A->rg : nullptr;
     g.maxiters = p.maxiters;
     g.abstol = p.abstol;
     g.reltol = p.reltol;
-    g.P = P;
     g.red = A->red;
-    g.bar = reinterpret_cast<uint32_t*>(A->red + 4 * (int64_t)P);
     g.out = A->out;
     g.timeout = wait_ticks(ctx, 20.0);
-    const size_t dynlds = plan.dynlds;
-    switch (rpt) {
-        case 1:
-            if (plan.rglob) hipLaunchKernelGGL((k_gmres<1, true>), dim3(P), dim3(GBS), dynlds, st, g);
-            else hipLaunchKernelGGL((k_gmres<1, false>), dim3(P), dim3(GBS), dynlds, st, g);
-            break;
-        case 4:
-            if (plan.rglob) hipLaunchKernelGGL((k_gmres<4, true>), dim3(P), dim3(GBS), dynlds, st, g);
-            else hipLaunchKernelGGL((k_gmres<4, false>), dim3(P), dim3(GBS), dynlds, st, g);
-            break;
-        case 8:
-            if (plan.rglob) hipLaunchKernelGGL((k_gmres<8, true>), dim3(P), dim3(GBS), dynlds, st, g);
-            else hipLaunchKernelGGL((k_gmres<8, false>), dim3(P), dim3(GBS), dynlds, st, g);
-            break;
-        default:
-            if (plan.rglob) hipLaunchKernelGGL((k_gmres<16, true>), dim3(P), dim3(GBS), dynlds, st, g);
-            else hipLaunchKernelGGL((k_gmres<16, false>), dim3(P), dim3(GBS), dynlds, st, g);
-            break;
+    auto go = [&](auto lds, auto hbm) {
+        if (plan.rglob) hipLaunchKernelGGL(hbm, dim3(P), dim3(plan.nt), plan.dynlds, st, g);
+        else hipLaunchKernelGGL(lds, dim3(P), dim3(plan.nt), plan.dynlds, st, g);
+    };
+    switch (plan.cls()) {
+        case 0: go(k_gmres<256, 1, false>, k_gmres<256, 1, true>); break;
+        case 1: go(k_gmres<512, 1, false>, k_gmres<512, 1, true>); break;
+        case 2: go(k_gmres<512, 2, false>, k_gmres<512, 2, true>); break;
+        case 4: go(k_gmres<512, 4, false>, k_gmres<512, 4, true>); break;
+        case 8: go(k_gmres<512, 8, false>, k_gmres<512, 8, true>); break;
+        default: go(k_gmres<1024, 8, false>, k_gmres<1024, 8, true>); break;
     }
     LSX_HIP(ctx, hipGetLastError());
     return LSX_OK;
@@ -722,7 +290,6 @@ using namespace lsx;
 static void csr_free(lsx_csr* A) {
     if (A->stream) (void)hipStreamSynchronize(A->stream);
     (void)hipFree(A->col_local);
-    (void)hipFree(A->bred);
     (void)hipFree(A->bitems);
     (void)hipFree(A->bfirst);
     (void)hipFree(A->bout);
@@ -808,7 +375,6 @@ int lsx_csr_create(lsx_ctx* ctx, int64_t N, int64_t nnz, const int32_t* rowptr, 
         hipMalloc(&A->rowptr, sizeof(int32_t) * (N + 1)) != hipSuccess ||
         hipMalloc(&A->col, sizeof(int32_t) * std::max<int64_t>(nnz, 1)) != hipSuccess ||
         hipMalloc(&A->val, sizeof(double) * std::max<int64_t>(nnz, 1)) != hipSuccess ||
-        hipMalloc(&A->red, sizeof(uint64_t) * 4 * PMAX_G + 256) != hipSuccess ||
         hipMalloc(&A->out, sizeof(GmresOut)) != hipSuccess ||
         hipHostMalloc(&A->hout, sizeof(GmresOut), hipHostMallocDefault) != hipSuccess ||
         hipMalloc(&A->db, sizeof(double) * N) != hipSuccess || hipMalloc(&A->dx, sizeof(double) * N) != hipSuccess ||
@@ -900,10 +466,10 @@ int lsx_gmres_solve_batched(lsx_csr* A, int64_t blocksize, const double* b, doub
     const int64_t nb = N / blocksize;
     GmresParams p{memory, restart ? 1 : 0, maxiters, 0.0, 0.0};
     GmresPlan plan;
-    int rc = gmres_plan(ctx, blocksize, p, &plan);
+    if (blocksize > 8192)
+        return fail(ctx, LSX_EINVAL, "lsx_gmres_solve_batched: blocks of more than %d rows are not supported", 8192);
+    int rc = gmres_plan(ctx, blocksize, p, &plan, false, true);
     if (rc) return rc;
-    if (plan.P != 1)
-        return fail(ctx, LSX_EINVAL, "lsx_gmres_solve_batched: blocks of more than %d rows are not supported", 16 * GBS);
     const hipStream_t st = A->stream;
     // local columns (once per block size), after checking that A is block diagonal
     if (A->local_bs != blocksize) {
@@ -919,18 +485,14 @@ int lsx_gmres_solve_batched(lsx_csr* A, int64_t blocksize, const double* b, doub
         A->local_bs = blocksize;
     }
     // buffers for nb blocks
-    const int64_t rw = gmres_red_words(1);
     if (nb > A->bcap) {
-        (void)hipFree(A->bred);
         (void)hipFree(A->bitems);
         (void)hipFree(A->bfirst);
         (void)hipFree(A->bout);
-        A->bred = nullptr;
         A->bitems = nullptr;
         A->bfirst = nullptr;
         A->bout = nullptr;
         A->bcap = 0;
-        LSX_HIP(ctx, hipMalloc(&A->bred, sizeof(uint64_t) * rw * nb));
         LSX_HIP(ctx, hipMalloc(&A->bitems, sizeof(GmresArgs) * nb));
         LSX_HIP(ctx, hipMalloc(&A->bfirst, sizeof(int) * (nb + 1)));
         LSX_HIP(ctx, hipMalloc(&A->bout, sizeof(GmresOut) * nb));
@@ -938,15 +500,8 @@ int lsx_gmres_solve_batched(lsx_csr* A, int64_t blocksize, const double* b, doub
         A->bkey[0] = 0;  // new table buffers: rebuild
     }
     if (!A->bticket) LSX_HIP(ctx, hipMalloc(&A->bticket, 256));
-    const size_t need = sizeof(double) * (size_t)N * (size_t)(plan.cap + 2);
-    if (need > A->ws_bytes) {
-        (void)hipFree(A->ws);
-        A->ws = nullptr;
-        A->ws_bytes = 0;
-        if (hipMalloc(&A->ws, need) != hipSuccess)
-            return fail(ctx, LSX_ENOMEM, "gmres: cannot allocate %zu bytes of Krylov workspace", need);
-        A->ws_bytes = need;
-    }
+    const int64_t ldv = gmres_ldv(blocksize), vstride = ldv * (plan.cap + 2);
+    if ((rc = grow(ctx, (void**)&A->ws, &A->ws_bytes, sizeof(double) * (size_t)(vstride * nb), "Krylov workspace"))) return rc;
     if (!A->bpart) LSX_HIP(ctx, hipMalloc(&A->bpart, sizeof(double) * NPART));
     const size_t vb = sizeof(double) * N;
     LSX_HIP(ctx, hipMemcpyAsync(A->db, b, vb, hipMemcpyDefault, st));
@@ -956,7 +511,7 @@ int lsx_gmres_solve_batched(lsx_csr* A, int64_t blocksize, const double* b, doub
     const int64_t memv = std::max<int64_t>(1, std::min<int64_t>(memory, maxiters));
     const int64_t wt = wait_ticks(ctx, 20.0);
     const int64_t key[9] = {blocksize, (pl_diag ? 1 : 0) | (pr_diag ? 2 : 0), memv, restart ? 1 : 0, maxiters,
-                            (int64_t)(uintptr_t)A->ws, (int64_t)(uintptr_t)A->bred, plan.cap, wt};
+                            (int64_t)(uintptr_t)A->ws, (int64_t)(uintptr_t)A->bitems, plan.cap, wt};
     if (!std::equal(key, key + 9, A->bkey)) {
         std::vector<GmresArgs> items(nb);
         std::vector<int> first(nb + 1);
@@ -971,17 +526,16 @@ int lsx_gmres_solve_batched(lsx_csr* A, int64_t blocksize, const double* b, doub
             a.x = A->dx + r0;
             a.pl = pl_diag ? A->dpl + r0 : nullptr;
             a.pr = pr_diag ? A->dpr + r0 : nullptr;
-            a.V = A->ws + r0 * (plan.cap + 2);
-            a.xr = a.V + blocksize * (plan.cap + 1);
+            a.V = A->ws + i * vstride;
+            a.ldv = ldv;
+            a.xp = a.V + ldv * (plan.cap + 1);
             a.memory = (int)memv;
             a.restart = restart ? 1 : 0;
-            a.cap = plan.cap;
+            gmres_plan_args(plan, &a);
             a.maxiters = maxiters;
             a.abstol = 0.0;
             a.reltol = 0.0;
-            a.P = 1;
-            a.red = A->bred + i * rw;
-            a.bar = reinterpret_cast<uint32_t*>(a.red + 4);
+            a.red = nullptr;
             a.out = A->bout + i;
             a.timeout = wt;
             first[i] = (int)i;
@@ -998,7 +552,7 @@ int lsx_gmres_solve_batched(lsx_csr* A, int64_t blocksize, const double* b, doub
     hipLaunchKernelGGL(k_batch_tol, dim3((unsigned)std::min<int64_t>(cdiv(nb, 256), 64)), dim3(256), 0, st, A->bpart,
                        abstol, reltol, A->bitems, nb);
     const int pool = (int)std::min<int64_t>(nb, 4 * (int64_t)ctx->num_cus);
-    rc = gmres_launch_multi(ctx, st, A->bitems, A->bfirst, (int)nb, pool, plan.rpt, plan.dynlds, A->bticket);
+    rc = gmres_launch_multi(ctx, st, A->bitems, A->bfirst, (int)nb, pool, plan.cls(), plan.dynlds, A->bticket);
     if (rc) return rc;
     std::vector<GmresOut> outs(nb);
     LSX_HIP(ctx, hipMemcpyAsync(outs.data(), A->bout, sizeof(GmresOut) * nb, hipMemcpyDeviceToHost, st));

@@ -208,7 +208,6 @@ struct GmresBlock {
     double* pl;
     double* x;
     double* V;
-    double* xr;
     uint64_t* red;
     size_t bytes;
 };
@@ -222,9 +221,8 @@ GmresBlock gmres_block(uintptr_t base, const Job& j) {
     g.b = c.take<double>(j.N);
     g.pl = c.take<double>(j.N);
     g.x = c.take<double>(j.N);
-    g.V = c.take<double>((int64_t)(j.plan.cap + 1) * j.N);
-    g.xr = c.take<double>(j.N);
-    g.red = c.take<uint64_t>(gmres_red_words(j.plan.P));
+    g.V = c.take<double>((int64_t)(j.plan.cap + 1) * gmres_ldv(j.N));
+    g.red = c.take<uint64_t>(gmres_red_words(j.plan.P, j.plan.cap));
     g.bytes = c.p - base;
     return g;
 }
@@ -468,7 +466,7 @@ void dense_worker(lsx_serve* s, int lane) {
 }
 
 // ---- GMRES lanes: multi-solve launches (called with s->mu held).  The front request must fit;
-// later requests of the same rows-per-thread class join while memory and workgroups allow.
+// later requests of the same kernel class join while memory and workgroups allow.
 int take_gmres(lsx_serve* s, std::vector<Job*>& group) {
     auto& q = s->lanes[LANE_GMRES];
     if (q.empty()) return 0;
@@ -486,7 +484,7 @@ int take_gmres(lsx_serve* s, std::vector<Job*>& group) {
     int scanned = 0;
     for (auto it = q.begin(); it != q.end() && (int)group.size() < MAXG && scanned < 512; ++scanned) {
         Job* j = *it;
-        if (j->plan.rpt != f->plan.rpt) {
+        if (j->plan.cls() != f->plan.cls()) {
             ++it;
             continue;
         }
@@ -574,17 +572,16 @@ void run_gmres_group(lsx_serve* s, GmresLane& L, std::vector<Job*>& group) {
         a.pl = has_pl[i] ? g.pl : nullptr;
         a.pr = nullptr;
         a.V = g.V;
-        a.xr = g.xr;
+        a.ldv = gmres_ldv(j->N);
+        a.xp = nullptr;
         a.memory = (int)std::max<int64_t>(1, std::min<int64_t>(r.memory, r.maxiters));
         a.restart = r.restart ? 1 : 0;
-        a.cap = j->plan.cap;
+        gmres_plan_args(j->plan, &a);
         a.Rg = nullptr;  // bookkeeping in LDS (the plan is made without the HBM option)
         a.maxiters = r.maxiters;
         a.abstol = r.abstol;
         a.reltol = r.reltol;
-        a.P = j->plan.P;
         a.red = g.red;
-        a.bar = reinterpret_cast<uint32_t*>(g.red + 4 * (int64_t)j->plan.P);
         a.out = L.d_out + m;
         a.timeout = wait_ticks(ctx, 20.0);
         L.h_first[m] = total;
@@ -600,7 +597,7 @@ void run_gmres_group(lsx_serve* s, GmresLane& L, std::vector<Job*>& group) {
             hipMemcpyAsync(L.d_first, L.h_first, sizeof(int) * (nl + 1), hipMemcpyHostToDevice, st) != hipSuccess)
             rc = LSX_EHIP;
         if (rc == LSX_OK)
-            rc = gmres_launch_multi(ctx, st, L.d_items, L.d_first, nl, pool, group[idx[0]]->plan.rpt, lds, L.d_ticket);
+            rc = gmres_launch_multi(ctx, st, L.d_items, L.d_first, nl, pool, group[idx[0]]->plan.cls(), lds, L.d_ticket);
         if (rc == LSX_OK &&
             hipMemcpyAsync(L.h_out, L.d_out, sizeof(GmresOut) * nl, hipMemcpyDeviceToHost, st) != hipSuccess)
             rc = LSX_EHIP;

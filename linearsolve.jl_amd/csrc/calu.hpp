@@ -75,26 +75,6 @@ __device__ __forceinline__ uint32_t calu_key(float x, uint32_t idx) {
     const uint32_t b = t == t ? __float_as_uint(t) : 0u;
     return (((b >> IB) + 1u) << IB) | ((1u << IB) - 1u - idx);
 }
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
-    uint32_t y;
-    y = dpp32<0xB1>(x);  x = y > x ? y : x;   // lane ^ 1
-    y = dpp32<0x4E>(x);  x = y > x ? y : x;   // lane ^ 2
-    y = dpp32<0x141>(x); x = y > x ? y : x;   // the two quads of each 8
-    y = dpp32<0x140>(x); x = y > x ? y : x;   // the two halves of each 16
-    y = xrow16(x);       x = y > x ? y : x;
-    y = xrow32(x);       x = y > x ? y : x;
-    return x;
-}
-// f(integral_constant<int, I>) for I = 0 .. N-1, each call with its index a compile-time constant
-// (a loop whose steps index register arrays, too long for the unroller).
-template <int I, int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
-}
-
 // Values C .. CW-1 of a 16-byte aligned row in LDS, read as the 16-byte words that hold them.
 template <int C>
 __device__ __forceinline__ void load_row(const float* row, float (&r)[CW]) {

@@ -12,7 +12,7 @@
 namespace lsx {
 
 template <typename T>
-static void launch_panel_t(lsx_lu* lu, T* F, int64_t ld, int64_t j0, int W) {
+static void launch_panel_t(lsx_lu* lu, T* F, int64_t ld, int64_t j0, int W, int64_t* list, int* count) {
     const int64_t m_rows = lu->n - j0;
     PanelArgs<T> a;
     a.A = F;
@@ -25,16 +25,18 @@ static void launch_panel_t(lsx_lu* lu, T* F, int64_t ld, int64_t j0, int W) {
     a.slots = lu->slots;
     a.seq = lu->seq;
     a.timeout = wait_ticks(lu->ctx, 5.0);
+    a.list = list;
+    a.count = count;
     lu->seq += (uint32_t)W + 1u;
     const int pi = lu->prof.begin(lu->cur, PK_PANEL, (double)m_rows * W * W,
                                   2.0 * sizeof(T) * (double)m_rows * W);
-    if (m_rows <= 256) {
-        a.P = 1;
-        hipLaunchKernelGGL((k_panel<T, 256>), dim3(1), dim3(256), 0, lu->cur, a);
-    } else {
-        a.P = (int)cdiv(m_rows, 512);
-        hipLaunchKernelGGL((k_panel<T, 512>), dim3(a.P), dim3(512), 0, lu->cur, a);
-    }
+    // one row per thread while 512 threads cover the panel, then two: the fewest entries to update per
+    // column (256 rows 32 us, 512 rows 40 us per panel), and no exchange between workgroups up to 1024
+    // rows (51 us; two workgroups of 512 rows took 105)
+    a.P = (int)cdiv(m_rows, 1024);
+    if (m_rows <= 256) hipLaunchKernelGGL((k_panel<T, 256, 1>), dim3(1), dim3(256), 0, lu->cur, a);
+    else if (m_rows <= 512) hipLaunchKernelGGL((k_panel<T, 512, 1>), dim3(1), dim3(512), 0, lu->cur, a);
+    else hipLaunchKernelGGL((k_panel<T, 512, 2>), dim3(a.P), dim3(512), 0, lu->cur, a);
     lu->prof.end(lu->cur, pi);
 }
 
@@ -107,18 +109,18 @@ int getrf_blocked(lsx_lu* lu, T* F, int64_t ld, T* DL, T* DU, GU gemm_upd, GT ge
         }
         for (int64_t ji = jo; ji < jo + jbo; ji += PW) {
             const int W = (int)std::min<int64_t>(PW, jo + jbo - ji);
-            launch_panel_t<T>(lu, F, ld, ji, W);
-            const bool left = ji > jo, right = ji + W < jo + jbo;
-            if (left || right) {
-                hipLaunchKernelGGL(k_perm_build, dim3(1), dim3(256), 0, lu->cur, lu->ipiv, ji, W, il, ic,
-                                   (int*)nullptr);
-                if (left) launch_laswp_t<T>(lu, F, ld, ji, W, il, ic, jo, ji, 0);
-                if (right) {
-                    launch_laswp_t<T>(lu, F, ld, ji, W, il, ic, ji + W, jo + jbo, 1);
-                    gemm_upd(F + ji * ld + (ji + W), ld, F + (ji + W) * ld + ji, ld, F + (ji + W) * ld + (ji + W), ld,
-                             n - ji - W, jo + jbo - ji - W, W, 0);
-                }
+            launch_panel_t<T>(lu, F, ld, ji, W, il, ic);
+            const int64_t nleft = ji - jo, nright = jo + jbo - ji - W;
+            if (nleft + nright > 0) {
+                const int pi = lu->prof.begin(lu->cur, PK_LASWP, (double)W * W * nright,
+                                              sizeof(T) * 4.0 * W * (nleft + nright));
+                hipLaunchKernelGGL(k_inner_swap<T>, dim3((unsigned)cdiv(nleft + nright, ICW)), dim3(256), 0, lu->cur, F,
+                                   ld, n, ji, W, il, ic, jo, (int)nleft, ji + W, jo + jbo);
+                lu->prof.end(lu->cur, pi);
             }
+            if (nright > 0)
+                gemm_upd(F + ji * ld + (ji + W), ld, F + (ji + W) * ld + ji, ld, F + (ji + W) * ld + (ji + W), ld,
+                         n - ji - W, nright, W, 0);
         }
         // the block's interchange list first: the update stream applies it to the columns right
         // of the block while the diagonal-block inverses are formed

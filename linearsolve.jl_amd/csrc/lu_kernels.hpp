@@ -32,6 +32,8 @@ struct PanelArgs {
     uint64_t* slots;
     uint32_t seq;
     int64_t timeout;
+    int64_t* list;   // the panel's row moves as (destination, source) pairs, in k_perm_build's form
+    int* count;
 };
 
 // Words (32-bit) per element of an exchange record, and word i of an element.
@@ -44,258 +46,335 @@ template <> struct Words<float> {
     static constexpr int W = 1;
     __device__ static uint32_t word(float x, int) { return __float_as_uint(x); }
 };
-// Exchange record (32-bit words): [0,1] key (lo, hi), [2] logical row, [3] pad, [4, ...) the
-// candidate row in the panel's register layout.  16-byte multiple, so the row data is aligned.
-template <typename T> constexpr int rec_words() { return 4 + PW * Words<T>::W; }
-
-// Each thread owns one row of the panel in registers, in a rotating layout: at column c the
-// physical slot p holds logical column c + p (p < PW - c, the not yet eliminated columns) and
-// the finished values (multipliers L[r, 0..c), or the U row of a pivot row) sit in the last c
-// slots.  Column c is therefore always v[0] and every register access is static, with a
-// compact (not unrolled) column loop.
-// Rows do not move while the panel is factored: each thread carries the logical row index lr
-// of the row it holds.  The interchange of column k relabels two threads (the pivot row's
-// becomes k, the one labelled k takes the pivot row's old label) and marks the pivot row
-// finished; at the end every row is written to its logical position.  Ties of the pivot search
-// are broken by the logical index, as an explicit row interchange would.
-// P workgroups of BS threads cover rows [j0, m); with P > 1 each column exchanges one record
-// per workgroup (its best candidate and that row's data) as flag-in-word messages.  There the
-// rank-1 update of column c is deferred into column c + 1: it is applied at once to the new
-// pivot column (needed for the pivot search) and to the published candidate row, and to the
-// rest of the row while the exchange is in flight.
-template <typename T, int BS>
-__global__ __launch_bounds__(BS) void k_panel(PanelArgs<T> a) {
-    constexpr int NW = BS / 64;
-    constexpr int RW = rec_words<T>();
-    constexpr int WPE = Words<T>::W;
-    const int tid = threadIdx.x, w = blockIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int64_t r = a.j0 + (int64_t)w * BS + tid;
-    const bool valid = r < a.m;
-    T* col0 = a.A + a.j0 * a.ld;
+// Candidate record: key, logical row, 1 / candidate, and the candidate row in the panel's register
+// layout.
+template <typename T>
+struct __align__(16) PanelRec {
+    uint64_t key;
+    int row;
+    int pad;
+    T inv;
+    T pad2[16 / sizeof(T) - 1];
     T v[PW];
-#pragma unroll
-    for (int q = 0; q < PW; ++q) v[q] = (valid && q < a.W) ? col0[q * a.ld + r] : T(0);
-    int lr = (int)r;
-    bool live = valid;
-    int64_t info0 = 0;
-    if (w == 0 && tid == 0) info0 = a.dinfo[0];
+};
+// Message words ahead of the row's entries: key (2), row, pad, inverse.
+template <typename T> constexpr int panel_head() { return 4 + Words<T>::W; }
 
-    __shared__ __align__(16) uint32_t s_cand[2][NW][RW];
-    __shared__ double s_candl[2][NW];
-    __shared__ __align__(16) uint32_t s_rec[2][PMAX * RW];
-
-    // interchange of column k with pivot row grow (relabelling), pivots and info.  A live row
-    // always wins the pivot search, so grow lies in [k, m); only a record left stale by a wait
-    // that gave up (the factorization then reports LSX_ETIMEOUT) could hold another label, and it
-    // is replaced by k so that every later row index stays inside the matrix.
-    auto pivot_bookkeeping = [&](int k, int grow, T pv) {
-        if (grow < k || (int64_t)grow >= a.m) grow = k;
-        if (lr == grow) {
-            live = false;
-            lr = k;
-        } else if (lr == k) {
-            lr = grow;
-        }
-        if (w == 0 && tid == 0) {
-            a.ipiv[k] = (int64_t)grow + 1;
-            if (pv == T(0) && info0 == 0) {
-                info0 = k + 1;
-                a.dinfo[0] = info0;
-            }
-        }
-    };
-    auto scale = [&](T x, T pv) -> T {
-        if (live && pv != T(0)) {
-            if (fabs(pv) >= std::numeric_limits<T>::min()) x *= (T(1) / pv);
-            else x /= pv;
-        }
-        return x;
-    };
-
-    const int P = a.P;
-    if (P == 1) {
-        // one workgroup: everything through LDS, update right after each pivot
-#pragma unroll 1
-        for (int c = 0; c < a.W; ++c) {
-            const int par = c & 1;
-            const int k = (int)(a.j0 + c);
-            const uint64_t u = live ? pivot_key(v[0]) : 0;
-            const int wl = wave_argmax(u, lr);
-            if (lane == wl) {
-                uint32_t* d = s_cand[par][wave];
-                *reinterpret_cast<uint64_t*>(d) = u;
-                d[2] = (uint32_t)lr;
-                T* dv = reinterpret_cast<T*>(d + 4);
+// Each thread holds RPT rows of the panel in registers.  Columns go by groups of eight: within a
+// group the code of column c is unrolled and its slot is v[.][c]; after a group the slots rotate by
+// eight, so the loop body is one group's code (it stays in the instruction cache) and every register
+// index is static.  Rows do not move while the panel is factored: each carries the logical row index
+// lr of the row it holds.  The interchange of column k relabels two rows (the pivot row's becomes k,
+// the one labelled k takes the pivot row's old label) and marks the pivot row finished; at the end
+// every row is written to its logical position, and the rows that moved are listed for the
+// interchanges of the other columns.  Ties of the pivot search are broken by the logical index, as an
+// explicit row interchange would.
+// A column is a chain of latencies: the pivot search in the wave (32-bit steps), each wave's best row
+// written to LDS (with its reciprocal, formed meanwhile), one barrier, the search among the waves, and
+// the pivot row read back as one value per lane of a row of 16 lanes and broadcast from there by DPP
+// moves (an LDS read per entry and wave would be bound by LDS bandwidth).  P workgroups cover rows
+// [j0, m); with P > 1 every column also exchanges one record per workgroup (its best candidate and that
+// row's entries) as flag-in-word messages, one round trip through memory.  1024 rows per
+// workgroup: panels of up to 1024 rows need no exchange at all, taller ones half the messages of 512.
+// Measured per 32-column panel against a rotating layout (one slot per column, selects instead of
+// static slots, 64-bit search steps, an LDS read per pivot-row entry, 512 rows per workgroup): 256
+// rows 59 -> 32 us, 512 rows 70 -> 40 us, 1024 rows 105 -> 51 us, 16384 rows 124 -> 105 us.
+template <typename T, int NT, int RPT>
+__global__ __launch_bounds__(NT) void k_panel(PanelArgs<T> a) {
+    constexpr int NW = NT / 64;
+    static_assert(NW <= 8, "the search among the waves takes eight lanes");
+    constexpr int WPE = Words<T>::W;
+    constexpr int HW = panel_head<T>();
+    constexpr int PR = PMAX / 2;  // workgroups of 1024 rows
+    const int tid = threadIdx.x, w = blockIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r0 = (int)a.j0 + w * NT * RPT + tid;
+    T* col0 = a.A + a.j0 * a.ld;
+    T v[RPT][PW];
+    int lr[RPT];
+    bool live[RPT];
 #pragma unroll
-                for (int q = 0; q < PW; ++q) dv[q] = v[q];
-            }
-            __syncthreads();
-            int wi;
-            {
-                const uint64_t cu = lane < NW ? *reinterpret_cast<const uint64_t*>(s_cand[par][lane]) : 0;
-                const int cl = lane < NW ? (int)s_cand[par][lane][2] : INT_MAX;
-                wi = wave_argmax(cu, cl);
-            }
-            const uint32_t* win = s_cand[par][wi];
-            const T* prow = reinterpret_cast<const T*>(win + 4);
-            const int grow = (int)win[2];
-            const T pv = prow[0];
-            pivot_bookkeeping(k, grow, pv);
-            const T l = scale(v[0], pv);
-            const int lim = live ? PW - 1 - c : 0;  // slots 1..lim hold columns still to eliminate
-            // in groups of 8 slots: the group's pivot-row values are all read (unconditionally, so
-            // the reads overlap) before the updates, which select instead of branch
+    for (int k = 0; k < RPT; ++k) {
+        const int r = r0 + k * NT;
+        live[k] = r < (int)a.m;
+        lr[k] = r;
 #pragma unroll
-            for (int p0 = 0; p0 < PW - 1; p0 += 8) {
-                T pr[8];
-#pragma unroll
-                for (int p = p0; p < p0 + 8 && p < PW - 1; ++p) pr[p - p0] = prow[p + 1];
-#pragma unroll
-                for (int p = p0; p < p0 + 8 && p < PW - 1; ++p) {
-                    const T nv = v[p + 1];
-                    const T u = fma(-l, pr[p - p0], nv);
-                    v[p] = (p < lim) ? u : nv;
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            v[PW - 1] = l;
-        }
-    } else {
-        // pending update (column c - 1): pend = this row takes it, multiplier lp, pivot row pprev
-        bool pend = false;
-        T lp = T(0);
-        const T* pprev = reinterpret_cast<const T*>(s_rec[1] + 4);  // read, unused, before column 1
-#pragma unroll 1
-        for (int c = 0; c < a.W; ++c) {
-            const int par = c & 1;
-            const int k = (int)(a.j0 + c);
-            const int plim = PW - c;  // the pending update covers slots [0, plim)
-            {
-                const T u0 = fma(-lp, pprev[1], v[0]);
-                v[0] = pend ? u0 : v[0];
-            }
-            const uint64_t u = live ? pivot_key(v[0]) : 0;
-            const int wl = wave_argmax(u, lr);
-            if (lane == wl) {  // raw row (slot 0 already current) and its pending multiplier
-                uint32_t* d = s_cand[par][wave];
-                *reinterpret_cast<uint64_t*>(d) = u;
-                d[2] = (uint32_t)lr;
-                T* dv = reinterpret_cast<T*>(d + 4);
-#pragma unroll
-                for (int q = 0; q < PW; ++q) dv[q] = v[q];
-                s_candl[par][wave] = (double)lp;
-            }
-            __syncthreads();
-            int wi;
-            {
-                const uint64_t cu = lane < NW ? *reinterpret_cast<const uint64_t*>(s_cand[par][lane]) : 0;
-                const int cl = lane < NW ? (int)s_cand[par][lane][2] : INT_MAX;
-                wi = wave_argmax(cu, cl);
-            }
-            const uint32_t seq = a.seq + (uint32_t)c + 1u;
-            uint64_t* g = a.slots + (size_t)par * (PMAX + 1) * RECS;
-            if (tid < RW) {
-                // word tid of this workgroup's record, the candidate row brought up to date
-                const uint32_t* win = s_cand[par][wi];
-                uint32_t word = win[tid];
-                if (tid >= 4 && c > 0) {
-                    const int q = (tid - 4) / WPE;
-                    if (q > 0 && q < plim) {
-                        const T x = fma(-(T)s_candl[par][wi], pprev[q + 1], reinterpret_cast<const T*>(win + 4)[q]);
-                        word = Words<T>::word(x, (tid - 4) % WPE);
-                    }
-                }
-                st_relaxed_u64(g + (size_t)w * RECS + tid, ll_pack(word, seq));
-            }
-            // the rest of the pending update, and the rotation by one slot, while the records
-            // travel (slot 0, column c, is kept in c0 until the pivot is known)
-            const T c0 = v[0];
-#pragma unroll
-            for (int p0 = 1; p0 < PW; p0 += 8) {
-#pragma unroll
-                for (int p = p0; p < p0 + 8 && p < PW; ++p) {
-                    const T nv = v[p];
-                    v[p - 1] = (pend && p < plim) ? fma(-lp, pprev[p + 1], nv) : nv;
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            // every thread reads a share of the words of all P records, CW words per chunk (one
-            // chunk for P <= 32): all words of the chunk that are not yet current are re-read
-            // together, round by round (the update above leaves the records time to arrive).
-            constexpr int CW = (32 * RW + BS - 1) / BS;
-            const int total = P * RW;
-#pragma unroll 1
-            for (int base = 0; base < total; base += CW * BS) {
-                uint64_t x[CW];
-                uint32_t stale = 0;  // bit i: word i of this chunk still to read
-#pragma unroll
-                for (int i = 0; i < CW; ++i)
-                    if (base + tid + i * BS < total) stale |= 1u << i;
-                const int64_t t0 = wall_clock64();
-                while (stale) {
-#pragma unroll
-                    for (int i = 0; i < CW; ++i) {
-                        const int idx = base + tid + i * BS;
-                        const int rr = idx / RW;
-                        if (stale & (1u << i)) x[i] = ld_relaxed_u64(g + (size_t)rr * RECS + (idx - rr * RW));
-                    }
-#pragma unroll
-                    for (int i = 0; i < CW; ++i) {
-                        if ((stale & (1u << i)) && (uint32_t)(x[i] >> 32) == seq) {
-                            s_rec[par][base + tid + i * BS] = (uint32_t)x[i];
-                            stale &= ~(1u << i);
-                        }
-                    }
-                    if (stale) {
-                        // give up at the bound, or at once when another wait of this
-                        // factorization already has (its results are invalid anyway)
-                        if (wall_clock64() - t0 > a.timeout) {
-                            atomicOr((unsigned long long*)&a.dinfo[1], 1ull);
-                            break;
-                        }
-                        if (ld_relaxed_u64((const uint64_t*)&a.dinfo[1]) != 0) break;
-                        __builtin_amdgcn_s_sleep(2);
-                    }
-                }
-            }
-            __syncthreads();
-            // winner among the P records: lane l looks at records l and l + 64
-            uint64_t bu = 0;
-            int bl = INT_MAX, bp = 0;
-#pragma unroll
-            for (int h = 0; h < PMAX / 64; ++h) {
-                const int pidx = lane + 64 * h;
-                if (pidx < P) {
-                    const uint32_t* rp = s_rec[par] + pidx * RW;
-                    const uint64_t pu = *reinterpret_cast<const uint64_t*>(rp);
-                    const int pl = (int)rp[2];
-                    if (pu > bu || (pu == bu && pl < bl)) { bu = pu; bl = pl; bp = pidx; }
-                }
-            }
-            const int wlane = wave_argmax(bu, bl);
-            const int pw = __shfl(bp, wlane);
-            const uint32_t* win = s_rec[par] + pw * RW;
-            const T* prow = reinterpret_cast<const T*>(win + 4);
-            const int grow = (int)win[2];
-            const T pv = prow[0];
-            pivot_bookkeeping(k, grow, pv);
-            const T l = scale(c0, pv);
-            v[PW - 1] = l;
-            pend = live;
-            lp = l;
-            pprev = prow;
-        }
-        // the update of the last column touches only columns >= W (padding): nothing pending
+        for (int q = 0; q < PW; ++q) v[k][q] = (live[k] && q < a.W) ? col0[q * a.ld + r] : T(0);
     }
-    if (valid) {
-        // after W rotations slot p holds logical column (p + W) mod PW; the row goes to its
-        // logical position
-        T* dst = col0 + lr;
+    int64_t info0 = 0;
+    __shared__ PanelRec<T> s_rec[2][NW];
+    __shared__ PanelRec<T> s_all[RPT > 1 ? PR : 1];
+    if (w == 0 && tid == 0) {
+        info0 = a.dinfo[0];
+        __hip_atomic_store(a.count, a.W, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // in memory before any workgroup counts its moved rows (which all have seen a message, or
+        // passed a barrier, of this one)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    const int P = a.P;
+#pragma unroll 1
+    for (int g = 0; g < PW / 8; ++g) {
+        if (8 * g >= a.W) break;
+        const int nb = 4 - g;  // groups of eight slots that hold columns not yet finished
+        static_for<0, 8>([&](auto cc) {
+            constexpr int c = decltype(cc)::value;
+            if (8 * g + c >= a.W) return;  // uniform: only the last panel is narrower
+            const int k = (int)a.j0 + 8 * g + c, par = c & 1;
+            // the workgroup's candidate
+            uint64_t key = live[0] ? pivot_key(v[0][c]) : 0;
+            int krow = lr[0];
+            bool second = false;
+            if constexpr (RPT > 1) {
+                const uint64_t k1 = live[1] ? pivot_key(v[1][c]) : 0;
+                second = k1 > key || (k1 == key && lr[1] < krow);
+                key = second ? k1 : key;
+                krow = second ? lr[1] : krow;
+            }
+            const int wl = wave_argmax32<false>(key, krow);
+            if (lane == wl) {
+                PanelRec<T>& d = s_rec[par][wave];
+                d.key = key;
+                d.row = krow;
+                T pv;
+                // (the asm statements keep the two branches from being merged into one that indexes v)
+                if (RPT > 1 && second) {
+                    pv = v[RPT - 1][c];
 #pragma unroll
-        for (int p = 0; p < PW; ++p) {
-            const int q = (p + a.W) & (PW - 1);
-            if (q < a.W) dst[q * a.ld] = v[p];
+                    for (int q = c & ~1; q < PW; ++q)
+                        if (q < 8 || (q >> 3) < nb) d.v[q] = v[RPT - 1][q];
+                    asm volatile("; second row" ::: "memory");
+                } else {
+                    pv = v[0][c];
+#pragma unroll
+                    for (int q = c & ~1; q < PW; ++q)
+                        if (q < 8 || (q >> 3) < nb) d.v[q] = v[0][q];
+                    asm volatile("; first row" ::: "memory");
+                }
+                d.inv = T(1) / pv;
+            }
+            __syncthreads();
+            int wi;
+            {
+                const PanelRec<T>& d = s_rec[par][lane & (NW - 1)];
+                wi = NW == 1 ? 0 : wave_argmax32<true>(lane < NW ? d.key : 0, lane < NW ? d.row : INT_MAX);
+            }
+            const PanelRec<T>* win = &s_rec[par][wi];
+            if (RPT > 1 && P > 1) {
+                const uint32_t seq = a.seq + (uint32_t)(8 * g + c) + 1u;
+                uint64_t* gs = a.slots + (size_t)par * (PMAX + 1) * RECS;
+                // the words of a record: the head, then the entries from slot c & ~1 on
+                const int q0 = c & ~1, nw = HW + WPE * (8 * nb - q0);
+                if (wave == 0) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const int x = lane + 64 * h;
+                        if (x < nw) {
+                            uint32_t word;
+                            if (x >= HW) word = reinterpret_cast<const uint32_t*>(win->v)[x - HW + WPE * q0];
+                            else if (x >= 4) word = reinterpret_cast<const uint32_t*>(&win->inv)[x - 4];
+                            else word = reinterpret_cast<const uint32_t*>(win)[x];
+                            st_relaxed_u64(gs + (size_t)w * RECS + x, ll_pack(word, seq));
+                        }
+                    }
+                }
+                // wave i reads the records of workgroups i, i + NW, ..., four at a time, all words in
+                // flight; words not yet current are read again together
+#pragma unroll 1
+                for (int p0 = wave; p0 < P; p0 += 4 * NW) {
+                    uint64_t x[8];
+                    uint32_t stale = 0;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        if (p0 + (i >> 1) * NW < P && lane + 64 * (i & 1) < nw) stale |= 1u << i;
+                    const int64_t t0 = wall_clock64();
+                    while (stale) {
+#pragma unroll
+                        for (int i = 0; i < 8; ++i)
+                            if (stale & (1u << i))
+                                x[i] = ld_relaxed_u64(gs + (size_t)(p0 + (i >> 1) * NW) * RECS + lane + 64 * (i & 1));
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) {
+                            if ((stale & (1u << i)) && (uint32_t)(x[i] >> 32) == seq) {
+                                PanelRec<T>& d = s_all[p0 + (i >> 1) * NW];
+                                const int xw = lane + 64 * (i & 1);
+                                uint32_t* to = xw >= HW ? reinterpret_cast<uint32_t*>(d.v) + (xw - HW + WPE * q0)
+                                               : xw >= 4 ? reinterpret_cast<uint32_t*>(&d.inv) + (xw - 4)
+                                                         : reinterpret_cast<uint32_t*>(&d) + xw;
+                                *to = (uint32_t)x[i];
+                                stale &= ~(1u << i);
+                            }
+                        }
+                        if (stale) {
+                            // give up at the bound, or at once when another wait of this
+                            // factorization already has (its results are invalid anyway)
+                            if (wall_clock64() - t0 > a.timeout) {
+                                atomicOr((unsigned long long*)&a.dinfo[1], 1ull);
+                                break;
+                            }
+                            if (ld_relaxed_u64((const uint64_t*)&a.dinfo[1]) != 0) break;
+                        }
+                    }
+                }
+                __syncthreads();
+                const int wlane = wave_argmax32<false>(lane < P ? s_all[lane & (PR - 1)].key : 0,
+                                                       lane < P ? s_all[lane & (PR - 1)].row : INT_MAX);
+                win = &s_all[wlane];
+            }
+            int grow = win->row;
+            const T pv = win->v[c], inv = win->inv;
+            const T pa = win->v[lane & 15], pb = win->v[16 + (lane & 15)];
+            // interchange of column k with pivot row grow (relabelling), pivots and info.  A live row
+            // always wins the pivot search, so grow lies in [k, m); only a record left stale by a wait
+            // that gave up (the factorization then reports LSX_ETIMEOUT) could hold another label, and
+            // it is replaced by k so that every later row index stays inside the matrix.
+            if (grow < k || grow >= (int)a.m) grow = k;
+            if (w == 0 && tid == 0) {
+                a.ipiv[k] = (int64_t)grow + 1;
+                if (pv == T(0) && info0 == 0) {
+                    info0 = k + 1;
+                    a.dinfo[0] = info0;
+                }
+            }
+            T nl[RPT];
+#pragma unroll
+            for (int t = 0; t < RPT; ++t) {
+                if (lr[t] == grow) {
+                    live[t] = false;
+                    lr[t] = k;
+                } else if (lr[t] == k) {
+                    lr[t] = grow;
+                }
+                T l = v[t][c];
+                if (live[t] && pv != T(0)) {
+                    if (fabs(pv) >= std::numeric_limits<T>::min()) l *= inv;
+                    else l /= pv;
+                }
+                v[t][c] = l;
+                nl[t] = -l;
+            }
+            // the live rows' update (a finished row must not take it: 0 times an infinite entry)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                if (b > 0 && b >= nb) continue;
+                T pr[8];
+                static_for<0, 8>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    pr[q] = (b & 1) ? row_bcast<8 + q>(b < 2 ? pa : pb) : row_bcast<q>(b < 2 ? pa : pb);
+                });
+#pragma unroll
+                for (int t = 0; t < RPT; ++t)
+                    if (live[t]) {
+#pragma unroll
+                        for (int q = 0; q < 8; ++q)
+                            if (8 * b + q > c) v[t][8 * b + q] = fma(nl[t], pr[q], v[t][8 * b + q]);
+                    }
+            }
+        });
+        // the next group's columns to slots 0 .. 7
+#pragma unroll
+        for (int t = 0; t < RPT; ++t) {
+            T done[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) done[q] = v[t][q];
+#pragma unroll
+            for (int q = 0; q < PW - 8; ++q) v[t][q] = v[t][q + 8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[t][PW - 8 + q] = done[q];
         }
+    }
+    const int rot = 8 * ((a.W + 7) / 8);  // slot q holds column (q + rot) mod PW
+#pragma unroll
+    for (int t = 0; t < RPT; ++t) {
+        const int r = r0 + t * NT;
+        if (r < (int)a.m) {
+            T* dst = col0 + lr[t];
+#pragma unroll
+            for (int p = 0; p < PW; ++p) {
+                const int q = (p + rot) & (PW - 1);
+                if (q < a.W) dst[q * a.ld] = v[t][p];
+            }
+            const int top = lr[t] - (int)a.j0;
+            if (top < a.W || lr[t] != r) {
+                const int pos = top < a.W ? top : atomicAdd(a.count, 1);
+                if (pos < 2 * PW) {  // always, unless a wait gave up and the workgroups disagree
+                    a.list[pos] = lr[t];
+                    a.list[2 * NBO + pos] = r;
+                }
+            }
+        }
+    }
+}
+
+// Applies a panel's row moves to the other columns of its outer block, 16 columns per workgroup: nl
+// columns left of the panel (from c0 on; nl a multiple of 32), then those from cr to cend, whose rows
+// j0 .. j0 + PW - 1 are also replaced by L11^{-1} times them, L11 the panel's unit lower triangle
+// (blocked_lufact.jl:126-178).  A row of 16 lanes solves one column, each lane two of its 32 rows, the
+// solved entries broadcast by DPP moves: no barriers.  It is bound by the latency of three dependent
+// accesses (list, rows, stores): 5 us; 32 columns per workgroup with a barrier per solved row took 10-14 us.
+constexpr int ICW = 16;
+template <typename T>
+__global__ __launch_bounds__(256) void k_inner_swap(T* __restrict A, int64_t ld, int64_t n, int64_t j0, int W,
+                                                    const int64_t* __restrict list, const int* __restrict count,
+                                                    int64_t c0, int nl, int64_t cr, int64_t cend) {
+    __shared__ int s_dst[2 * PW], s_src[2 * PW];
+    __shared__ T s_buf[2 * PW][ICW + 1];
+    __shared__ T s_L[PW][PW + 1];
+    const int t = threadIdx.x;
+    const int first = (int)blockIdx.x * ICW;
+    const bool right = first >= nl;
+    const int64_t cb = right ? cr + (first - nl) : c0 + first;
+    const int ncol = right ? (int)min((int64_t)ICW, cend - cb) : ICW;
+    const int M = min(*count, 2 * PW);
+    if (t < M) {
+        // rows of [j0, n); clamped, since after a wait that gave up the list may hold anything
+        s_dst[t] = (int)min(max(list[t], j0), n - 1);
+        s_src[t] = (int)min(max(list[2 * NBO + t], j0), n - 1);
+    }
+    T lv[4];
+    if (right) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) lv[u] = A[(j0 + (t >> 5) + 8 * u) * ld + j0 + (t & 31)];
+    }
+    __syncthreads();
+    T v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int i = t & 63, cc = (t >> 6) + 4 * u;
+        v[u] = (i < M && cc < ncol) ? A[(cb + cc) * ld + s_src[i]] : T(0);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) s_buf[t & 63][(t >> 6) + 4 * u] = v[u];
+    if (right) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s_L[t & 31][(t >> 5) + 8 * u] = lv[u];
+    }
+    __syncthreads();  // every source row read before any row is written
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int i = t & 63, cc = (t >> 6) + 4 * u;
+        if (i < M && cc < ncol && (i >= W || !right)) A[(cb + cc) * ld + s_dst[i]] = v[u];
+    }
+    if (!right) return;
+    // here W == PW: columns right of a panel exist only if it is whole
+    const int cc = t >> 4, i0 = t & 15, i1 = i0 + 16;
+    T x0 = s_buf[i0][cc], x1 = s_buf[i1][cc];
+    auto step0 = [&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        const T b = row_bcast<k>(x0);
+        const T y0 = fma(-s_L[i0][k], b, x0);
+        x0 = i0 > k ? y0 : x0;
+        x1 = fma(-s_L[i1][k], b, x1);
+    };
+    auto step1 = [&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        const T b = row_bcast<k>(x1);
+        const T y1 = fma(-s_L[i1][16 + k], b, x1);
+        x1 = i0 > k ? y1 : x1;
+    };
+    static_for<0, 16>(step0);
+    static_for<0, 16>(step1);
+    if (cc < ncol) {
+        A[(cb + cc) * ld + j0 + i0] = x0;
+        A[(cb + cc) * ld + j0 + i1] = x1;
     }
 }
 

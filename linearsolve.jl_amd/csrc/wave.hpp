@@ -3,10 +3,21 @@
 #pragma once
 #include <climits>
 #include <cstdint>
+#include <type_traits>
 
 #include <hip/hip_runtime.h>
 
 namespace lsx {
+
+// f(integral_constant<int, I>) for I = 0 .. N-1, each call with its index a compile-time constant
+// (a loop whose steps index register arrays, too long for the unroller).
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<I + 1, N>(f);
+    }
+}
 
 // ---- wave-wide reductions (64 lanes): DPP within rows of 16 lanes, then two cross-row steps
 template <int CTRL> __device__ __forceinline__ uint32_t dpp32(uint32_t x) {
@@ -60,6 +71,55 @@ __device__ __forceinline__ int wave_argmax(uint64_t u, int lr) {
     if (__popcll(tie) == 1 || m == 0) return __ffsll((unsigned long long)tie) - 1;
     const int mn = wave_min_i32(u == m ? lr : INT_MAX);
     return __ffsll((unsigned long long)__ballot(u == m && lr == mn)) - 1;
+}
+template <int CTRL> __device__ __forceinline__ uint32_t dpp_max_u32(uint32_t x) {
+    const uint32_t y = dpp32<CTRL>(x);
+    return y > x ? y : x;
+}
+// Largest 32-bit value of the wave, uniform.
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
+    x = dpp_max_u32<0xB1>(x);
+    x = dpp_max_u32<0x4E>(x);
+    x = dpp_max_u32<0x141>(x);
+    x = dpp_max_u32<0x140>(x);
+    uint32_t y = xrow16(x);
+    x = y > x ? y : x;
+    y = xrow32(x);
+    x = y > x ? y : x;
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
+}
+__device__ __forceinline__ uint32_t oct_max_u32(uint32_t x) {
+    x = dpp_max_u32<0xB1>(x);
+    x = dpp_max_u32<0x4E>(x);
+    x = dpp_max_u32<0x141>(x);
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
+}
+// Lane holding the best (u, lr) pair, as wave_argmax, in 32-bit steps: the upper halves decide almost
+// always, the lower halves and then the rows are compared only among lanes that tie.  OCT: only lanes
+// 0 .. 7 hold candidates.
+template <bool OCT>
+__device__ __forceinline__ int wave_argmax32(uint64_t u, int lr) {
+    const uint32_t hi = (uint32_t)(u >> 32);
+    const uint32_t mh = OCT ? oct_max_u32(hi) : wave_max_u32(hi);
+    uint64_t tie = __ballot(hi == mh && (!OCT || (threadIdx.x & 63) < 8));
+    if (__popcll(tie) > 1) {
+        const uint32_t lo = (tie >> (threadIdx.x & 63)) & 1 ? (uint32_t)u : 0u;
+        const uint32_t ml = OCT ? oct_max_u32(lo) : wave_max_u32(lo);
+        tie &= __ballot(lo == ml);
+        if (__popcll(tie) > 1) {
+            const bool in = (tie >> (threadIdx.x & 63)) & 1;
+            const int mn = wave_min_i32(in ? lr : INT_MAX);
+            tie &= __ballot(in && lr == mn);
+        }
+    }
+    return __ffsll((unsigned long long)tie) - 1;
+}
+// Value of lane S of each row of 16 lanes, in all lanes of the row (all lanes active).
+template <int S> __device__ __forceinline__ double row_bcast(double x) {
+    return __longlong_as_double(__builtin_amdgcn_mov_dpp((long long)__double_as_longlong(x), 0x150 + S, 0xF, 0xF, true));
+}
+template <int S> __device__ __forceinline__ float row_bcast(float x) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(x), 0x150 + S, 0xF, 0xF, true));
 }
 // Pivot key: |a| as its (monotone) bit pattern + 1, NaN counted as 0; 0 = not a candidate.
 template <typename T> __device__ __forceinline__ uint64_t pivot_key(T x) {

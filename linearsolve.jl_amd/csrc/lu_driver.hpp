@@ -212,11 +212,11 @@ int getrf_blocked(lsx_lu* lu, T* F, int64_t ld, T* DL, T* DU, GU gemm_upd, GT ge
     return (int)std::min<int64_t>(lu->hinfo[0], INT32_MAX);
 }
 
-// X = A \ B with the resident factors (device buffers; FP64 right-hand sides, arithmetic in
-// FP64 whatever the factor type).  The lower solve writes lu->wy; X may alias B.  A wait that
-// gives up sets lu->dinfo[1], which the public entry point clears once (lu_clear_err) and reads
-// after its last launch, so a timeout in any of its solves is reported.
-template <typename T>
+// X = A \ B (TR: X = A^{-T} B) with the resident factors (device buffers; FP64 right-hand sides,
+// arithmetic in FP64 whatever the factor type).  The first solve writes lu->wy; X may alias B.  A
+// wait that gives up sets lu->dinfo[1], which the public entry point clears once (lu_clear_err) and
+// reads after its last launch, so a timeout in any of its solves is reported.
+template <typename T, bool TR = false>
 int getrs_blocked(lsx_lu* lu, const T* F, int64_t ld, const T* DL, const T* DU, int64_t nrhs, const double* dB,
                   int64_t ldb, double* dX, int64_t ldx) {
     lsx_ctx* ctx = lu->ctx;
@@ -227,49 +227,23 @@ int getrs_blocked(lsx_lu* lu, const T* F, int64_t ld, const T* DL, const T* DU, 
         lu->tseq = 1;
     }
     const int64_t timeout = wait_ticks(ctx, 5.0);
+    const T *d1 = TR ? DU : DL, *d2 = TR ? DL : DU;  // the triangle solved first (blocks forward), then the other
     for (int64_t c0 = 0; c0 < nrhs; c0 += TRHS) {
         const int nr = (int)std::min<int64_t>(TRHS, nrhs - c0);
         const uint32_t s1 = lu->tseq++, s2 = lu->tseq++;
         const int pi = lu->prof.begin(lu->stream, PK_TRSV, 2.0 * n * n * nr, sizeof(T) * (double)n * n);
+        const double *b = dB + c0 * ldb, *y = lu->wy;
+        double* x = dX + c0 * ldx;
+        auto grid = [&](auto kern, auto... args) {
+            hipLaunchKernelGGL(kern, dim3(nblk), dim3(256), 0, lu->stream, F, ld, n, (const int*)lu->perm, args...);
+        };
         if (nr == 1) {
-            hipLaunchKernelGGL((k_trsv<T, true, 1>), dim3(nblk), dim3(256), 0, lu->stream, F, ld, n, lu->perm, DL,
-                               dB + c0 * ldb, ldb, lu->wy, n, nr, lu->tmsg, s1, timeout, lu->dinfo + 1);
-            hipLaunchKernelGGL((k_trsv<T, false, 1>), dim3(nblk), dim3(256), 0, lu->stream, F, ld, n, lu->perm, DU,
-                               (const double*)lu->wy, n, dX + c0 * ldx, ldx, nr, lu->tmsg, s2, timeout,
-                               lu->dinfo + 1);
+            grid(k_trsv<T, true, TR>, d1, b, lu->wy, lu->tmsg, s1, timeout, lu->dinfo + 1);
+            grid(k_trsv<T, false, TR>, d2, y, x, lu->tmsg, s2, timeout, lu->dinfo + 1);
         } else {
-            hipLaunchKernelGGL((k_trsv<T, true, TRHS>), dim3(nblk), dim3(256), 0, lu->stream, F, ld, n, lu->perm,
-                               DL, dB + c0 * ldb, ldb, lu->wy, n, nr, lu->tmsg, s1, timeout, lu->dinfo + 1);
-            hipLaunchKernelGGL((k_trsv<T, false, TRHS>), dim3(nblk), dim3(256), 0, lu->stream, F, ld, n, lu->perm,
-                               DU, (const double*)lu->wy, n, dX + c0 * ldx, ldx, nr, lu->tmsg, s2, timeout,
-                               lu->dinfo + 1);
+            grid(k_trsv_mrhs<T, true, TR>, d1, b, ldb, lu->wy, n, nr, lu->tmsg, s1, timeout, lu->dinfo + 1);
+            grid(k_trsv_mrhs<T, false, TR>, d2, y, n, x, ldx, nr, lu->tmsg, s2, timeout, lu->dinfo + 1);
         }
-        lu->prof.end(lu->stream, pi);
-    }
-    LSX_HIP(ctx, hipGetLastError());
-    return LSX_OK;
-}
-
-// X = A^{-T} B with the resident factors (one right-hand side per launch pair; FP64 values).
-// The first solve writes lu->wy; X may alias B.
-template <typename T>
-int getrs_t_blocked(lsx_lu* lu, const T* F, int64_t ld, const T* DL, const T* DU, int64_t nrhs, const double* dB,
-                    int64_t ldb, double* dX, int64_t ldx) {
-    lsx_ctx* ctx = lu->ctx;
-    const int64_t n = lu->n;
-    const int nblk = (int)cdiv(n, DB);
-    if (lu->tseq > 0xF0000000u) {
-        LSX_HIP(ctx, hipMemsetAsync(lu->tmsg, 0, sizeof(uint64_t) * nblk * TMW, lu->stream));
-        lu->tseq = 1;
-    }
-    const int64_t timeout = wait_ticks(ctx, 5.0);
-    for (int64_t s = 0; s < nrhs; ++s) {
-        const uint32_t s1 = lu->tseq++, s2 = lu->tseq++;
-        const int pi = lu->prof.begin(lu->stream, PK_TRSV, 2.0 * n * n, sizeof(T) * (double)n * n);
-        hipLaunchKernelGGL((k_trsv_t<T, true>), dim3(nblk), dim3(256), 0, lu->stream, F, ld, n, lu->perm, DU,
-                           dB + s * ldb, lu->wy, lu->tmsg, s1, timeout, lu->dinfo + 1);
-        hipLaunchKernelGGL((k_trsv_t<T, false>), dim3(nblk), dim3(256), 0, lu->stream, F, ld, n, lu->perm, DL,
-                           (const double*)lu->wy, dX + s * ldx, lu->tmsg, s2, timeout, lu->dinfo + 1);
         lu->prof.end(lu->stream, pi);
     }
     LSX_HIP(ctx, hipGetLastError());

@@ -100,11 +100,13 @@ __global__ __launch_bounds__(NT) void k_panel(PanelArgs<T> a) {
 #pragma unroll
         for (int q = 0; q < PW; ++q) v[k][q] = (live[k] && q < a.W) ? col0[q * a.ld + r] : T(0);
     }
-    int64_t info0 = 0;
+    // pivots and the first zero pivot are kept here and written at the end: a store in the column loop
+    // would be waited for by the next global access (or the next wait the compiler places)
+    int info = 0;
+    __shared__ int s_piv[PW];
     __shared__ PanelRec<T> s_rec[2][NW];
     __shared__ PanelRec<T> s_all[RPT > 1 ? PR : 1];
     if (w == 0 && tid == 0) {
-        info0 = a.dinfo[0];
         __hip_atomic_store(a.count, a.W, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // in memory before any workgroup counts its moved rows (which all have seen a message, or
         // passed a barrier, of this one)
@@ -122,34 +124,34 @@ __global__ __launch_bounds__(NT) void k_panel(PanelArgs<T> a) {
             // the workgroup's candidate
             uint64_t key = live[0] ? pivot_key(v[0][c]) : 0;
             int krow = lr[0];
+            T best = v[0][c];
             bool second = false;
             if constexpr (RPT > 1) {
                 const uint64_t k1 = live[1] ? pivot_key(v[1][c]) : 0;
                 second = k1 > key || (k1 == key && lr[1] < krow);
                 key = second ? k1 : key;
                 krow = second ? lr[1] : krow;
+                best = second ? v[1][c] : best;
             }
+            const T binv = T(1) / best;  // formed in the shadow of the search
             const int wl = wave_argmax32<false>(key, krow);
             if (lane == wl) {
                 PanelRec<T>& d = s_rec[par][wave];
                 d.key = key;
                 d.row = krow;
-                T pv;
+                d.inv = binv;
                 // (the asm statements keep the two branches from being merged into one that indexes v)
                 if (RPT > 1 && second) {
-                    pv = v[RPT - 1][c];
 #pragma unroll
                     for (int q = c & ~1; q < PW; ++q)
                         if (q < 8 || (q >> 3) < nb) d.v[q] = v[RPT - 1][q];
                     asm volatile("; second row" ::: "memory");
                 } else {
-                    pv = v[0][c];
 #pragma unroll
                     for (int q = c & ~1; q < PW; ++q)
                         if (q < 8 || (q >> 3) < nb) d.v[q] = v[0][q];
                     asm volatile("; first row" ::: "memory");
                 }
-                d.inv = T(1) / pv;
             }
             __syncthreads();
             int wi;
@@ -227,13 +229,8 @@ __global__ __launch_bounds__(NT) void k_panel(PanelArgs<T> a) {
             // that gave up (the factorization then reports LSX_ETIMEOUT) could hold another label, and
             // it is replaced by k so that every later row index stays inside the matrix.
             if (grow < k || grow >= (int)a.m) grow = k;
-            if (w == 0 && tid == 0) {
-                a.ipiv[k] = (int64_t)grow + 1;
-                if (pv == T(0) && info0 == 0) {
-                    info0 = k + 1;
-                    a.dinfo[0] = info0;
-                }
-            }
+            if (tid == 0) s_piv[8 * g + c] = grow;
+            if (pv == T(0) && info == 0) info = k + 1;
             T nl[RPT];
 #pragma unroll
             for (int t = 0; t < RPT; ++t) {
@@ -280,6 +277,11 @@ __global__ __launch_bounds__(NT) void k_panel(PanelArgs<T> a) {
 #pragma unroll
             for (int q = 0; q < 8; ++q) v[t][PW - 8 + q] = done[q];
         }
+    }
+    if (w == 0) {
+        __syncthreads();
+        if (tid < a.W) a.ipiv[a.j0 + tid] = (int64_t)s_piv[tid] + 1;
+        if (tid == 0 && info != 0 && a.dinfo[0] == 0) a.dinfo[0] = info;
     }
     const int rot = 8 * ((a.W + 7) / 8);  // slot q holds column (q + rot) mod PW
 #pragma unroll
@@ -661,8 +663,12 @@ __global__ __launch_bounds__(256) void k_diag_inv(const T* __restrict F, int64_t
 
 // ------------------------------------------------------------------------------------------
 // Triangular solves (getrs), one workgroup per DB-row block.
-//   LOWER: Out = L^{-1} (P In)  (unit lower; the permutation gathers In by perm)
-//   UPPER: Out = U^{-1} In
+//   LOWER, not TR: Out = L^{-1} (P In)  (unit lower; the permutation gathers In by perm)
+//   not LOWER, not TR: Out = U^{-1} In
+// and with the transposed factors (trans = 'T': A^T x = b with P A = L U is U^T w = b, L^T v = w,
+// x = P^T v):
+//   LOWER, TR: Out = U^{-T} In  (U^T is lower triangular: blocks in forward order)
+//   not LOWER, TR: Out[perm[i]] = (L^{-T} In)[i]  (blocks in backward order)
 // Each block publishes its solution (DB x nrhs FP64 values) as flag-in-word messages: two
 // 64-bit words per value, its 32-bit halves each with the launch's sequence number.  The blocks
 // after it read those words directly, so a dependency costs one memory round trip (no flags, no
@@ -670,33 +676,55 @@ __global__ __launch_bounds__(256) void k_diag_inv(const T* __restrict F, int64_t
 // k-quarters of partial sums per row), the message reads of the next block issued before the
 // current one is used, then applies the inverse of its diagonal block.
 constexpr int TMW = 2 * DB * TRHS;  // message words of one block
-// NR: right-hand-side slots handled (1, or TRHS for nrhs > 1); the arithmetic of each value is
-// the same for both.  The block's right-hand side is read before the chain reaches the block.
-template <typename T, bool LOWER, int NR>
+
+// Words x[0 .. K) of block message m (word tid + 256 i) until they carry sequence number seq (mask:
+// which of them the thread reads; they were loaded once before).  A wait that gives up sets err.
+template <int K>
+__device__ __forceinline__ void trsv_wait(uint64_t (&x)[K], uint32_t mask, const uint64_t* m, uint32_t seq,
+                                          int64_t timeout, int64_t* err) {
+    uint32_t stale = 0;
+#pragma unroll
+    for (int i = 0; i < K; ++i)
+        if ((mask >> i & 1) && (uint32_t)(x[i] >> 32) != seq) stale |= 1u << i;
+    if (!stale) return;
+    const int64_t t0 = wall_clock64();
+    while (stale) {
+        __builtin_amdgcn_s_sleep(1);
+#pragma unroll
+        for (int i = 0; i < K; ++i)
+            if (stale & (1u << i)) x[i] = ld_relaxed_u64(m + threadIdx.x + 256 * i);
+#pragma unroll
+        for (int i = 0; i < K; ++i)
+            if ((stale & (1u << i)) && (uint32_t)(x[i] >> 32) == seq) stale &= ~(1u << i);
+        if (stale && wall_clock64() - t0 > timeout) {
+            atomicOr((unsigned long long*)err, 2ull);
+            break;
+        }
+        if (stale && ld_relaxed_u64((const uint64_t*)err) != 0) break;  // an earlier wait gave up
+    }
+}
+
+// One right-hand side.  The block's right-hand side is read before the chain reaches the block.  The
+// chain is bound by one memory round trip per block; the tiles are loaded one block ahead.  TR: the
+// tile (j, b) of F is loaded down its columns (coalesced) and turned through LDS.  n = 6000, per
+// triangle: 138 us forward, 140 us transposed (385-409 us with each transposed tile loaded where it was
+// used and its row sums left to wave reductions).
+template <typename T, bool LOWER, bool TR>
 __global__ __launch_bounds__(256) void k_trsv(const T* __restrict F, int64_t ld, int64_t n,
                                               const int* __restrict perm, const T* __restrict Dinv,
-                                              const double* In, int64_t ldin, double* Out, int64_t ldout,
-                                              int nrhs, uint64_t* msg, uint32_t seq, int64_t timeout,
-                                              int64_t* err) {
-    constexpr int WPT = (2 * DB * NR + 255) / 256;  // message words per thread
-    constexpr int BPT = (DB * NR + 255) / 256;      // right-hand-side values per thread
+                                              const double* In, double* Out, uint64_t* msg, uint32_t seq,
+                                              int64_t timeout, int64_t* err) {
     const int nblk = (int)((n + DB - 1) / DB);
     const int bw = LOWER ? (int)blockIdx.x : nblk - 1 - (int)blockIdx.x;
     const int64_t r0 = (int64_t)bw * DB;
     const int tid = threadIdx.x, rr = tid & 63, g = tid >> 6;
     const int64_t row = r0 + rr;
     __shared__ double Ds[DB][DB + 1];
-    __shared__ double Ys[2][DB][NR + 1];
-    __shared__ double Ps[4][DB][NR + 1];
-    double bin[BPT];
-#pragma unroll
-    for (int i = 0; i < BPT; ++i) {
-        const int idx = tid + 256 * i, k = idx & (DB - 1), s = idx >> 6;
-        const int64_t gr = r0 + k;
-        bin[i] = 0.0;
-        if (idx < DB * NR && gr < n && s < nrhs)
-            bin[i] = LOWER ? In[(int64_t)s * ldin + perm[gr]] : In[(int64_t)s * ldin + gr];
-    }
+    __shared__ double Ys[2][DB];
+    __shared__ double Ps[4][DB];
+    __shared__ T Ts[TR ? 2 : 1][TR ? DB : 1][DB + 1];  // TR: the tile, Ts[.][r][c] = F[j DB + r, r0 + c]
+    double bin = 0.0;
+    if (tid < DB && row < n) bin = In[LOWER && !TR ? (int64_t)perm[row] : row];
     {
         T dv[DB * DB / 256];  // all loads in flight before the LDS stores
 #pragma unroll
@@ -704,79 +732,53 @@ __global__ __launch_bounds__(256) void k_trsv(const T* __restrict F, int64_t ld,
 #pragma unroll
         for (int u = 0; u < DB * DB / 256; ++u) {
             const int idx = tid + 256 * u, i = idx & (DB - 1), k = idx >> 6;
-            Ds[i][k] = (double)dv[u];
+            if (TR) Ds[k][i] = (double)dv[u];
+            else Ds[i][k] = (double)dv[u];
         }
     }
-    double acc[NR];
-#pragma unroll
-    for (int s = 0; s < NR; ++s) acc[s] = 0.0;
-    // word w of a block's message: value (row k, rhs s) half h at w = 2 (s DB + k) + h
+    double acc = 0.0;
+    // word w of a block's message: row w / 2, half w & 1
     const int nj = LOWER ? bw : nblk - 1 - bw;  // blocks before this one in solve order
     auto jblk = [&](int t) { return LOWER ? t : nblk - 1 - t; };
-    uint64_t x[WPT];
+    uint64_t x[1] = {0};
+    const uint32_t mask = tid < 2 * DB;
     auto issue = [&](int t) {
-        const uint64_t* m = msg + (size_t)jblk(t) * TMW;
-#pragma unroll
-        for (int i = 0; i < WPT; ++i) {
-            const int w = tid + 256 * i;
-            x[i] = (w < 2 * DB * NR && w / (2 * DB) < nrhs) ? ld_relaxed_u64(m + w) : 0;
-        }
+        if (mask) x[0] = ld_relaxed_u64(msg + (size_t)jblk(t) * TMW + tid);
     };
-    // the 64 x 64 tile of block j: lane rr of group g holds F[row, j DB + 16 g + q], q < 16, in
-    // the factor's own type (converted where it is used, so that no wait for the load is placed
-    // early); tiles are loaded one block ahead of their use
+    // the 64 x 64 tile of block j: lane rr of group g holds F[row, j DB + 16 g + q] (TR:
+    // F[j DB + rr, r0 + 16 g + q]), q < 16, in the factor's own type (converted where it is used, so
+    // that no wait for the load is placed early)
     auto tload = [&](int t, T (&lv)[16]) {
         const int j = jblk(t);
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
-            const int64_t col = (int64_t)j * DB + 16 * g + q;
-            lv[q] = (row < n && col < n) ? F[col * ld + row] : T(0);
+            const int64_t fr = TR ? (int64_t)j * DB + rr : row;
+            const int64_t col = (TR ? r0 : (int64_t)j * DB) + 16 * g + q;
+            lv[q] = (fr < n && col < n) ? F[col * ld + fr] : T(0);
         }
     };
     // block t of the solve order: its message (issued earlier) until current, into Ys, the next
     // block's message issued, then acc += tile * x_j
     auto step = [&](int t, const T (&lv)[16]) {
-        const int j = jblk(t), buf = t & 1;
-        const uint64_t* m = msg + (size_t)j * TMW;
-        uint32_t stale = 0;
+        const int buf = t & 1;
+        if constexpr (TR) {
 #pragma unroll
-        for (int i = 0; i < WPT; ++i) {
-            const int w = tid + 256 * i;
-            if (w < 2 * DB * NR && w / (2 * DB) < nrhs && (uint32_t)(x[i] >> 32) != seq) stale |= 1u << i;
+            for (int q = 0; q < 16; ++q) Ts[buf][rr][16 * g + q] = lv[q];
         }
-        if (stale) {
-            const int64_t t0 = wall_clock64();
-            while (stale) {
-                __builtin_amdgcn_s_sleep(1);
-#pragma unroll
-                for (int i = 0; i < WPT; ++i)
-                    if (stale & (1u << i)) x[i] = ld_relaxed_u64(m + tid + 256 * i);
-#pragma unroll
-                for (int i = 0; i < WPT; ++i)
-                    if ((stale & (1u << i)) && (uint32_t)(x[i] >> 32) == seq) stale &= ~(1u << i);
-                if (stale && wall_clock64() - t0 > timeout) {
-                    atomicOr((unsigned long long*)err, 2ull);
-                    break;
-                }
-                if (stale && ld_relaxed_u64((const uint64_t*)err) != 0) break;  // an earlier wait gave up
-            }
-        }
+        trsv_wait<1>(x, mask, msg + (size_t)jblk(t) * TMW, seq, timeout, err);
         // the two halves of a value sit in words w, w + 1 of threads tid, tid ^ 1
-#pragma unroll
-        for (int i = 0; i < WPT; ++i) {
-            const int w = tid + 256 * i;
-            const uint32_t mine = (uint32_t)x[i];
-            const uint32_t other = (uint32_t)__shfl_xor((int)mine, 1);
-            const int k = (w >> 1) & (DB - 1), s = w / (2 * DB);
-            if (!(w & 1) && w < 2 * DB * NR && s < nrhs) Ys[buf][k][s] = __hiloint2double((int)other, (int)mine);
-        }
+        const uint32_t mine = (uint32_t)x[0];
+        const uint32_t other = (uint32_t)__shfl_xor((int)mine, 1);
+        if (mask && !(tid & 1)) Ys[buf][tid >> 1] = __hiloint2double((int)other, (int)mine);
         if (t + 1 < nj) issue(t + 1);  // the next block's words travel while this one is used
         __syncthreads();
 #pragma unroll
-        for (int q = 0; q < 16; ++q)
-#pragma unroll
-            for (int s = 0; s < NR; ++s) acc[s] = fma((double)lv[q], Ys[buf][16 * g + q][s], acc[s]);
-        // Ys is double-buffered: buffer buf is written again two blocks on, after the next barrier
+        for (int q = 0; q < 16; ++q) {
+            const double f = TR ? (double)Ts[buf][16 * g + q][rr] : (double)lv[q];
+            acc = fma(f, Ys[buf][16 * g + q], acc);
+        }
+        // Ys and Ts are double-buffered: buffer buf is written again two blocks on, after the next
+        // barrier
     };
     if (nj > 0) {
         issue(0);
@@ -790,163 +792,140 @@ __global__ __launch_bounds__(256) void k_trsv(const T* __restrict F, int64_t ld,
             step(t + 1, lb);
         }
     }
-#pragma unroll
-    for (int s = 0; s < NR; ++s) Ps[g][rr][s] = acc[s];
+    Ps[g][rr] = acc;
     __syncthreads();
-    // right-hand side minus contributions, one (row, rhs) per thread-slot
-    double (*Yb)[NR + 1] = Ys[nj & 1];
-#pragma unroll
-    for (int i = 0; i < BPT; ++i) {
-        const int idx = tid + 256 * i, k = idx & (DB - 1), s = idx >> 6;
-        if (idx < DB * NR) Yb[k][s] = bin[i] - (Ps[0][k][s] + Ps[1][k][s] + Ps[2][k][s] + Ps[3][k][s]);
-    }
+    double* Yb = Ys[nj & 1];
+    if (tid < DB) Yb[tid] = bin - (Ps[0][tid] + Ps[1][tid] + Ps[2][tid] + Ps[3][tid]);
     __syncthreads();
     // y = Dinv Yb: group g forms the partial products over k in [16 g, 16 g + 16) (four short
     // chains instead of one of 64), reduced through Ps
+    double y = 0.0;
 #pragma unroll
-    for (int s = 0; s < NR; ++s) {
-        double y = 0.0;
-#pragma unroll
-        for (int q = 0; q < 16; ++q) y = fma(Ds[rr][16 * g + q], Yb[16 * g + q][s], y);
-        Ps[g][rr][s] = y;
-    }
+    for (int q = 0; q < 16; ++q) y = fma(Ds[rr][16 * g + q], Yb[16 * g + q], y);
+    Ps[g][rr] = y;
     __syncthreads();
-    uint64_t* mine = msg + (size_t)bw * TMW;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int s = g + 4 * q;
-        if (s >= NR) continue;
-        const double y = (Ps[0][rr][s] + Ps[1][rr][s]) + (Ps[2][rr][s] + Ps[3][rr][s]);
-        if (s < nrhs) {
-            if (row < n) Out[(int64_t)s * ldout + row] = y;
-            st_relaxed_u64(mine + 2 * (s * DB + rr), ll_pack((uint32_t)__double2loint(y), seq));
-            st_relaxed_u64(mine + 2 * (s * DB + rr) + 1, ll_pack((uint32_t)__double2hiint(y), seq));
-        }
+    if (g == 0) {
+        y = (Ps[0][rr] + Ps[1][rr]) + (Ps[2][rr] + Ps[3][rr]);
+        uint64_t* mine = msg + (size_t)bw * TMW;
+        st_relaxed_u64(mine + 2 * rr, ll_pack((uint32_t)__double2loint(y), seq));
+        st_relaxed_u64(mine + 2 * rr + 1, ll_pack((uint32_t)__double2hiint(y), seq));
+        if (row < n) Out[TR && !LOWER ? (int64_t)perm[row] : row] = y;
     }
 }
 
-// Transposed triangular solves (getrs with trans = 'T', A^T x = b with P A = L U:
-// U^T w = b, L^T v = w, x = P^T v), one workgroup per DB-row block, one right-hand side.
-//   FIRST:  Out = U^{-T} In         (U^T is lower triangular: blocks in forward order)
-//   !FIRST: Out[perm[i]] = (L^{-T} In)[i]   (L^T unit upper: blocks in backward order)
-// The tile of block row b and block column j of the transposed factor is the (j, b) tile of F
-// read by columns: lane r of wave g reads F[(r0 + 16 g + q) ld + j DB + r] (coalesced) and keeps
-// its own partial sums of the 16 output rows 16 g + q over all earlier blocks but the last one;
-// those are reduced across the wave while the last block's solution travels.  The last block's
-// tile is read by rows instead (four threads per output row, 16 values each, loaded before the
-// wait), so after its solution arrives only a two-step shuffle remains; the product with the
-// diagonal block's inverse (the transpose of the stored one) is split the same way.  Block solutions travel as in k_trsv (two 64-bit words per value, 32-bit halves
-// each with the launch's sequence number).
-template <typename T, bool FIRST>
-__global__ __launch_bounds__(256) void k_trsv_t(const T* __restrict F, int64_t ld, int64_t n,
-                                                const int* __restrict perm, const T* __restrict Dinv,
-                                                const double* In, double* Out, uint64_t* msg, uint32_t seq,
-                                                int64_t timeout, int64_t* err) {
+// Up to TRHS right-hand sides: the same chain with the products on MFMA (v_mfma_f64_16x16x4f64), wave w
+// forming rows 16 w .. of the block for all right-hand sides.  Lane l gives the tile's entry (row l & 15,
+// column 4 s + l / 16) and x_j's (row 4 s + l / 16, right-hand side l & 15) at k-step s and holds rows
+// l / 16 + 4 q, right-hand side l & 15 of the sums.  The message word of (row k, right-hand side s, half
+// h) is 2 (16 k + s) + h.  With the products as vector arithmetic (an LDS read per term) a block took
+// 6-8 us; factor + solve of 16 right-hand sides at n = 16384 went from 115.3 to 112.2 ms, of 5 at
+// n = 3001 from 11.0 to 10.5 ms.
+template <typename T, bool LOWER, bool TR>
+__global__ __launch_bounds__(256) void k_trsv_mrhs(const T* __restrict F, int64_t ld, int64_t n,
+                                                   const int* __restrict perm, const T* __restrict Dinv,
+                                                   const double* In, int64_t ldin, double* Out, int64_t ldout,
+                                                   int nrhs, uint64_t* msg, uint32_t seq, int64_t timeout,
+                                                   int64_t* err) {
+    typedef double v4d __attribute__((ext_vector_type(4)));
+    static_assert(TRHS == 16, "one MFMA column block of right-hand sides");
+    constexpr int WPT = TMW / 256;  // message words per thread
     const int nblk = (int)((n + DB - 1) / DB);
-    const int bw = FIRST ? (int)blockIdx.x : nblk - 1 - (int)blockIdx.x;
+    const int bw = LOWER ? (int)blockIdx.x : nblk - 1 - (int)blockIdx.x;
     const int64_t r0 = (int64_t)bw * DB;
-    const int tid = threadIdx.x, r = tid & 63, g = tid >> 6;
-    __shared__ double Ds[DB][DB + 1];  // Ds[i][k] = Dinv^T(i, k)
-    __shared__ double Wb[2][DB];       // solution of the block being consumed (double-buffered)
-    __shared__ double Red[DB];
-    __shared__ double Yb[DB];
-    __shared__ double Bb[DB];          // the block's right-hand side
-    if (tid < DB) Bb[tid] = (r0 + tid < n) ? In[r0 + tid] : 0.0;
-    for (int idx = tid; idx < DB * DB; idx += 256) {
-        const int i = idx >> 6, k = idx & (DB - 1);
-        Ds[i][k] = (double)Dinv[(int64_t)bw * DB * DB + (int64_t)i * DB + k];
-    }
-    double acc[16];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lo = lane & 15, hi = lane >> 4;
+    const int64_t frow = r0 + 16 * w + lo;  // the row whose tile entries this lane gives
+    __shared__ double Ys[2][DB][TRHS + 1];
+    __shared__ T Ts[TR ? 2 : 1][TR ? DB : 1][DB + 1];  // TR: the tile, Ts[.][r][c] = F[j DB + r, r0 + c]
+    for (int i = tid; i < 2 * DB * (TRHS + 1); i += 256) (&Ys[0][0][0])[i] = 0.0;  // unused right-hand sides
+    double bin[4];
+    T dv[16];  // the diagonal block's inverse, as tile entries
 #pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = 0.0;
-    const int nj = FIRST ? bw : nblk - 1 - bw;
-    auto jblk = [&](int t) { return FIRST ? t : nblk - 1 - t; };
-    uint64_t x = 0;
+    for (int q = 0; q < 4; ++q) {
+        const int64_t gr = r0 + 16 * w + hi + 4 * q;
+        bin[q] = (gr < n && lo < nrhs) ? In[(int64_t)lo * ldin + (LOWER && !TR ? (int64_t)perm[gr] : gr)] : 0.0;
+    }
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+        const int i = 16 * w + lo, k = 4 * s + hi;
+        dv[s] = Dinv[(int64_t)bw * DB * DB + (TR ? i * DB + k : k * DB + i)];
+    }
+    const int nj = LOWER ? bw : nblk - 1 - bw;  // blocks before this one in solve order
+    auto jblk = [&](int t) { return LOWER ? t : nblk - 1 - t; };
+    uint64_t x[WPT];
+    uint32_t mask = 0;
+#pragma unroll
+    for (int i = 0; i < WPT; ++i)
+        if (((tid + 256 * i) >> 1 & 15) < nrhs) mask |= 1u << i;
     auto issue = [&](int t) {
-        if (tid < 2 * DB) x = ld_relaxed_u64(msg + (size_t)jblk(t) * TMW + tid);
-    };
-    // the solution of chain block j into Wb[buf] (bounded wait)
-    auto receive = [&](int j, int buf) {
-        if (tid < 2 * DB && (uint32_t)(x >> 32) != seq) {
-            const uint64_t* m = msg + (size_t)j * TMW + tid;
-            const int64_t t0 = wall_clock64();
-            while (true) {
-                __builtin_amdgcn_s_sleep(1);
-                x = ld_relaxed_u64(m);
-                if ((uint32_t)(x >> 32) == seq) break;
-                if (wall_clock64() - t0 > timeout) {
-                    atomicOr((unsigned long long*)err, 2ull);
-                    break;
-                }
-                if (ld_relaxed_u64((const uint64_t*)err) != 0) break;  // an earlier wait gave up
-            }
-        }
-        const uint32_t mine = (uint32_t)x;
-        const uint32_t other = (uint32_t)__shfl_xor((int)mine, 1);
-        if (tid < 2 * DB && !(tid & 1)) Wb[buf][tid >> 1] = __hiloint2double((int)other, (int)mine);
-    };
-    if (nj > 0) issue(0);
-    // every block but the last one in the chain: wave lanes over the source rows
-    for (int t = 0; t + 1 < nj; ++t) {
-        const int j = jblk(t), buf = t & 1;
-        const int64_t srow = (int64_t)j * DB + r;
-        double lv[16];
 #pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const int64_t ocol = r0 + 16 * g + q;
-            lv[q] = (ocol < n && srow < n) ? (double)F[ocol * ld + srow] : 0.0;
+        for (int i = 0; i < WPT; ++i)
+            x[i] = (mask >> i & 1) ? ld_relaxed_u64(msg + (size_t)jblk(t) * TMW + tid + 256 * i) : 0;
+    };
+    auto tload = [&](int t, T (&lv)[16]) {
+        const int64_t j0 = (int64_t)jblk(t) * DB;
+#pragma unroll
+        for (int s = 0; s < 16; ++s) {
+            const int64_t fr = TR ? j0 + lane : frow;
+            const int64_t col = TR ? r0 + 16 * w + s : j0 + 4 * s + hi;
+            lv[s] = (fr < n && col < n) ? F[col * ld + fr] : T(0);
         }
-        receive(j, buf);
-        issue(t + 1);
+    };
+    v4d acc = {0.0, 0.0, 0.0, 0.0};
+    auto step = [&](int t, const T (&lv)[16]) {
+        const int buf = t & 1;
+        if constexpr (TR) {
+#pragma unroll
+            for (int s = 0; s < 16; ++s) Ts[buf][lane][16 * w + s] = lv[s];
+        }
+        trsv_wait<WPT>(x, mask, msg + (size_t)jblk(t) * TMW, seq, timeout, err);
+#pragma unroll
+        for (int i = 0; i < WPT; ++i) {
+            const int v = (tid + 256 * i) >> 1;
+            const uint32_t mine = (uint32_t)x[i];
+            const uint32_t other = (uint32_t)__shfl_xor((int)mine, 1);
+            if (!(tid & 1) && (mask >> i & 1)) Ys[buf][v >> 4][v & 15] = __hiloint2double((int)other, (int)mine);
+        }
+        if (t + 1 < nj) issue(t + 1);
         __syncthreads();
-        const double wr = Wb[buf][r];
 #pragma unroll
-        for (int q = 0; q < 16; ++q) acc[q] = fma(lv[q], wr, acc[q]);
-    }
-    // their sums across the wave, while the last block's solution travels
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        double v = acc[q];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-        if (r == 0) Red[16 * g + q] = v;
-    }
-    // the last block: four threads per output row (i = tid / 4), each with 16 values of column
-    // r0 + i of F, loaded before the wait, and a two-step sum over the four
-    double last = 0.0;
+        for (int s = 0; s < 16; ++s) {
+            const double f = TR ? (double)Ts[buf][4 * s + hi][16 * w + lo] : (double)lv[s];
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(f, Ys[buf][4 * s + hi][lo], acc, 0, 0, 0);
+        }
+    };
+    __syncthreads();
     if (nj > 0) {
-        const int jl = jblk(nj - 1), buf = (nj - 1) & 1;
-        const int i = tid >> 2, p4 = tid & 3;
-        double f[16];
-#pragma unroll
-        for (int kk = 0; kk < 16; ++kk) {
-            const int64_t srow = (int64_t)jl * DB + 16 * p4 + kk;
-            f[kk] = (r0 + i < n && srow < n) ? (double)F[(r0 + i) * ld + srow] : 0.0;
+        issue(0);
+        T la[16], lb[16];
+        tload(0, la);
+        for (int t = 0; t < nj; t += 2) {
+            if (t + 1 < nj) tload(t + 1, lb);
+            step(t, la);
+            if (t + 1 >= nj) break;
+            if (t + 2 < nj) tload(t + 2, la);
+            step(t + 1, lb);
         }
-        receive(jl, buf);
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < 16; ++kk) last = fma(f[kk], Wb[buf][16 * p4 + kk], last);
-        last += __shfl_xor(last, 1);
-        last += __shfl_xor(last, 2);
     }
-    __syncthreads();
-    if ((tid & 3) == 0) Yb[tid >> 2] = Bb[tid >> 2] - Red[tid >> 2] - last;
-    __syncthreads();
-    // y = Dinv^T Yb, again four threads per row, 16 terms each
-    {
-        const int i = tid >> 2, p4 = tid & 3;
-        double y = 0.0;
+    double (*Yb)[TRHS + 1] = Ys[nj & 1];
 #pragma unroll
-        for (int kk = 0; kk < 16; ++kk) y = fma(Ds[i][16 * p4 + kk], Yb[16 * p4 + kk], y);
-        y += __shfl_xor(y, 1);
-        y += __shfl_xor(y, 2);
-        if (p4 == 0) {
-            const int64_t row = r0 + i;
-            if (row < n) Out[FIRST ? row : (int64_t)perm[row]] = y;
-            uint64_t* mine = msg + (size_t)bw * TMW;
-            st_relaxed_u64(mine + 2 * i, ll_pack((uint32_t)__double2loint(y), seq));
-            st_relaxed_u64(mine + 2 * i + 1, ll_pack((uint32_t)__double2hiint(y), seq));
+    for (int q = 0; q < 4; ++q) Yb[16 * w + hi + 4 * q][lo] = bin[q] - acc[q];
+    __syncthreads();
+    v4d y = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < 16; ++s)
+        y = __builtin_amdgcn_mfma_f64_16x16x4f64((double)dv[s], Yb[4 * s + hi][lo], y, 0, 0, 0);
+    uint64_t* mine = msg + (size_t)bw * TMW;
+    if (lo < nrhs) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int k = 16 * w + hi + 4 * q;
+            st_relaxed_u64(mine + 2 * (16 * k + lo), ll_pack((uint32_t)__double2loint(y[q]), seq));
+            st_relaxed_u64(mine + 2 * (16 * k + lo) + 1, ll_pack((uint32_t)__double2hiint(y[q]), seq));
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t row = r0 + 16 * w + hi + 4 * q;
+            if (row < n) Out[(int64_t)lo * ldout + (TR && !LOWER ? (int64_t)perm[row] : row)] = y[q];
         }
     }
 }

@@ -1,9 +1,9 @@
 // lu.hpp — resident dense-LU handle and the FP64 getrf/getrs driver entry points.
 #pragma once
 #include "common.hpp"
+#include "panel.hpp"
 
 namespace lsx {
-constexpr int PW = 32;        // panel width held in registers by the panel kernel
 constexpr int NBO = 128;      // outer block: K of the trailing MFMA update
 constexpr int PMAX = 128;     // max workgroups cooperating on one panel (512 rows each)
 constexpr int REC = 6 + 2 * PW;   // words of one FP64 exchange record: key lo/hi, row, pad, inverse, data

@@ -31,8 +31,8 @@ static void launch_panel_t(lsx_lu* lu, T* F, int64_t ld, int64_t j0, int W, int6
     const int pi = lu->prof.begin(lu->cur, PK_PANEL, (double)m_rows * W * W,
                                   2.0 * sizeof(T) * (double)m_rows * W);
     // one row per thread while 512 threads cover the panel, then two: the fewest entries to update per
-    // column (256 rows 32 us, 512 rows 40 us per panel), and no exchange between workgroups up to 1024
-    // rows (51 us; two workgroups of 512 rows took 105)
+    // column (256 rows 32 us, 512 rows 38 us per panel), and no exchange between workgroups up to 1024
+    // rows (47 us; two workgroups of 512 rows took 105)
     a.P = (int)cdiv(m_rows, 1024);
     if (m_rows <= 256) hipLaunchKernelGGL((k_panel<T, 256, 1>), dim3(1), dim3(256), 0, lu->cur, a);
     else if (m_rows <= 512) hipLaunchKernelGGL((k_panel<T, 512, 1>), dim3(1), dim3(512), 0, lu->cur, a);

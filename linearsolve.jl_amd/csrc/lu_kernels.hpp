@@ -13,7 +13,7 @@
 #include <limits>
 
 #include "lu.hpp"
-#include "wave.hpp"
+#include "panel.hpp"
 
 namespace lsx {
 
@@ -36,49 +36,10 @@ struct PanelArgs {
     int* count;
 };
 
-// Words (32-bit) per element of an exchange record, and word i of an element.
-template <typename T> struct Words;
-template <> struct Words<double> {
-    static constexpr int W = 2;
-    __device__ static uint32_t word(double x, int i) { return (uint32_t)(i ? __double2hiint(x) : __double2loint(x)); }
-};
-template <> struct Words<float> {
-    static constexpr int W = 1;
-    __device__ static uint32_t word(float x, int) { return __float_as_uint(x); }
-};
-// Candidate record: key, logical row, 1 / candidate, and the candidate row in the panel's register
-// layout.
-template <typename T>
-struct __align__(16) PanelRec {
-    uint64_t key;
-    int row;
-    int pad;
-    T inv;
-    T pad2[16 / sizeof(T) - 1];
-    T v[PW];
-};
-// Message words ahead of the row's entries: key (2), row, pad, inverse.
-template <typename T> constexpr int panel_head() { return 4 + Words<T>::W; }
-
-// Each thread holds RPT rows of the panel in registers.  Columns go by groups of eight: within a
-// group the code of column c is unrolled and its slot is v[.][c]; after a group the slots rotate by
-// eight, so the loop body is one group's code (it stays in the instruction cache) and every register
-// index is static.  Rows do not move while the panel is factored: each carries the logical row index
-// lr of the row it holds.  The interchange of column k relabels two rows (the pivot row's becomes k,
-// the one labelled k takes the pivot row's old label) and marks the pivot row finished; at the end
-// every row is written to its logical position, and the rows that moved are listed for the
-// interchanges of the other columns.  Ties of the pivot search are broken by the logical index, as an
-// explicit row interchange would.
-// A column is a chain of latencies: the pivot search in the wave (32-bit steps), each wave's best row
-// written to LDS (with its reciprocal, formed meanwhile), one barrier, the search among the waves, and
-// the pivot row read back as one value per lane of a row of 16 lanes and broadcast from there by DPP
-// moves (an LDS read per entry and wave would be bound by LDS bandwidth).  P workgroups cover rows
-// [j0, m); with P > 1 every column also exchanges one record per workgroup (its best candidate and that
-// row's entries) as flag-in-word messages, one round trip through memory.  1024 rows per
-// workgroup: panels of up to 1024 rows need no exchange at all, taller ones half the messages of 512.
-// Measured per 32-column panel against a rotating layout (one slot per column, selects instead of
-// static slots, 64-bit search steps, an LDS read per pivot-row entry, 512 rows per workgroup): 256
-// rows 59 -> 32 us, 512 rows 70 -> 40 us, 1024 rows 105 -> 51 us, 16384 rows 124 -> 105 us.
+// The panel on P workgroups covering rows [j0, m) (panel_columns does the columns).  With P > 1 every
+// column exchanges one record per workgroup (its best candidate and that row's entries) as flag-in-word
+// messages, one round trip through memory.  1024 rows per workgroup: panels of up to 1024 rows need no
+// exchange at all, taller ones half the messages of 512.
 template <typename T, int NT, int RPT>
 __global__ __launch_bounds__(NT) void k_panel(PanelArgs<T> a) {
     constexpr int NW = NT / 64;
@@ -103,8 +64,7 @@ __global__ __launch_bounds__(NT) void k_panel(PanelArgs<T> a) {
     // pivots and the first zero pivot are kept here and written at the end: a store in the column loop
     // would be waited for by the next global access (or the next wait the compiler places)
     int info = 0;
-    __shared__ int s_piv[PW];
-    __shared__ PanelRec<T> s_rec[2][NW];
+    __shared__ PanelLds<T, NW> sh;
     __shared__ PanelRec<T> s_all[RPT > 1 ? PR : 1];
     if (w == 0 && tid == 0) {
         __hip_atomic_store(a.count, a.W, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -113,174 +73,78 @@ __global__ __launch_bounds__(NT) void k_panel(PanelArgs<T> a) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     const int P = a.P;
-#pragma unroll 1
-    for (int g = 0; g < PW / 8; ++g) {
-        if (8 * g >= a.W) break;
-        const int nb = 4 - g;  // groups of eight slots that hold columns not yet finished
-        static_for<0, 8>([&](auto cc) {
-            constexpr int c = decltype(cc)::value;
-            if (8 * g + c >= a.W) return;  // uniform: only the last panel is narrower
-            const int k = (int)a.j0 + 8 * g + c, par = c & 1;
-            // the workgroup's candidate
-            uint64_t key = live[0] ? pivot_key(v[0][c]) : 0;
-            int krow = lr[0];
-            T best = v[0][c];
-            bool second = false;
-            if constexpr (RPT > 1) {
-                const uint64_t k1 = live[1] ? pivot_key(v[1][c]) : 0;
-                second = k1 > key || (k1 == key && lr[1] < krow);
-                key = second ? k1 : key;
-                krow = second ? lr[1] : krow;
-                best = second ? v[1][c] : best;
-            }
-            const T binv = T(1) / best;  // formed in the shadow of the search
-            const int wl = wave_argmax32<false>(key, krow);
-            if (lane == wl) {
-                PanelRec<T>& d = s_rec[par][wave];
-                d.key = key;
-                d.row = krow;
-                d.inv = binv;
-                // (the asm statements keep the two branches from being merged into one that indexes v)
-                if (RPT > 1 && second) {
-#pragma unroll
-                    for (int q = c & ~1; q < PW; ++q)
-                        if (q < 8 || (q >> 3) < nb) d.v[q] = v[RPT - 1][q];
-                    asm volatile("; second row" ::: "memory");
-                } else {
-#pragma unroll
-                    for (int q = c & ~1; q < PW; ++q)
-                        if (q < 8 || (q >> 3) < nb) d.v[q] = v[0][q];
-                    asm volatile("; first row" ::: "memory");
-                }
-            }
+    auto exchange = [&](const PanelRec<T>* own, int col, bool sender) -> const PanelRec<T>* {
+        if (RPT == 1 || P == 1) {
             __syncthreads();
-            int wi;
-            {
-                const PanelRec<T>& d = s_rec[par][lane & (NW - 1)];
-                wi = NW == 1 ? 0 : wave_argmax32<true>(lane < NW ? d.key : 0, lane < NW ? d.row : INT_MAX);
-            }
-            const PanelRec<T>* win = &s_rec[par][wi];
-            if (RPT > 1 && P > 1) {
-                const uint32_t seq = a.seq + (uint32_t)(8 * g + c) + 1u;
-                uint64_t* gs = a.slots + (size_t)par * (PMAX + 1) * RECS;
-                // the words of a record: the head, then the entries from slot c & ~1 on
-                const int q0 = c & ~1, nw = HW + WPE * (8 * nb - q0);
-                if (wave == 0) {
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const int x = lane + 64 * h;
-                        if (x < nw) {
-                            uint32_t word;
-                            if (x >= HW) word = reinterpret_cast<const uint32_t*>(win->v)[x - HW + WPE * q0];
-                            else if (x >= 4) word = reinterpret_cast<const uint32_t*>(&win->inv)[x - 4];
-                            else word = reinterpret_cast<const uint32_t*>(win)[x];
-                            st_relaxed_u64(gs + (size_t)w * RECS + x, ll_pack(word, seq));
-                        }
-                    }
-                }
-                // wave i reads the records of workgroups i, i + NW, ..., four at a time, all words in
-                // flight; words not yet current are read again together
-#pragma unroll 1
-                for (int p0 = wave; p0 < P; p0 += 4 * NW) {
-                    uint64_t x[8];
-                    uint32_t stale = 0;
-#pragma unroll
-                    for (int i = 0; i < 8; ++i)
-                        if (p0 + (i >> 1) * NW < P && lane + 64 * (i & 1) < nw) stale |= 1u << i;
-                    const int64_t t0 = wall_clock64();
-                    while (stale) {
-#pragma unroll
-                        for (int i = 0; i < 8; ++i)
-                            if (stale & (1u << i))
-                                x[i] = ld_relaxed_u64(gs + (size_t)(p0 + (i >> 1) * NW) * RECS + lane + 64 * (i & 1));
-#pragma unroll
-                        for (int i = 0; i < 8; ++i) {
-                            if ((stale & (1u << i)) && (uint32_t)(x[i] >> 32) == seq) {
-                                PanelRec<T>& d = s_all[p0 + (i >> 1) * NW];
-                                const int xw = lane + 64 * (i & 1);
-                                uint32_t* to = xw >= HW ? reinterpret_cast<uint32_t*>(d.v) + (xw - HW + WPE * q0)
-                                               : xw >= 4 ? reinterpret_cast<uint32_t*>(&d.inv) + (xw - 4)
-                                                         : reinterpret_cast<uint32_t*>(&d) + xw;
-                                *to = (uint32_t)x[i];
-                                stale &= ~(1u << i);
-                            }
-                        }
-                        if (stale) {
-                            // give up at the bound, or at once when another wait of this
-                            // factorization already has (its results are invalid anyway)
-                            if (wall_clock64() - t0 > a.timeout) {
-                                atomicOr((unsigned long long*)&a.dinfo[1], 1ull);
-                                break;
-                            }
-                            if (ld_relaxed_u64((const uint64_t*)&a.dinfo[1]) != 0) break;
-                        }
-                    }
-                }
-                __syncthreads();
-                const int wlane = wave_argmax32<false>(lane < P ? s_all[lane & (PR - 1)].key : 0,
-                                                       lane < P ? s_all[lane & (PR - 1)].row : INT_MAX);
-                win = &s_all[wlane];
-            }
-            int grow = win->row;
-            const T pv = win->v[c], inv = win->inv;
-            const T pa = win->v[lane & 15], pb = win->v[16 + (lane & 15)];
-            // interchange of column k with pivot row grow (relabelling), pivots and info.  A live row
-            // always wins the pivot search, so grow lies in [k, m); only a record left stale by a wait
-            // that gave up (the factorization then reports LSX_ETIMEOUT) could hold another label, and
-            // it is replaced by k so that every later row index stays inside the matrix.
-            if (grow < k || grow >= (int)a.m) grow = k;
-            if (tid == 0) s_piv[8 * g + c] = grow;
-            if (pv == T(0) && info == 0) info = k + 1;
-            T nl[RPT];
-#pragma unroll
-            for (int t = 0; t < RPT; ++t) {
-                if (lr[t] == grow) {
-                    live[t] = false;
-                    lr[t] = k;
-                } else if (lr[t] == k) {
-                    lr[t] = grow;
-                }
-                T l = v[t][c];
-                if (live[t] && pv != T(0)) {
-                    if (fabs(pv) >= std::numeric_limits<T>::min()) l *= inv;
-                    else l /= pv;
-                }
-                v[t][c] = l;
-                nl[t] = -l;
-            }
-            // the live rows' update (a finished row must not take it: 0 times an infinite entry)
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                if (b > 0 && b >= nb) continue;
-                T pr[8];
-                static_for<0, 8>([&](auto qc) {
-                    constexpr int q = decltype(qc)::value;
-                    pr[q] = (b & 1) ? row_bcast<8 + q>(b < 2 ? pa : pb) : row_bcast<q>(b < 2 ? pa : pb);
-                });
-#pragma unroll
-                for (int t = 0; t < RPT; ++t)
-                    if (live[t]) {
-#pragma unroll
-                        for (int q = 0; q < 8; ++q)
-                            if (8 * b + q > c) v[t][8 * b + q] = fma(nl[t], pr[q], v[t][8 * b + q]);
-                    }
-            }
-        });
-        // the next group's columns to slots 0 .. 7
-#pragma unroll
-        for (int t = 0; t < RPT; ++t) {
-            T done[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) done[q] = v[t][q];
-#pragma unroll
-            for (int q = 0; q < PW - 8; ++q) v[t][q] = v[t][q + 8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) v[t][PW - 8 + q] = done[q];
+            return own;
         }
-    }
-    if (w == 0) {
+        const uint32_t seq = a.seq + (uint32_t)col + 1u;
+        uint64_t* gs = a.slots + (size_t)(col & 1) * (PMAX + 1) * RECS;
+        // the words of a record: the head, then the entries from column col & ~1 on; sent by the wave
+        // that wrote the record (its own LDS writes need no barrier)
+        const int q0 = col & ~1, nw = HW + WPE * (PW - q0);
+        if (sender) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int x = lane + 64 * h;
+                if (x < nw) {
+                    uint32_t word;
+                    if (x >= HW) word = reinterpret_cast<const uint32_t*>(own->v)[x - HW + WPE * q0];
+                    else if (x >= 4) word = reinterpret_cast<const uint32_t*>(&own->inv)[x - 4];
+                    else word = reinterpret_cast<const uint32_t*>(own)[x];
+                    st_relaxed_u64(gs + (size_t)w * RECS + x, ll_pack(word, seq));
+                }
+            }
+        }
+        // wave i reads the records of workgroups i, i + NW, ..., four at a time, all words in
+        // flight; words not yet current are read again together
+#pragma unroll 1
+        for (int p0 = wave; p0 < P; p0 += 4 * NW) {
+            uint64_t x[8];
+            uint32_t stale = 0;
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (p0 + (i >> 1) * NW < P && lane + 64 * (i & 1) < nw) stale |= 1u << i;
+            const int64_t t0 = wall_clock64();
+            for (unsigned spin = 1; stale; ++spin) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    if (stale & (1u << i))
+                        x[i] = ld_relaxed_u64(gs + (size_t)(p0 + (i >> 1) * NW) * RECS + lane + 64 * (i & 1));
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    if ((stale & (1u << i)) && (uint32_t)(x[i] >> 32) == seq) {
+                        PanelRec<T>& d = s_all[p0 + (i >> 1) * NW];
+                        const int xw = lane + 64 * (i & 1);
+                        uint32_t* to = xw >= HW ? reinterpret_cast<uint32_t*>(d.v) + (xw - HW + WPE * q0)
+                                       : xw >= 4 ? reinterpret_cast<uint32_t*>(&d.inv) + (xw - 4)
+                                                 : reinterpret_cast<uint32_t*>(&d) + xw;
+                        *to = (uint32_t)x[i];
+                        stale &= ~(1u << i);
+                    }
+                }
+                if (stale) {
+                    // give up at the bound, or soon after another wait of this factorization has
+                    // (its results are invalid anyway); the error word is read only every 16th
+                    // round, since its load would double the period of the polling
+                    if (wall_clock64() - t0 > a.timeout) {
+                        atomicOr((unsigned long long*)&a.dinfo[1], 1ull);
+                        break;
+                    }
+                    if (spin % 16 == 0 && ld_relaxed_u64((const uint64_t*)&a.dinfo[1]) != 0) break;
+                }
+            }
+        }
         __syncthreads();
-        if (tid < a.W) a.ipiv[a.j0 + tid] = (int64_t)s_piv[tid] + 1;
+        const int wlane = wave_argmax32(lane < P ? s_all[lane & (PR - 1)].key : 0,
+                                               lane < P ? s_all[lane & (PR - 1)].row : INT_MAX);
+        return &s_all[wlane];
+    };
+    panel_columns<T, NT, RPT>(v, lr, live, a.W, (int)a.j0, (int)a.m, sh, info, exchange);
+    __syncthreads();
+    if (w == 0) {
+        if (tid < a.W) a.ipiv[a.j0 + tid] = (int64_t)sh.piv[tid] + 1;
         if (tid == 0 && info != 0 && a.dinfo[0] == 0) a.dinfo[0] = info;
     }
     const int rot = 8 * ((a.W + 7) / 8);  // slot q holds column (q + rot) mod PW
@@ -289,12 +153,18 @@ __global__ __launch_bounds__(NT) void k_panel(PanelArgs<T> a) {
         const int r = r0 + t * NT;
         if (r < (int)a.m) {
             T* dst = col0 + lr[t];
-#pragma unroll
-            for (int p = 0; p < PW; ++p) {
-                const int q = (p + rot) & (PW - 1);
-                if (q < a.W) dst[q * a.ld] = v[t][p];
-            }
             const int top = lr[t] - (int)a.j0;
+            if (top >= a.W) {
+#pragma unroll
+                for (int p = 0; p < PW; ++p) {
+                    const int q = (p + rot) & (PW - 1);
+                    if (q < a.W) dst[q * a.ld] = v[t][p];
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < PW; ++q)
+                    if (q < a.W) dst[q * a.ld] = sh.fin[top].v[q];
+            }
             if (top < a.W || lr[t] != r) {
                 const int pos = top < a.W ? top : atomicAdd(a.count, 1);
                 if (pos < 2 * PW) {  // always, unless a wait gave up and the workgroups disagree
@@ -688,7 +558,7 @@ __device__ __forceinline__ void trsv_wait(uint64_t (&x)[K], uint32_t mask, const
         if ((mask >> i & 1) && (uint32_t)(x[i] >> 32) != seq) stale |= 1u << i;
     if (!stale) return;
     const int64_t t0 = wall_clock64();
-    while (stale) {
+    for (unsigned spin = 1; stale; ++spin) {
         __builtin_amdgcn_s_sleep(1);
 #pragma unroll
         for (int i = 0; i < K; ++i)
@@ -700,7 +570,8 @@ __device__ __forceinline__ void trsv_wait(uint64_t (&x)[K], uint32_t mask, const
             atomicOr((unsigned long long*)err, 2ull);
             break;
         }
-        if (stale && ld_relaxed_u64((const uint64_t*)err) != 0) break;  // an earlier wait gave up
+        // an earlier wait gave up (read every 16th round: its load would double the polling period)
+        if (stale && spin % 16 == 0 && ld_relaxed_u64((const uint64_t*)err) != 0) break;
     }
 }
 

@@ -88,23 +88,14 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
     x = y > x ? y : x;
     return (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
 }
-__device__ __forceinline__ uint32_t oct_max_u32(uint32_t x) {
-    x = dpp_max_u32<0xB1>(x);
-    x = dpp_max_u32<0x4E>(x);
-    x = dpp_max_u32<0x141>(x);
-    return (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
-}
 // Lane holding the best (u, lr) pair, as wave_argmax, in 32-bit steps: the upper halves decide almost
-// always, the lower halves and then the rows are compared only among lanes that tie.  OCT: only lanes
-// 0 .. 7 hold candidates.
-template <bool OCT>
+// always, the lower halves and then the rows are compared only among lanes that tie.
 __device__ __forceinline__ int wave_argmax32(uint64_t u, int lr) {
     const uint32_t hi = (uint32_t)(u >> 32);
-    const uint32_t mh = OCT ? oct_max_u32(hi) : wave_max_u32(hi);
-    uint64_t tie = __ballot(hi == mh && (!OCT || (threadIdx.x & 63) < 8));
+    uint64_t tie = __ballot(hi == wave_max_u32(hi));
     if (__popcll(tie) > 1) {
         const uint32_t lo = (tie >> (threadIdx.x & 63)) & 1 ? (uint32_t)u : 0u;
-        const uint32_t ml = OCT ? oct_max_u32(lo) : wave_max_u32(lo);
+        const uint32_t ml = wave_max_u32(lo);
         tie &= __ballot(lo == ml);
         if (__popcll(tie) > 1) {
             const bool in = (tie >> (threadIdx.x & 63)) & 1;
@@ -113,6 +104,29 @@ __device__ __forceinline__ int wave_argmax32(uint64_t u, int lr) {
         }
     }
     return __ffsll((unsigned long long)tie) - 1;
+}
+// The same over N candidates (N = 2, 4 or 8), candidate l & (N - 1) in lane l.
+template <int N>
+__device__ __forceinline__ int wave_argmax_rep(uint64_t u, int lr) {
+    static_assert(N == 2 || N == 4 || N == 8, "two, four or eight candidates");
+    constexpr uint64_t first = (1ull << N) - 1;
+    auto mx = [](uint32_t x) {
+        x = dpp_max_u32<0xB1>(x);
+        if constexpr (N > 2) x = dpp_max_u32<0x4E>(x);
+        if constexpr (N > 4) x = dpp_max_u32<0x141>(x);
+        return (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
+    };
+    const uint32_t hi = (uint32_t)(u >> 32);
+    uint64_t tie = __ballot(hi == mx(hi));
+    if (__popcll(tie & first) > 1) {
+        const uint32_t lo = (tie >> (threadIdx.x & 63)) & 1 ? (uint32_t)u : 0u;
+        tie &= __ballot(lo == mx(lo));
+        if (__popcll(tie & first) > 1) {
+            const bool in = (tie >> (threadIdx.x & 63)) & 1;
+            tie &= __ballot(in && ~(uint32_t)lr == mx(in ? ~(uint32_t)lr : 0u));  // the smallest row
+        }
+    }
+    return __ffsll((unsigned long long)(tie & first)) - 1;
 }
 // Value of lane S of each row of 16 lanes, in all lanes of the row (all lanes active).
 template <int S> __device__ __forceinline__ double row_bcast(double x) {

@@ -4,10 +4,8 @@ For every factor type (FP64; FP32 with FP64 refinement) and size bin it builds a
 that bin's sizes (A = I - g J, the batched workload's distribution, generated on the GPU), times
 the persistent batched launch with each candidate panel width, keeps the fastest, and writes the
 tables to tile_table.json beside this file; _BatchHandle loads the table of its factor type when
-the file exists (lsx_batch_set_tiles).  The panel width fixes the blocking of a system: widths 8
-and 16 hold the panel's L21 in LDS (FP64) for trailing-update tiles dealt to the waves in turn;
-width 32 keeps a row block of L21 in each wave's registers and sweeps its columns, with half the
-trailing-matrix traffic of width 16.
+the file exists (lsx_batch_set_tiles).  The table is a hint: the library runs every size with
+32-column panels, which it measures fastest from n = 1 to 512.
 
     python linearsolve.jl_amd/autotune.py [out.json]   # default: tile_table.json beside this file
 """

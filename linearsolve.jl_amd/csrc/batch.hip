@@ -11,16 +11,14 @@
 //
 // Scheduling: systems are sorted by decreasing size on the host (longest first); a persistent
 // grid of workgroups takes them from an atomic counter, one workgroup per system.
-// Per system (BT threads): right-looking blocked LU with panels of BW columns factored in
-// registers (pivot search on packed keys by DPP).  A panel's row interchanges are applied in
-// memory to the columns right of it as U12 is formed (one thread per column moves the at most
-// 2 BW rows involved), so the trailing update A22 -= L21 U12 reads and writes contiguous rows;
-// it runs on MFMA: FP64 panels of 8 or 16 columns hold L21 in LDS and deal 64 x 32 tiles to the
-// waves in turn; 32-column panels (and every FP32 panel) keep a 32-row block of L21 in each
-// wave's registers and sweep the 32 x 32 tiles of its rows, U12 read from L2.  The L columns
+// Per system (BT threads): right-looking blocked LU, panels of 32 columns factored by the blocked LU's panel
+// code (panel.hpp), two of them per step: the second panel's columns take the first's interchanges and
+// update, then the columns right of both take the interchanges, U12 and one trailing update
+// A22 -= L21 U12 of 64 columns on MFMA, so A22 is read and written once per 64 columns.  Row
+// interchanges are applied in memory to the columns right of the panels as U12 is formed, so the
+// trailing updates read and write contiguous rows; the L columns
 // take the interchanges of later panels in one gather after the last panel (like dlaswp on the
-// left, but once).  The panel width BW (8, 16 or 32) is chosen per system from a size-binned
-// tile table (set by the autotuner through lsx_batch_set_tiles).  Triangular solves go by
+// left, but once).  Triangular solves go by
 // blocks of 64 (FP32: 32) rows: the diagonal block is staged in LDS and solved by one wave with
 // shuffles, the rows beyond it are updated by all threads, sixteen loads in flight per row.
 // The launch sequence of a handle (counter reset + persistent kernel) is captured once in a HIP
@@ -34,7 +32,7 @@
 #include <vector>
 
 #include "batch.hpp"
-#include "wave.hpp"
+#include "panel.hpp"
 
 namespace lsx {
 
@@ -46,46 +44,27 @@ constexpr int BNMAX = 512;         // largest system
 constexpr int RPT = (BNMAX + BT - 1) / BT;  // panel rows per thread
 static_assert(RPT <= 2, "a pivot row is held by the first or the last of a thread's panel rows");
 
-// Per factor type: systems (workgroups) per CU, the trailing-update block of a wave in 16 x 16
-// tiles, whether L21 and the pivot row are held (L21 in LDS, the pivot row in registers) or read
-// where they are used, and the row block SB of the triangular solves.
-// FP64: two systems per CU (up to 256 registers, 80 KB of LDS each) with L21 in LDS and 64-row
-// solve blocks.  FP32: three systems per CU (168 registers, 36 KB of LDS each: 17 KB of them
-// stage U12 of 32-column panels), L21 read back from the factor in L2 and 32-row solve blocks;
-// the extra systems hide the latency of its refinement passes.  (FP64 at four systems per CU
-// spills registers and runs slower; FP32 at four spills 129 registers once U12 is staged.)
+// Per factor type: systems (workgroups) per CU and the row block SB of the triangular solves.  FP64: two
+// systems per CU (up to 256 registers, 80 KB of LDS each).  FP32: three (168 registers, 53 KB), which
+// hide the latency of its refinement passes.
 template <typename T> struct BatchCfg;
-// Panels of 32 columns never hold L21 (it would take 136 KB of LDS); their trailing update
-// (and every FP32 one) keeps a row block of L21 in registers and sweeps the column blocks of
-// its rows, in RB2 x CB2 tiles.
-// (Loading a wave's next tile while it forms the current one measured slower: the registers
-// it takes cost spills and occupancy.)
-template <> struct BatchCfg<double> {
-    static constexpr int WG = 2, RB = 4, CB = 2, RB2 = 2, CB2 = 2, SB = 64;
-    static constexpr bool HOLD = true;
-};
-template <> struct BatchCfg<float> {
-    static constexpr int WG = 3, RB = 2, CB = 2, RB2 = 2, CB2 = 2, SB = 32;
-    static constexpr bool HOLD = false;
-};
-constexpr int PMAX = 32;  // widest panel
-constexpr int UCH_F = 128;  // FP32: columns of U12 staged in LDS at a time
-// Whether a panel of width BW holds L21 in LDS and the pivot row in registers.
-template <typename T, int BW> struct PanelHold { static constexpr bool value = BatchCfg<T>::HOLD && BW <= 16; };
-
-// Panel-width index (0: 8, 1: 16, 2: 32 columns) of a system without a tile table (the widths
-// the autotuner picks on MI355X for both factor types; the serving lane's batches use these).
-__host__ __device__ inline int default_cfg(int n) { return n <= 64 ? 0 : (n <= 192 ? 1 : 2); }
+template <> struct BatchCfg<double> { static constexpr int WG = 2, SB = 64; };
+template <> struct BatchCfg<float> { static constexpr int WG = 3, SB = 32; };
+constexpr int SW = 2 * PW;  // columns of a step of factor_sys (two panels)
+constexpr int UCH = 128;    // columns of U12 staged in LDS at a time
+// Stride of a staged column of U12, such that the 16 columns and the k entries that a wave (FP64: half a
+// wave) reads at once fall into different LDS banks.
+template <typename T> constexpr int ust() { return sizeof(T) == 8 ? SW + 2 : SW + 4; }
 
 struct BatchArgs {
     int64_t count;
     const int32_t* order;     // systems by decreasing n
     const int32_t* n;
-    const uint8_t* cfg;       // per-system panel-width index (nullable: default by n)
     const int64_t* aoff;      // offset of A_i (n_i^2 elements)
     const int64_t* voff;      // offset of b_i / x_i / ipiv_i
     void* A;                  // workspace of the factor type: factored in place
-    const double* A64;        // FP32 path: the FP64 matrices (refinement residuals)
+    const double* const* src; // device word holding the matrices' address: they are read there and factored
+                              // in A (null, or a null address: A holds them; FP32 needs an address)
     const double* b;
     double* x;
     int64_t* ipiv;            // LAPACK swap sequence (1-based), packed like b
@@ -102,22 +81,15 @@ template <typename T>
 struct BatchShared {
     static constexpr int SB = BatchCfg<T>::SB;
     static_assert(BNMAX <= SB * (SB + 1), "the FP32 residual is kept in the solve staging block");
-    static_assert(PMAX * (PMAX + 1) <= SB * (SB + 1), "L11 of the widest panel fits the staging block");
     union {
-        double l21[BatchCfg<T>::HOLD ? BNMAX * 17 : 1];  // held L21 (row r of the panel at r * 17;
-                                                         // its first rows are L11)
+        // factor_sys: the panel's LDS and the second panel's U12 / L11 of both panels / staged U12
+        __align__(16) T wide[UCH * ust<T>()];
         double dblk[SB][SB + 1];   // staged diagonal block of the solves / FP32 path: the residual /
                                    // during the factorization, L11 of a panel without held L21
     };
-    uint64_t wkey[BT / 64];   // pivot search: each wave's best key and row
-    int wrow[BT / 64];
-    double rowbuf[2][PMAX];    // pivot row and the row it displaces (panel columns)
     double red[2][BT / 64];
-    int chg[PMAX];             // rows below the panel that its interchanges move
+    int chg[SW];               // rows below the panel(s) that the interchanges move
     int nchg;
-    // FP32, 32-column panels: staged U12 of the trailing update (UCH_F columns, padded rows);
-    // FP64 stages it in the held-L21 area instead
-    T ustg[BatchCfg<T>::HOLD ? 1 : UCH_F * (PMAX + 1)];
     double xs[BNMAX];          // solve vector
     union {
         double xr[BNMAX];      // FP32 path: the refined solution (after the factorization)
@@ -164,352 +136,13 @@ __device__ __forceinline__ void block_max2(BatchShared<T>& sh, double& a, double
     __syncthreads();
 }
 
-// Column C of a panel held in registers (v: thread tid's logical rows tid + k BT): pivot
-// search, the interchange of rows C and the pivot row through LDS, elimination below row C.
-// Two barriers per column.  Instantiated for C = 0..BW-1 so that v is indexed by constants.
-template <typename T, int BW, int C>
-__device__ __forceinline__ void panel_col(BatchShared<T>& sh, T (&v)[RPT][BW], int m, int j0, int jb, int64_t vo,
-                                          int64_t* ipiv, int64_t& info) {
-    if constexpr (C < BW) {
-        const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-        if (C < jb) {  // uniform: only the last panel is narrower
-            // pivot: first row of max |a| among logical rows C..m-1 (NaN counts as 0), by packed
-            // keys (0: no candidate): the thread's rows, the wave (DPP), then the four waves
-            uint64_t key = 0;
-            int krow = INT_MAX;
-#pragma unroll
-            for (int k = 0; k < RPT; ++k) {
-                const int r = tid + k * BT;
-                if (r >= C && r < m) {
-                    const uint64_t u = pivot_key(v[k][C]);
-                    if (u > key) { key = u; krow = r; }  // rows increase with k: a tie keeps the first
-                }
-            }
-            const int wl = wave_argmax(key, krow);
-            if (lane == wl) { sh.wkey[wave] = key; sh.wrow[wave] = krow; }
-            __syncthreads();
-            uint64_t bk = sh.wkey[0];
-            int pr = sh.wrow[0];
-#pragma unroll
-            for (int i = 1; i < BT / 64; ++i) {
-                const uint64_t ki = sh.wkey[i];
-                const int ri = sh.wrow[i];
-                if (ki > bk || (ki == bk && ri < pr)) { bk = ki; pr = ri; }
-            }
-            // the pivot row and (when they differ) row C through LDS; row C is thread C's first row
-            if (tid == (pr & (BT - 1))) {
-#pragma unroll
-                for (int q = 0; q < BW; ++q) {
-                    T x = v[0][q];
-                    if constexpr (RPT > 1) x = (pr >= BT) ? v[RPT - 1][q] : x;
-                    sh.rowbuf[0][q] = (double)x;
-                }
-            }
-            if (pr != C && tid == C) {
-#pragma unroll
-                for (int q = 0; q < BW; ++q) sh.rowbuf[1][q] = (double)v[0][q];
-            }
-            if (tid == 0) {
-                const int k = j0 + C;
-                sh.piv[k] = j0 + pr;
-                if (ipiv) ipiv[vo + k] = (int64_t)(j0 + pr) + 1;
-                if (pr != C) {
-                    const int t = sh.perm[k];
-                    sh.perm[k] = sh.perm[j0 + pr];
-                    sh.perm[j0 + pr] = t;
-                }
-            }
-            __syncthreads();
-            // the pivot row: held in registers, or read from LDS where it is used
-            T prh[BW];
-#pragma unroll
-            for (int q = 0; q < BW; ++q) prh[q] = PanelHold<T, BW>::value ? (T)sh.rowbuf[0][q] : T(0);
-            auto prow = [&](int q) -> T { return PanelHold<T, BW>::value ? prh[q] : (T)sh.rowbuf[0][q]; };
-            if (pr != C) {
-                if (tid == C) {
-#pragma unroll
-                    for (int q = 0; q < BW; ++q) v[0][q] = prow(q);
-                }
-                if (tid == (pr & (BT - 1))) {
-#pragma unroll
-                    for (int q = 0; q < BW; ++q) {
-                        const T t = (T)sh.rowbuf[1][q];
-                        if constexpr (RPT > 1) {
-                            if (pr >= BT) v[RPT - 1][q] = t;
-                            else v[0][q] = t;
-                        } else {
-                            v[0][q] = t;
-                        }
-                    }
-                }
-            }
-            const T pv = prow(C);
-            if (pv == T(0) && info == 0) info = j0 + C + 1;
-#pragma unroll
-            for (int k = 0; k < RPT; ++k) {
-                const int r = tid + k * BT;
-                if (r > C && r < m) {
-                    T l = v[k][C];
-                    if (pv != T(0)) {
-                        if (fabs((double)pv) >= (double)std::numeric_limits<T>::min()) l *= (T(1) / pv);
-                        else l /= pv;
-                    }
-                    v[k][C] = l;
-#pragma unroll
-                    for (int q = C + 1; q < BW; ++q) v[k][q] = fma(-l, prow(q), v[k][q]);
-                }
-            }
-    }
-        panel_col<T, BW, C + 1>(sh, v, m, j0, jb, vo, ipiv, info);
-    }
-}
-
-// LU with partial pivoting of one n x n system (column-major, in place).  Each panel's row
-// interchanges reach the columns right of it while U12 is formed, so the trailing update reads
-// and writes rows in place (coalesced); the columns left of it (L) take all later interchanges in
-// one gather at the end, which also leaves the system's permutation (logical row -> original row)
-// in sh.perm.  On return A holds L and U in LAPACK's row order.
+// The columns of panel p (BW columns) hold their rows below the panel in the order after panel p; later
+// panels swapped those rows.  S (kept in sh.perm, which ends as the system's permutation) is the
+// composition of the swaps after panel p, built from the last panel back (row i of the final order is row
+// S(i) of that order).
 template <typename T, int BW>
-__device__ __forceinline__ void factor_sys(BatchShared<T>& sh, T* A, int n, int64_t vo, int64_t* ipiv, int64_t& info) {
-    static_assert(BW == 8 || BW == 16 || BW == PMAX, "panel width");
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    constexpr bool HL = PanelHold<T, BW>::value;
-    double (*L11)[PMAX + 1] = reinterpret_cast<double (*)[PMAX + 1]>(&sh.dblk[0][0]);
-    for (int j0 = 0; j0 < n; j0 += BW) {
-        const int jb = min(BW, n - j0);
-        const int m = n - j0;
-        // rows j0..n-1 of columns j0..n-1 are in place: the panel's permutation starts as identity
-        for (int i = j0 + tid; i < n; i += BT) sh.perm[i] = i;
-        // the panel in registers: thread tid holds logical rows tid + k BT, k < RPT (m <= RPT BT)
-        T v[RPT][BW];
-#pragma unroll
-        for (int k = 0; k < RPT; ++k) {
-            const int r = tid + k * BT;
-#pragma unroll
-            for (int q = 0; q < BW; ++q) v[k][q] = (r < m && q < jb) ? A[(j0 + q) * n + j0 + r] : T(0);
-        }
-        panel_col<T, BW, 0>(sh, v, m, j0, jb, vo, ipiv, info);
-        // the factored panel, rows in LAPACK's order, to A; L11 also to LDS for U12, and L21 to
-        // LDS when it is held (else the trailing update reads it back from A, out of L2)
-#pragma unroll
-        for (int k = 0; k < RPT; ++k) {
-            const int r = tid + k * BT;
-            if (r < m) {
-#pragma unroll
-                for (int q = 0; q < BW; ++q) {
-                    if (q < jb) A[(j0 + q) * n + j0 + r] = v[k][q];
-                    if constexpr (HL) sh.l21[r * 17 + q] = (double)v[k][q];
-                    else if (k == 0 && r < BW) L11[r][q] = (double)v[k][q];
-                }
-            }
-        }
-        __syncthreads();
-        const int c1 = j0 + jb;
-        if (c1 < n) {
-            // the rows below the panel that its swaps move: those it swaps with (at most jb), in
-            // the order of the swaps, each once.  Lane k of wave 0 keeps swap k's row unless an
-            // earlier swap names it; the kept rows are compacted by a ballot.
-            if (wave == 0) {
-                const int p = lane < jb ? sh.piv[j0 + lane] : -1;
-                bool keep = p >= c1;
-                for (int k = 0; k < jb; ++k) keep = keep && !(k < lane && sh.piv[j0 + k] == p);
-                const unsigned long long kept = __ballot(keep);
-                if (keep) sh.chg[__popcll(kept & ((1ull << lane) - 1ull))] = p;
-                if (lane == 0) sh.nchg = __popcll(kept);
-            }
-            __syncthreads();
-            const int nchg = sh.nchg;
-            // here jb == BW (only the last panel is narrower, and it has no columns right of it).
-            // Right of the panel, one thread per column: the interchanges, then U12 = L11^{-1} A12.
-            // The new rows j0..c1-1 come from anywhere at or below j0, so they are read first.
-            // A moved row below c1 takes the old content of a row in [j0, c1) (a row below the
-            // panel only ever receives what a swap brings from the panel's own rows), which is
-            // not written until U12 is, so the moves go in chunks once the U12 rows are read
-            // (slots past nchg repeat the last move).  Offsets within a system fit 32 bits.
-            for (int col = c1 + tid; col < n; col += BT) {
-                const int co = col * n;
-                T u[BW];
-#pragma unroll
-                for (int i = 0; i < BW; ++i) u[i] = A[co + sh.perm[j0 + i]];
-#pragma unroll
-                for (int t0 = 0; t0 < BW; t0 += 8) {
-                    if (t0 < nchg) {
-                        T w[8];
-#pragma unroll
-                        for (int t = 0; t < 8; ++t) w[t] = A[co + sh.perm[sh.chg[min(t0 + t, nchg - 1)]]];
-#pragma unroll
-                        for (int t = 0; t < 8; ++t) A[co + sh.chg[min(t0 + t, nchg - 1)]] = w[t];
-                    }
-                }
-#pragma unroll
-                for (int kk = 0; kk < BW; ++kk) {
-#pragma unroll
-                    for (int i = kk + 1; i < BW; ++i) {
-                        double l;
-                        if constexpr (HL) l = sh.l21[i * 17 + kk];
-                        else l = L11[i][kk];
-                        u[i] = fma(-(T)l, u[kk], u[i]);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);  // L11 read column by column, not all at once
-                }
-#pragma unroll
-                for (int i = 0; i < BW; ++i) A[co + j0 + i] = u[i];
-            }
-            __syncthreads();
-            const int mr = n - c1;
-            T* A22 = A + c1 * n + c1;
-            const T* U12 = A + c1 * n + j0;
-            const T* L21 = A + j0 * n + c1;
-            using acc_t = typename BMma<T>::acc_t;
-            constexpr int KS = BW / 4, NW = BT / 64;
-            // C tile (R x C 16 x 16 blocks at rows rb, columns cb of A22) and its U12 operands
-            // (lane l, k-step s: -U12(4 s + l / 16, column cb + 16 b + l % 16))
-            auto load_c = [&](auto& c, int rb, int cb) {
-                constexpr int R = sizeof(c) / sizeof(c[0]), C = sizeof(c[0]) / sizeof(c[0][0]);
-#pragma unroll
-                for (int a2 = 0; a2 < R; ++a2)
-#pragma unroll
-                    for (int b2 = 0; b2 < C; ++b2)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const int lr = rb + 16 * a2 + (lane & 15), lc = cb + 16 * b2 + BMma<T>::ccol(lane, q);
-                            c[a2][b2][q] = (lr < mr && lc < mr) ? A22[lc * n + lr] : T(0);
-                        }
-            };
-            auto load_u = [&](auto& x, int cb) {
-                constexpr int C = sizeof(x) / sizeof(x[0]);
-#pragma unroll
-                for (int b2 = 0; b2 < C; ++b2) {
-                    const int lc = cb + 16 * b2 + (lane & 15);
-#pragma unroll
-                    for (int k4 = 0; k4 < KS; ++k4) x[b2][k4] = (lc < mr) ? -U12[lc * n + k4 * 4 + (lane >> 4)] : T(0);
-                }
-            };
-            auto store_c = [&](const auto& c, int rb, int cb) {
-                constexpr int R = sizeof(c) / sizeof(c[0]), C = sizeof(c[0]) / sizeof(c[0][0]);
-#pragma unroll
-                for (int a2 = 0; a2 < R; ++a2)
-#pragma unroll
-                    for (int b2 = 0; b2 < C; ++b2)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const int lr = rb + 16 * a2 + (lane & 15), lc = cb + 16 * b2 + BMma<T>::ccol(lane, q);
-                            if (lr < mr && lc < mr) A22[lc * n + lr] = c[a2][b2][q];
-                        }
-            };
-            if constexpr (HL) {
-                // A22 -= L21 U12 on MFMA: tiles of RBT x CBT 16 x 16 blocks, waves round-robin,
-                // L21 from LDS
-                constexpr int RBT = BatchCfg<T>::RB, CBT = BatchCfg<T>::CB;
-                const int tbr = (mr + 16 * RBT - 1) / (16 * RBT), tbc = (mr + 16 * CBT - 1) / (16 * CBT);
-                for (int t = wave; t < tbr * tbc; t += NW) {
-                    const int rb = (t % tbr) * (16 * RBT), cb = (t / tbr) * (16 * CBT);
-                    acc_t acc[RBT][CBT];
-                    T xv[CBT][KS];
-                    load_c(acc, rb, cb);
-                    load_u(xv, cb);
-#pragma unroll
-                    for (int k4 = 0; k4 < KS; ++k4) {
-                        const int kk = k4 * 4 + (lane >> 4);
-                        T yv[RBT];
-#pragma unroll
-                        for (int a2 = 0; a2 < RBT; ++a2) {
-                            const int lr = rb + 16 * a2 + (lane & 15);
-                            yv[a2] = lr < mr ? (T)sh.l21[(BW + lr) * 17 + kk] : T(0);
-                        }
-#pragma unroll
-                        for (int a2 = 0; a2 < RBT; ++a2)
-#pragma unroll
-                            for (int b2 = 0; b2 < CBT; ++b2) acc[a2][b2] = BMma<T>::mma(xv[b2][k4], yv[a2], acc[a2][b2]);
-                    }
-                    store_c(acc, rb, cb);
-                }
-            } else {
-                // A22 -= L21 U12 on MFMA by row blocks of 16 R2 rows: a wave loads its row block
-                // of L21 into registers once and sweeps the column blocks (16 C2 columns) of a
-                // segment of A22's columns; with fewer row blocks than waves, the columns are cut
-                // into segments so that every wave has work.  32-column panels stage U12 in LDS,
-                // UCH columns at a time (FP64: in the held-L21 area; FP32: in a buffer of its
-                // own), so the waves do not read it again from L2 or HBM for every row block;
-                // narrower FP32 panels read it per tile (out of L2).
-                constexpr int R2 = BatchCfg<T>::RB2, C2 = BatchCfg<T>::CB2;
-                constexpr bool HOLDT = BatchCfg<T>::HOLD;
-                constexpr bool STG = BW == PMAX;
-                constexpr int UCH = !STG ? BNMAX : (HOLDT ? (BNMAX * 17) / (BW + 1) / (16 * C2) * (16 * C2) : UCH_F);
-                static_assert(UCH >= 16 * C2 && UCH % (16 * C2) == 0, "a staged U12 chunk holds whole column blocks");
-                auto ubuf = [&]() -> T* {
-                    if constexpr (HOLDT) return reinterpret_cast<T*>(&sh.l21[0]);
-                    else return &sh.ustg[0];
-                };
-                const int tbr = (mr + 16 * R2 - 1) / (16 * R2);
-                for (int cc0 = 0; cc0 < mr; cc0 += UCH) {
-                    const int ncc = min(UCH, mr - cc0);
-                    if constexpr (STG) {
-                        T* Us = ubuf();   // Us[c (BW + 1) + k] = -U12(k, column cc0 + c)
-                        __syncthreads();  // the previous chunk's tiles are done with Us
-                        for (int base = tid; base < ncc * BW; base += 8 * BT) {
-                            T t8[8];
-#pragma unroll
-                            for (int u8 = 0; u8 < 8; ++u8) {
-                                const int idx = base + u8 * BT, c = idx / BW, k = idx - c * BW;
-                                t8[u8] = idx < ncc * BW ? U12[(cc0 + c) * n + k] : T(0);
-                            }
-#pragma unroll
-                            for (int u8 = 0; u8 < 8; ++u8) {
-                                const int idx = base + u8 * BT, c = idx / BW, k = idx - c * BW;
-                                if (idx < ncc * BW) Us[c * (BW + 1) + k] = -t8[u8];
-                            }
-                        }
-                        __syncthreads();
-                    }
-                    const int tbc = (ncc + 16 * C2 - 1) / (16 * C2);
-                    const int nseg = min(tbc, (NW + tbr - 1) / tbr);
-                    const int segw = (tbc + nseg - 1) / nseg;
-                    for (int u = wave; u < tbr * nseg; u += NW) {
-                        const int rb = (u % tbr) * (16 * R2), sg = u / tbr;
-                        T yl[R2][KS];
-#pragma unroll
-                        for (int a2 = 0; a2 < R2; ++a2) {
-                            const int lr = rb + 16 * a2 + (lane & 15);
-#pragma unroll
-                            for (int k4 = 0; k4 < KS; ++k4) yl[a2][k4] = lr < mr ? L21[(k4 * 4 + (lane >> 4)) * n + lr] : T(0);
-                        }
-                        const int cbs = sg * segw, cbe = min(tbc, (sg + 1) * segw);
-                        for (int cbi = cbs; cbi < cbe; ++cbi) {
-                            const int cb = cc0 + cbi * (16 * C2);
-                            acc_t acc[R2][C2];
-                            T xv[C2][KS];
-                            load_c(acc, rb, cb);
-                            if constexpr (STG) {
-                                const T* Us = ubuf();
-#pragma unroll
-                                for (int b2 = 0; b2 < C2; ++b2) {
-                                    const int lc = cb + 16 * b2 + (lane & 15);
-#pragma unroll
-                                    for (int k4 = 0; k4 < KS; ++k4)
-                                        xv[b2][k4] = (lc < mr) ? Us[(lc - cc0) * (BW + 1) + k4 * 4 + (lane >> 4)] : T(0);
-                                }
-                            } else {
-                                load_u(xv, cb);
-                            }
-#pragma unroll
-                            for (int k4 = 0; k4 < KS; ++k4)
-#pragma unroll
-                                for (int a2 = 0; a2 < R2; ++a2)
-#pragma unroll
-                                    for (int b2 = 0; b2 < C2; ++b2)
-                                        acc[a2][b2] = BMma<T>::mma(xv[b2][k4], yl[a2][k4], acc[a2][b2]);
-                            store_c(acc, rb, cb);
-                        }
-                    }
-                }
-            }
-        }
-        __syncthreads();
-    }
-    // The columns of panel p hold their rows below the panel in the order after panel p; later
-    // panels swapped those rows.  S (kept in sh.perm) is the composition of the swaps after panel
-    // p, built from the last panel back (row i of the final order is row S(i) of that order).
+__device__ __forceinline__ void gather_left(BatchShared<T>& sh, T* A, int n) {
+    const int tid = threadIdx.x;
     for (int i = tid; i < n; i += BT) sh.perm[i] = i;
     __syncthreads();
     bool moved = false;  // some later swap exchanges two different rows
@@ -556,18 +189,337 @@ __device__ __forceinline__ void factor_sys(BatchShared<T>& sh, T* A, int n, int6
     }
 }
 
-// s - sum_{k0 <= k < k1} a[k * n] x[k] in the order of k (FP64), sixteen loads in flight.
+// MFMA tiles of the trailing updates: a C tile (R x C 16 x 16 blocks at rows rb, columns cb of the mr x nc
+// matrix at A, leading dimension ld).  S (nullable): the tile's entries are read from there instead, row
+// rb + 16 a2 + l of the tile being row sr[a2] of S (lane l's).
+template <typename T, int R, int C>
+__device__ __forceinline__ void tile_load(typename BMma<T>::acc_t (&c)[R][C], const T* A, const double* S, const int (&sr)[R],
+                                          int ld, int mr, int nc, int rb, int cb, int lane) {
+    if (S) {
+#pragma unroll
+        for (int a2 = 0; a2 < R; ++a2)
+#pragma unroll
+            for (int b2 = 0; b2 < C; ++b2)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int lr = rb + 16 * a2 + (lane & 15), lc = cb + 16 * b2 + BMma<T>::ccol(lane, q);
+                    c[a2][b2][q] = (lr < mr && lc < nc) ? (T)S[lc * ld + sr[a2]] : T(0);
+                }
+        return;
+    }
+#pragma unroll
+    for (int a2 = 0; a2 < R; ++a2)
+#pragma unroll
+        for (int b2 = 0; b2 < C; ++b2)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int lr = rb + 16 * a2 + (lane & 15), lc = cb + 16 * b2 + BMma<T>::ccol(lane, q);
+                c[a2][b2][q] = (lr < mr && lc < nc) ? A[lc * ld + lr] : T(0);
+            }
+}
+template <typename T, int R, int C>
+__device__ __forceinline__ void tile_store(const typename BMma<T>::acc_t (&c)[R][C], T* A, int ld, int mr, int nc, int rb, int cb, int lane) {
+#pragma unroll
+    for (int a2 = 0; a2 < R; ++a2)
+#pragma unroll
+        for (int b2 = 0; b2 < C; ++b2)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int lr = rb + 16 * a2 + (lane & 15), lc = cb + 16 * b2 + BMma<T>::ccol(lane, q);
+                if (lr < mr && lc < nc) A[lc * ld + lr] = c[a2][b2][q];
+            }
+}
+// C (mr x nc at A22) -= L21 U12 for KB columns of L21 (at L21), U12 staged negated in LDS (column c's KB
+// entries at Us + c us), by the waves in turn: a wave keeps a block of 32 rows of L21 in registers and
+// sweeps the 32-column blocks of its segment of the columns, the next tile of C loaded while the
+// current one is formed.  S (nullable): C is read from there, its row r being row map[r] (LDS) of S, and
+// written to A22.
+template <typename T, int KB>
+__device__ __forceinline__ void tiles_update(T* A22, const double* S, const int* map, const T* L21, const T* Us, int us, int ld,
+                                             int mr, int nc) {
+    constexpr int R2 = 2, C2 = 2, KS = KB / 4, NW = BT / 64;
+    using acc_t = typename BMma<T>::acc_t;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // (addresses are formed here, not before the loop over the steps)
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tbr = (mr + 16 * R2 - 1) / (16 * R2), tbc = (nc + 16 * C2 - 1) / (16 * C2);
+    const int nseg = min(tbc, (NW + tbr - 1) / tbr), segw = (tbc + nseg - 1) / nseg;
+    for (int u = wave; u < tbr * nseg; u += NW) {
+        const int rb = (u % tbr) * (16 * R2), sg = u / tbr;
+        const int cbs = sg * segw, cbe = min(tbc, (sg + 1) * segw);
+        if (cbs >= cbe) continue;
+        acc_t acc[R2][C2];
+        int sr[R2];
+#pragma unroll
+        for (int a2 = 0; a2 < R2; ++a2) sr[a2] = S ? map[min(rb + 16 * a2 + (lane & 15), mr - 1)] : 0;
+        tile_load<T, R2, C2>(acc, A22, S, sr, ld, mr, nc, rb, cbs * (16 * C2), lane);
+        T yl[R2][KS];
+#pragma unroll
+        for (int a2 = 0; a2 < R2; ++a2) {
+            const int lr = rb + 16 * a2 + (lane & 15);
+#pragma unroll
+            for (int k4 = 0; k4 < KS; ++k4) yl[a2][k4] = lr < mr ? L21[(k4 * 4 + (lane >> 4)) * ld + lr] : T(0);
+        }
+        for (int cbi = cbs; cbi < cbe; ++cbi) {
+            const int cb = cbi * (16 * C2);
+            acc_t nxt[R2][C2];
+            if (cbi + 1 < cbe) tile_load<T, R2, C2>(nxt, A22, S, sr, ld, mr, nc, rb, cb + 16 * C2, lane);
+            const T* x0 = Us + (cb + (lane & 15)) * us + (lane >> 4);
+#pragma unroll
+            for (int k4 = 0; k4 < KS; ++k4) {
+                T xv[C2];
+#pragma unroll
+                for (int b2 = 0; b2 < C2; ++b2) xv[b2] = x0[16 * b2 * us + 4 * k4];
+#pragma unroll
+                for (int a2 = 0; a2 < R2; ++a2)
+#pragma unroll
+                    for (int b2 = 0; b2 < C2; ++b2) acc[a2][b2] = BMma<T>::mma(xv[b2], yl[a2][k4], acc[a2][b2]);
+            }
+            tile_store<T, R2, C2>(acc, A22, ld, mr, nc, rb, cb, lane);
+#pragma unroll
+            for (int a2 = 0; a2 < R2; ++a2)
+#pragma unroll
+                for (int b2 = 0; b2 < C2; ++b2) acc[a2][b2] = nxt[a2][b2];
+        }
+    }
+}
+
+// The interchanges (sh.perm: row i of the new order is row sh.perm[i] of the old one; sh.chg: the rows below
+// the panels that change) of columns [c0, c1), and U12 = L11^{-1} A12 in their rows j0 .. j0 + 32 NB - 1,
+// L11's strictly lower part given by lf(i, k).  A row of 16 lanes takes one column (two with NB = 2, which
+// share the reads of L11), each lane every 16th of its rows, the solved entries broadcast by DPP.  A row
+// below the panels only ever receives what a swap brings from the panels' own rows, and every row is
+// read before any is written.  S (nullable): the columns are read from there and only the U12 rows are
+// written (the update that follows reads the other rows there too).  neg: also stores -U12 there (entry k of column c at neg[(c - c0) ns + k]).
+template <typename T, int NB, typename LF>
+__device__ __forceinline__ void swap_solve(BatchShared<T>& sh, T* A, const double* S, int n, int j0, int c0, int c1, LF&& lf, T* neg, int ns) {
+    constexpr int NR = 2 * NB, NC = NB, CP = BT / 16;  // rows and columns per lane, columns per round
+    int tid = threadIdx.x;
+    const int nchg = S ? 0 : sh.nchg;
+    for (int b = c0; b < c1; b += CP * NC) {
+        // (hides the thread's number and the LDS contents, or L11's entries would be read before the loop
+        // and spilled)
+        asm volatile("" : "+v"(tid) : : "memory");
+        const int l16 = tid & 15, grp = tid >> 4;
+        T x[NC][NR], w[NC][NR];
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            const int c = b + u * CP + grp, co = c * n;
+            if (S) {
+#pragma unroll
+                for (int t = 0; t < NR; ++t) x[u][t] = c < c1 ? (T)S[co + sh.perm[j0 + l16 + 16 * t]] : T(0);
+            } else {
+#pragma unroll
+                for (int t = 0; t < NR; ++t) {
+                    x[u][t] = c < c1 ? A[co + sh.perm[j0 + l16 + 16 * t]] : T(0);
+                    const int i = l16 + 16 * t;
+                    w[u][t] = (c < c1 && i < nchg) ? A[co + sh.perm[sh.chg[i]]] : T(0);
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            const int c = b + u * CP + grp, co = c * n;
+#pragma unroll
+            for (int t = 0; t < NR; ++t) {
+                const int i = l16 + 16 * t;
+                if (c < c1 && i < nchg) A[co + sh.chg[i]] = w[u][t];
+            }
+        }
+        static_for<0, 16 * NR>([&](auto kc) {
+            constexpr int k = decltype(kc)::value, t0 = k / 16;
+            T bx[NC];
+#pragma unroll
+            for (int u = 0; u < NC; ++u) bx[u] = row_bcast<(k & 15)>(x[u][t0]);
+#pragma unroll
+            for (int t = t0; t < NR; ++t) {
+                const T l = lf(l16 + 16 * t, k);
+#pragma unroll
+                for (int u = 0; u < NC; ++u) {
+                    const T y = fma(-l, bx[u], x[u][t]);
+                    x[u][t] = (t > t0 || l16 > (k & 15)) ? y : x[u][t];
+                }
+            }
+            if ((k & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // L11 read a few columns ahead, not all
+        });
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            const int c = b + u * CP + grp;
+#pragma unroll
+            for (int t = 0; t < NR; ++t)
+                if (c < c1) {
+                    A[c * n + j0 + l16 + 16 * t] = x[u][t];
+                    if (neg) neg[(c - c0) * ns + l16 + 16 * t] = -x[u][t];
+                }
+        }
+    }
+}
+
+// LU with partial pivoting of one n x n system, panels of 32 columns, two per step (column-major, in
+// place; on return A holds L and U in LAPACK's row order and sh.perm the system's permutation).
+// What bounds a large system is its traffic on A22 (16 n^3 / (3 * 64) bytes at FP64; once per 32
+// columns it was twice that) and the panel's chain (about 1.2 us a column, two systems to a CU).
+// src: the matrix where the caller has it, read by the first step (so no copy is made first).
+// 20,000 systems of n in [8, 512], FP64: 58.2 -> 39.1 ms against one update per 32-column panel (8
+// or 16 columns below n = 192), panels with two barriers and two rows through LDS per column, and a
+// copy of the matrices first; of the time 31 % is the panels', 28 % the trailing updates', 13 % the
+// solves', 12 % U12's.  3,000 systems, FP32 factors: 11.2 -> 8.9 ms.
 template <typename T>
-__device__ __forceinline__ double row_dot_sub(double s, const T* a, int n, const double* x, int k0, int k1) {
+__device__ __forceinline__ void factor_sys(BatchShared<T>& sh, T* A, const double* src, int n, int64_t vo, int64_t* ipiv,
+                                           int64_t& info) {
+    int tid = threadIdx.x;
+    PanelLds<T, BT / 64>& pl = *reinterpret_cast<PanelLds<T, BT / 64>*>(sh.wide);
+    constexpr int POFF = (int)((sizeof(PanelLds<T, BT / 64>) + 15) / 16 * 16 / sizeof(T));  // LDS after the panel's
+    constexpr int BST = PW + 2;                                                          // stride of panel B's U12 there
+    static_assert(POFF + PW * BST <= UCH * ust<T>() && SW * (SW + 1) <= UCH * ust<T>(), "LDS of factor_sys");
+    int zero = (int)info;
+    for (int j0 = 0; j0 < n; j0 += SW) {
+        const int c1 = min(j0 + PW, n), c2 = min(j0 + SW, n);
+        const double* S = j0 == 0 ? src : nullptr;  // the first step reads the matrix where the caller has it
+        for (int i = j0 + tid; i < n; i += BT) sh.perm[i] = i;
+        __syncthreads();
+#pragma unroll 1
+        for (int j = j0; j < c2; j += PW) {
+            asm volatile("" : "+v"(tid));  // (as in tiles_update)
+            // the panel of columns [j, j + w), rows j .. n - 1: to A in logical order, its interchanges
+            // composed into sh.perm and applied to the step's first panel when this is the second
+            const int w = min(PW, n - j);
+            int lr[RPT];
+            {
+                T v[RPT][PW];
+                bool live[RPT];
+                int old[RPT];
+#pragma unroll
+                for (int t = 0; t < RPT; ++t) {
+                    const int r = j + tid + t * BT;
+                    live[t] = r < n;
+                    lr[t] = r;
+                    old[t] = r < n ? sh.perm[r] : 0;
+                    if (S && j == 0) {
+#pragma unroll
+                        for (int q = 0; q < PW; ++q) v[t][q] = (r < n && q < w) ? (T)S[q * n + r] : T(0);
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < PW; ++q) v[t][q] = (r < n && q < w) ? A[(j + q) * n + r] : T(0);
+                    }
+                }
+                panel_columns<T, BT, RPT>(v, lr, live, w, j, n, pl, zero, [](const PanelRec<T>* r, int, bool) {
+                    __syncthreads();
+                    return r;
+                });
+                __syncthreads();
+                if (tid == 0) sh.nchg = 0;
+                if (tid < w) {
+                    sh.piv[j + tid] = pl.piv[tid];
+                    if (ipiv) ipiv[vo + j + tid] = (int64_t)pl.piv[tid] + 1;
+                }
+                const int rot = 8 * ((w + 7) / 8);
+#pragma unroll
+                for (int t = 0; t < RPT; ++t) {
+                    if (j + tid + t * BT >= n) continue;
+                    const int top = lr[t] - j;
+                    sh.perm[lr[t]] = old[t];
+                    T* dst = A + j * n + lr[t];
+                    if (top < w) {
+#pragma unroll
+                        for (int q = 0; q < PW; ++q)
+                            if (q < w) dst[q * n] = pl.fin[top].v[q];
+                    } else {
+#pragma unroll
+                        for (int p = 0; p < PW; ++p) {
+                            const int q = (p + rot) & (PW - 1);
+                            if (q < w) dst[q * n] = v[t][p];
+                        }
+                    }
+                }
+            }
+            if (j > j0) {
+                T g[RPT][PW];
+#pragma unroll
+                for (int t = 0; t < RPT; ++t) {
+                    const int r = j + tid + t * BT;
+                    if (r < n && lr[t] != r) {
+#pragma unroll
+                        for (int q = 0; q < PW; ++q) g[t][q] = A[(j0 + q) * n + r];
+                    }
+                }
+                __syncthreads();
+#pragma unroll
+                for (int t = 0; t < RPT; ++t) {
+                    const int r = j + tid + t * BT;
+                    if (r < n && lr[t] != r) {
+#pragma unroll
+                        for (int q = 0; q < PW; ++q) A[(j0 + q) * n + lr[t]] = g[t][q];
+                    }
+                }
+            }
+            __syncthreads();
+            // the rows below the panel that are not in their places of the step's start
+            for (int i = j + w + tid; i < n; i += BT)
+                if (sh.perm[i] != i) sh.chg[atomicAdd(&sh.nchg, 1)] = i;
+            __syncthreads();
+            if (j > j0 || c1 >= n) continue;
+            // the second panel's columns: interchanges, U12 and update of the first
+            T* Ub = sh.wide + POFF;
+            swap_solve<T, 1>(sh, A, S, n, j0, c1, c2, [&](int i, int k) { return pl.fin[i].v[k]; }, Ub, BST);
+            __syncthreads();
+            tiles_update<T, PW>(A + c1 * n + c1, S ? S + c1 * n : nullptr, sh.perm + c1, A + j0 * n + c1, Ub, BST, n, n - c1, c2 - c1);
+            __syncthreads();
+        }
+        if (c2 >= n) break;
+        // the columns right of both panels
+        T* L11 = sh.wide;  // L11[i (SW + 1) + k]
+        for (int i = tid; i < SW * SW; i += BT) {
+            const int r = i & (SW - 1), k = i / SW;
+            L11[r * (SW + 1) + k] = A[(j0 + k) * n + j0 + r];
+        }
+        __syncthreads();
+        swap_solve<T, 2>(sh, A, S, n, j0, c2, n, [&](int i, int k) { return L11[i * (SW + 1) + k]; }, (T*)nullptr, 0);
+        for (int cc = c2; cc < n; cc += UCH) {
+            const int nc = min(UCH, n - cc);
+            __syncthreads();  // L11, or the previous columns' U12, is no longer read; U12 is in memory
+            for (int b0 = tid; b0 < nc * SW; b0 += 8 * BT) {
+                T t8[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int i = b0 + u * BT;
+                    t8[u] = i < nc * SW ? A[(cc + i / SW) * n + j0 + (i & (SW - 1))] : T(0);
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int i = b0 + u * BT;
+                    if (i < nc * SW) sh.wide[(i / SW) * ust<T>() + (i & (SW - 1))] = -t8[u];
+                }
+            }
+            __syncthreads();
+            tiles_update<T, SW>(A + cc * n + c2, S ? S + cc * n : nullptr, sh.perm + c2, A + j0 * n + c2, sh.wide, ust<T>(), n, n - c2, nc);
+        }
+        __syncthreads();
+    }
+    info = zero;
+    gather_left<T, SW>(sh, A, n);
+}
+
+// s - sum_{k0 <= k < k1} a[k * n] x[k] in the order of k (FP64), sixteen loads in flight; ABS: ra += the
+// sum of |a[k * n]| too.
+template <bool ABS, typename T>
+__device__ __forceinline__ double row_dot_sub(double s, const T* a, int n, const double* x, int k0, int k1, double& ra) {
     int k = k0;
     for (; k + 16 <= k1; k += 16) {
         T av[16];
 #pragma unroll
         for (int u = 0; u < 16; ++u) av[u] = a[(int64_t)(k + u) * n];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) s = fma(-(double)av[u], x[k + u], s);
+        for (int u = 0; u < 16; ++u) {
+            s = fma(-(double)av[u], x[k + u], s);
+            if (ABS) ra += fabs((double)av[u]);
+        }
     }
-    for (; k < k1; ++k) s = fma(-(double)a[(int64_t)k * n], x[k], s);
+    for (; k < k1; ++k) {
+        const double av = (double)a[(int64_t)k * n];
+        s = fma(-av, x[k], s);
+        if (ABS) ra += fabs(av);
+    }
     return s;
 }
 
@@ -601,6 +553,7 @@ template <typename T>
 __device__ __forceinline__ void solve_sys(BatchShared<T>& sh, const T* A, int n) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     constexpr int SB = BatchCfg<T>::SB;
+    double dummy = 0.0;
     static_assert((SB * SB) % BT == 0, "a full diagonal block is whole loads per thread");
     double (*D)[SB + 1] = sh.dblk;
     // forward: unit lower L
@@ -617,7 +570,7 @@ __device__ __forceinline__ void solve_sys(BatchShared<T>& sh, const T* A, int n)
             if (lane < kb) sh.xs[k0 + lane] = xv;
         }
         __syncthreads();
-        for (int i = k0 + kb + tid; i < n; i += BT) sh.xs[i] = row_dot_sub(sh.xs[i], A + i, n, sh.xs, k0, k0 + kb);
+        for (int i = k0 + kb + tid; i < n; i += BT) sh.xs[i] = row_dot_sub<false>(sh.xs[i], A + i, n, sh.xs, k0, k0 + kb, dummy);
         __syncthreads();
     }
     // backward: U
@@ -635,7 +588,7 @@ __device__ __forceinline__ void solve_sys(BatchShared<T>& sh, const T* A, int n)
             if (lane < kb) sh.xs[k0 + lane] = xv;
         }
         __syncthreads();
-        for (int i = tid; i < k0; i += BT) sh.xs[i] = row_dot_sub(sh.xs[i], A + i, n, sh.xs, k0, k1);
+        for (int i = tid; i < k0; i += BT) sh.xs[i] = row_dot_sub<false>(sh.xs[i], A + i, n, sh.xs, k0, k1, dummy);
         __syncthreads();
     }
 }
@@ -657,45 +610,18 @@ __global__ __launch_bounds__(BT, BatchCfg<T>::WG * BT / 256) void k_batch_lu(Bat
         T* A = reinterpret_cast<T*>(a.A) + ao;
         const int64_t vo = uniform64(a.voff[sys]);
         int64_t info = 0;
-        const double* A64 = a.A64 ? a.A64 + ao : nullptr;
-        double an = 0.0;  // FP32 path: this thread's rows' largest sum |a_ij| (||A||_inf)
-        if (A64) {  // FP32 path: working copy of the FP64 matrix, by rows, with the row sums
-            for (int i = tid; i < n; i += BT) {
-                double rs = 0.0;
-                int j = 0;
-                for (; j + 16 <= n; j += 16) {
-                    double v[16];
-#pragma unroll
-                    for (int u = 0; u < 16; ++u) v[u] = A64[(j + u) * n + i];
-#pragma unroll
-                    for (int u = 0; u < 16; ++u) {
-                        A[(j + u) * n + i] = (T)v[u];
-                        rs += fabs(v[u]);
-                    }
-                }
-                for (; j < n; ++j) {
-                    const double v = A64[j * n + i];
-                    A[j * n + i] = (T)v;
-                    rs += fabs(v);
-                }
-                an = fmax(an, rs);
-            }
-        }
+        const double* src = a.src ? *a.src : nullptr;
+        if (src) src += ao;
         for (int i = tid; i < n; i += BT) sh.perm[i] = i;
         __syncthreads();
-        const int cfg = a.cfg ? a.cfg[sys] : default_cfg(n);
-        if (cfg == 0) factor_sys<T, 8>(sh, A, n, vo, a.ipiv, info);
-        else if (cfg == 1) factor_sys<T, 16>(sh, A, n, vo, a.ipiv, info);
-        else factor_sys<T, PMAX>(sh, A, n, vo, a.ipiv, info);
+        factor_sys<T>(sh, A, src, n, vo, a.ipiv, info);
         // solve: x = U^{-1} L^{-1} P b
         for (int i = tid; i < n; i += BT) sh.xs[i] = a.b[vo + sh.perm[i]];
         __syncthreads();
         solve_sys<T>(sh, A, n);
-        if (A64) {
+        if constexpr (sizeof(T) == 4) {
             // FP64 refinement
-            double bn = 0.0;
-            for (int i = tid; i < n; i += BT) bn = fmax(bn, fabs(a.b[vo + i]));
-            block_max2(sh, an, bn);
+            double an = 0.0, bn = 0.0;  // ||A||_inf (summed during the first residual), ||b||_inf
             for (int i = tid; i < n; i += BT) sh.xr[i] = sh.xs[i];
             __syncthreads();
             double* rr = &sh.dblk[0][0];  // residual by original row (n <= (SB + 1) SB)
@@ -704,12 +630,20 @@ __global__ __launch_bounds__(BT, BatchCfg<T>::WG * BT / 256) void k_batch_lu(Bat
             while (true) {
                 double rn = 0.0, xn = 0.0;
                 for (int i = tid; i < n; i += BT) {
-                    const double s = row_dot_sub(a.b[vo + i], A64 + i, n, sh.xr, 0, n);
+                    double s, ra = 0.0;
+                    if (it == 0) {
+                        s = row_dot_sub<true>(a.b[vo + i], src + i, n, sh.xr, 0, n, ra);
+                        an = fmax(an, ra);
+                        bn = fmax(bn, fabs(a.b[vo + i]));
+                    } else {
+                        s = row_dot_sub<false>(a.b[vo + i], src + i, n, sh.xr, 0, n, ra);
+                    }
                     rr[i] = s;
                     rn = fmax(rn, fabs(s));
                     xn = fmax(xn, fabs(sh.xr[i]));
                 }
                 block_max2(sh, rn, xn);
+                if (it == 0) block_max2(sh, an, bn);
                 const double den = an * xn + bn;
                 be = den > 0.0 ? rn / den : 0.0;
                 if (!(be > a.tol) || it >= a.maxref || info != 0) break;
@@ -748,7 +682,6 @@ int batch_launch_raw(lsx_ctx* ctx, hipStream_t st, int64_t count, const int32_t*
     a.count = count;
     a.order = order;
     a.n = n;
-    a.cfg = nullptr;
     a.aoff = aoff;
     a.voff = voff;
     a.A = A;
@@ -771,7 +704,6 @@ static void batch_enqueue(lsx_batch* B) {
     a.count = B->count;
     a.order = B->order;
     a.n = B->n;
-    a.cfg = B->cfg;
     a.aoff = B->aoff;
     a.voff = B->voff;
     a.b = B->b;
@@ -784,22 +716,32 @@ static void batch_enqueue(lsx_batch* B) {
     a.maxref = B->maxref;
     a.tol = B->tol;
     a.counter = B->counter;
+    a.src = B->dsrc;
     auto grid = [&](int wg) { return (int)std::max<int64_t>(1, std::min<int64_t>(B->count, (int64_t)B->ctx->num_cus * wg)); };
     if (B->dtype == LSX_F64) {
         a.A = B->A;
-        a.A64 = nullptr;
         hipLaunchKernelGGL(k_batch_lu<double>, dim3(grid(BatchCfg<double>::WG)), dim3(BT), 0, B->stream, a);
     } else {
         a.A = B->A32;
-        a.A64 = B->A;
         hipLaunchKernelGGL(k_batch_lu<float>, dim3(grid(BatchCfg<float>::WG)), dim3(BT), 0, B->stream, a);
     }
 }
 
-int batch_run(lsx_batch* B, const double* dA_src, const double* db, double* dx, bool copy_a) {
+int batch_run(lsx_batch* B, const double* A, const double* db, double* dx) {
     lsx_ctx* ctx = B->ctx;
-    if (copy_a)
-        LSX_HIP(ctx, hipMemcpyAsync(B->A, dA_src, sizeof(double) * B->total_a, hipMemcpyDefault, B->stream));
+    // matrices in this GPU's memory are read where they are (a copy of them took a ninth of a call's
+    // time); others are copied into the handle, where FP64 batches factor them in place
+    const double* src = A;
+    if (!is_device_ptr(ctx->device, A)) {
+        if (!B->A && hipMalloc(&B->A, sizeof(double) * B->total_a) != hipSuccess) {
+            B->A = nullptr;
+            return fail(ctx, LSX_ENOMEM, "lsx_batch_factor_solve: cannot stage the matrices");
+        }
+        LSX_HIP(ctx, hipMemcpyAsync(B->A, A, sizeof(double) * B->total_a, hipMemcpyDefault, B->stream));
+        src = B->dtype == LSX_F64 ? nullptr : B->A;
+    }
+    *B->hsrc = src;
+    LSX_HIP(ctx, hipMemcpyAsync(B->dsrc, B->hsrc, sizeof(src), hipMemcpyHostToDevice, B->stream));
     if (db != B->b) LSX_HIP(ctx, hipMemcpyAsync(B->b, db, sizeof(double) * B->total_v, hipMemcpyDefault, B->stream));
     const int pi = B->prof.begin(B->stream, PK_OTHER, B->flops, sizeof(double) * 2.0 * (double)B->total_a);
     if (B->use_graph) {
@@ -822,27 +764,6 @@ int batch_run(lsx_batch* B, const double* dA_src, const double* db, double* dx, 
     return LSX_OK;
 }
 
-// Per-system panel-width indices from a size-binned table (first bin with n <= upper).
-static int tiles_to_cfg(lsx_ctx* ctx, const std::vector<int32_t>& hn, int nbins, const int32_t* upper,
-                        const int32_t* bw, std::vector<uint8_t>& cfg) {
-    for (int k = 0; k < nbins; ++k)
-        if (bw[k] != 8 && bw[k] != 16 && bw[k] != PMAX)
-            return fail(ctx, LSX_EINVAL, "lsx_batch_set_tiles: panel width %d is not 8, 16 or 32", bw[k]);
-    cfg.resize(hn.size());
-    for (size_t i = 0; i < hn.size(); ++i) {
-        const int n = hn[i];
-        int c = default_cfg(n);
-        for (int k = 0; k < nbins; ++k) {
-            if (n <= upper[k]) {
-                c = bw[k] == 8 ? 0 : (bw[k] == 16 ? 1 : 2);
-                break;
-            }
-        }
-        cfg[i] = (uint8_t)c;
-    }
-    return LSX_OK;
-}
-
 }  // namespace lsx
 
 using namespace lsx;
@@ -852,10 +773,11 @@ static void batch_free(lsx_batch* B) {
     if (B->graph_exec) (void)hipGraphExecDestroy(B->graph_exec);
     (void)hipFree(B->order);
     (void)hipFree(B->n);
-    (void)hipFree(B->cfg);
     (void)hipFree(B->aoff);
     (void)hipFree(B->voff);
     (void)hipFree(B->A);
+    (void)hipFree(B->dsrc);
+    if (B->hsrc) (void)hipHostFree((void*)B->hsrc);
     (void)hipFree(B->A32);
     (void)hipFree(B->b);
     (void)hipFree(B->x);
@@ -895,8 +817,6 @@ int lsx_batch_create(lsx_ctx* ctx, int64_t count, const int64_t* n, int dtype, l
     std::vector<int32_t> order(count);
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(), [&](int32_t x, int32_t y) { return hn[x] > hn[y]; });
-    std::vector<uint8_t> cfg(count);
-    for (int64_t i = 0; i < count; ++i) cfg[i] = (uint8_t)default_cfg(hn[i]);
     DeviceGuard g(ctx);
     lsx_batch* B = new (std::nothrow) lsx_batch();
     if (!B) return LSX_ENOMEM;
@@ -906,7 +826,6 @@ int lsx_batch_create(lsx_ctx* ctx, int64_t count, const int64_t* n, int dtype, l
     B->total_a = ta;
     B->total_v = tv;
     B->flops = flops;
-    B->hn = hn;
     const char* ng = std::getenv("LSX_BATCH_NO_GRAPH");
     B->use_graph = !(ng && ng[0] == '1');
     auto bad = [&](int rc) {
@@ -917,10 +836,11 @@ int lsx_batch_create(lsx_ctx* ctx, int64_t count, const int64_t* n, int dtype, l
     if (hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking) != hipSuccess ||
         hipMalloc(&B->order, sizeof(int32_t) * count) != hipSuccess ||
         hipMalloc(&B->n, sizeof(int32_t) * count) != hipSuccess ||
-        hipMalloc(&B->cfg, sizeof(uint8_t) * count) != hipSuccess ||
         hipMalloc(&B->aoff, sizeof(int64_t) * count) != hipSuccess ||
         hipMalloc(&B->voff, sizeof(int64_t) * count) != hipSuccess ||
-        hipMalloc(&B->A, sizeof(double) * ta) != hipSuccess ||
+        (dtype == LSX_F64 && hipMalloc(&B->A, sizeof(double) * ta) != hipSuccess) ||
+        hipMalloc(&B->dsrc, sizeof(double*)) != hipSuccess ||
+        hipHostMalloc(&B->hsrc, sizeof(double*), hipHostMallocDefault) != hipSuccess ||
         (dtype == LSX_F32 && hipMalloc(&B->A32, sizeof(float) * ta) != hipSuccess) ||
         hipMalloc(&B->b, sizeof(double) * tv) != hipSuccess ||
         hipMalloc(&B->x, sizeof(double) * tv) != hipSuccess || hipMalloc(&B->ipiv, sizeof(int64_t) * tv) != hipSuccess ||
@@ -933,7 +853,6 @@ int lsx_batch_create(lsx_ctx* ctx, int64_t count, const int64_t* n, int dtype, l
         return bad(fail(ctx, LSX_ENOMEM, "lsx_batch_create: device allocation failed"));
     if (hipMemcpy(B->order, order.data(), sizeof(int32_t) * count, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(B->n, hn.data(), sizeof(int32_t) * count, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(B->cfg, cfg.data(), sizeof(uint8_t) * count, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(B->aoff, aoff.data(), sizeof(int64_t) * count, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(B->voff, voff.data(), sizeof(int64_t) * count, hipMemcpyHostToDevice) != hipSuccess)
         return bad(fail(ctx, LSX_EHIP, "lsx_batch_create: upload failed"));
@@ -952,12 +871,9 @@ int lsx_batch_destroy(lsx_batch* B) {
 int lsx_batch_set_tiles(lsx_batch* B, int32_t nbins, const int32_t* upper, const int32_t* bw) {
     if (!B || nbins < 0 || (nbins > 0 && (!upper || !bw))) return LSX_EINVAL;
     lsx_ctx* ctx = B->ctx;
-    DeviceGuard g(ctx);
-    std::vector<uint8_t> cfg;
-    const int rc = tiles_to_cfg(ctx, B->hn, nbins, upper, bw, cfg);
-    if (rc) return rc;
-    LSX_HIP(ctx, hipMemcpyAsync(B->cfg, cfg.data(), sizeof(uint8_t) * B->count, hipMemcpyHostToDevice, B->stream));
-    LSX_HIP(ctx, hipStreamSynchronize(B->stream));
+    for (int k = 0; k < nbins; ++k)
+        if (bw[k] != 8 && bw[k] != 16 && bw[k] != PW)
+            return fail(ctx, LSX_EINVAL, "lsx_batch_set_tiles: panel width %d is not 8, 16 or 32", bw[k]);
     return LSX_OK;
 }
 
@@ -977,7 +893,7 @@ int lsx_batch_factor_solve(lsx_batch* B, const double* A, const double* b, doubl
     if (!B || !A || !b || !x) return LSX_EINVAL;
     lsx_ctx* ctx = B->ctx;
     DeviceGuard g(ctx);
-    int rc = batch_run(B, A, b, x, true);
+    int rc = batch_run(B, A, b, x);
     if (rc) return rc;
     LSX_HIP(ctx, hipMemcpyAsync(B->hinfo, B->info, sizeof(int64_t) * B->count, hipMemcpyDeviceToHost, B->stream));
     if (info) LSX_HIP(ctx, hipMemcpyAsync(info, B->info, sizeof(int64_t) * B->count, hipMemcpyDefault, B->stream));

@@ -1,7 +1,5 @@
 // batch.hpp — handle of a batch of small dense systems resident on the device.
 #pragma once
-#include <vector>
-
 #include "common.hpp"
 
 struct lsx_batch {
@@ -12,12 +10,12 @@ struct lsx_batch {
     hipStream_t stream = nullptr;
     int32_t* order = nullptr;      // systems by decreasing n
     int32_t* n = nullptr;
-    uint8_t* cfg = nullptr;        // per-system panel-width index (tile table)
-    std::vector<int32_t> hn;       // sizes (host)
     int64_t* aoff = nullptr;
     int64_t* voff = nullptr;
-    double* A = nullptr;           // FP64: factors (physical row order) of the last factorization;
-                                   // FP32 path: the FP64 matrices (refinement residuals)
+    double* A = nullptr;           // FP64: factors of the last factorization; FP32 path: the FP64 matrices
+                                   // when the caller's are not in this GPU's memory (made when needed)
+    const double** dsrc = nullptr; // device word: where this call's matrices are (null: in A)
+    const double** hsrc = nullptr; // pinned
     float* A32 = nullptr;          // FP32 path: factors
     double* b = nullptr;
     double* x = nullptr;
@@ -36,6 +34,6 @@ struct lsx_batch {
 };
 
 namespace lsx {
-// Factor and solve every system: A copied from dA_src (device or host) when copy_a.
-int batch_run(lsx_batch* B, const double* dA_src, const double* db, double* dx, bool copy_a);
+// Factor and solve every system (A, db, dx: host or device).
+int batch_run(lsx_batch* B, const double* A, const double* db, double* dx);
 }  // namespace lsx

@@ -1,6 +1,6 @@
 // lu_mixed.hip — mixed-precision LU: factor with FP32 arithmetic (trailing products of three BF16
 // pieces per operand, FP32 accumulation: FP32 accuracy at BF16 MFMA rates) or with BF16 trailing
-// products (two pieces per operand, relative error ~2^-17), with tournament pivoting, then recover
+// products (two pieces per operand, relative error ~2^-17), with partial pivoting, then recover
 // FP64 accuracy by iterative refinement (IR) or GMRES-IR with FP64 residuals.
 //
 // The API shape follows OpenBLAS32MixedLUFactorization (src/openblas.jl:461-543: cast A to
@@ -15,7 +15,6 @@
 
 #include "gemm.hpp"
 #include "gemm_split.hpp"
-#include "calu.hpp"
 #include "lu_driver.hpp"
 #include "residual.hpp"
 
@@ -108,16 +107,7 @@ int mixed_alloc(lsx_lu* lu) {
     const int64_t pw = std::max<int64_t>(resid_part_words(n), cdiv(n, 256) * 64);
     LSX_HIP(ctx, hipMalloc(&m->part, sizeof(double) * pw));
     LSX_HIP(ctx, hipHostMalloc(&m->hpart, sizeof(double) * pw, hipHostMallocDefault));
-    // tournament pivoting: candidate records, broadcast, arrival counter
-    LSX_HIP(ctx, hipMalloc(&lu->calu_cand, sizeof(uint64_t) * CCAND));
-    LSX_HIP(ctx, hipMalloc(&lu->calu_bc, sizeof(uint64_t) * CBC));
-    LSX_HIP(ctx, hipMalloc(&lu->calu_ctr, 256));
-    LSX_HIP(ctx, hipMemsetAsync(lu->calu_cand, 0, sizeof(uint64_t) * CCAND, lu->stream));
-    LSX_HIP(ctx, hipMemsetAsync(lu->calu_bc, 0, sizeof(uint64_t) * CBC, lu->stream));
-    LSX_HIP(ctx, hipMemsetAsync(lu->calu_ctr, 0, 256, lu->stream));
     LSX_HIP(ctx, hipStreamSynchronize(lu->stream));
-    lu->calu_cbase = 0;
-    lu->calu_seq = 1;
     return LSX_OK;
 }
 
@@ -138,11 +128,6 @@ void mixed_free(lsx_lu* lu) {
     (void)hipFree(m->V);
     (void)hipFree(m->w);
     (void)hipFree(m->hvec);
-    (void)hipFree(lu->calu_cand);
-    (void)hipFree(lu->calu_bc);
-    (void)hipFree(lu->calu_ctr);
-    lu->calu_cand = lu->calu_bc = nullptr;
-    lu->calu_ctr = nullptr;
     delete m;
     lu->aux = nullptr;
 }
@@ -169,36 +154,12 @@ static void gemm_lowp(lsx_lu* lu, const float* A, int64_t lda, const float* B, i
     lu->prof.end(lu->cur, pi);
 }
 
-// Block column [jo, jo + jbo) by tournament pivoting (k_block_calu) on lu->cur; false when the
-// block has more rows than one launch holds (the exact panels take it then).
-static bool calu_block(lsx_lu* lu, int64_t jo, int jbo) {
-    const int64_t m = lu->n - jo;
-    const int P = (int)cdiv(m, CBS);
-    if (P > CALU_PMAX) return false;
-    const int np = (int)cdiv(jbo, CW);
-    CaluArgs a;
-    a.A = lu->F32;
-    a.ld = lu->ld32;
-    a.n = lu->n;
-    a.jo = jo;
-    a.JB = jbo;
-    a.P = P;
-    a.ipiv = lu->ipiv;
-    a.dinfo = lu->dinfo;
-    a.cand = lu->calu_cand;
-    a.bc = lu->calu_bc;
-    a.ctr = lu->calu_ctr;
-    a.cbase = lu->calu_cbase;
-    a.seq = lu->calu_seq;
-    a.timeout = wait_ticks(lu->ctx, 5.0);
-    lu->calu_cbase += (uint32_t)(np * P);
-    lu->calu_seq += (uint32_t)np;
-    const int pi = lu->prof.begin(lu->cur, PK_PANEL, (double)m * jbo * jbo, 2.0 * sizeof(float) * (double)m * jbo);
-    hipLaunchKernelGGL(k_block_calu, dim3(P), dim3(CBS), 0, lu->cur, a);
-    lu->prof.end(lu->cur, pi);
-    return true;
-}
-
+// The factors are formed by the FP64 path's driver and panels (getrf_blocked).  Tournament pivoting of
+// a 128-column block in one launch, two exchanges per 32 columns instead of one per column, took 458 us
+// a block at n = 9000; four exact panels with their interchanges and updates take less at every order
+// (factor and refine one right-hand side: n = 300 1291 -> 928 us, 1000 4.08 -> 2.65 ms, 3000 12.7 ->
+// 10.3, 9000 41.6 -> 36.4, 14000 71.6 -> 64.1), since a panel's columns cost 1 to 1.5 us up to 1024
+// rows and an exchange 1.5 us more above.
 int mixed_getrf(lsx_lu* lu) {
     lsx_ctx* ctx = lu->ctx;
     MixedState* m = ms(lu);
@@ -215,15 +176,7 @@ int mixed_getrf(lsx_lu* lu) {
                    int64_t N, int64_t K, int mode) { gemm_f32(lu, A, lda, B, ldb, C, ldc, M, N, K, mode); };
     auto gu = [lu](const float* A, int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc, int64_t M,
                    int64_t N, int64_t K, int) { gemm_lowp(lu, A, lda, B, ldb, C, ldc, M, N, K); };
-    if (lu->calu_seq > 0xF0000000u || lu->calu_cbase > 0xF0000000u) {
-        LSX_HIP(ctx, hipMemsetAsync(lu->calu_ctr, 0, 256, lu->stream));
-        LSX_HIP(ctx, hipMemsetAsync(lu->calu_cand, 0, sizeof(uint64_t) * CCAND, lu->stream));
-        LSX_HIP(ctx, hipMemsetAsync(lu->calu_bc, 0, sizeof(uint64_t) * CBC, lu->stream));
-        lu->calu_cbase = 0;
-        lu->calu_seq = 1;
-    }
-    auto bf = [lu](int64_t jo, int jbo) { return calu_block(lu, jo, jbo); };
-    const int rc = getrf_blocked<float>(lu, lu->F32, lu->ld32, m->DL, m->DU, gu, gt, bf);
+    const int rc = getrf_blocked<float>(lu, lu->F32, lu->ld32, m->DL, m->DU, gu, gt);
     double an = 0.0;
     for (int64_t i = 0; i < nb; ++i) an = nanmax(an, m->hpart[i]);
     m->anorm_h = an;

@@ -5,6 +5,7 @@
 
 namespace lsx {
 constexpr int NBO = 128;      // outer block: K of the trailing MFMA update
+constexpr int64_t MTAIL = 3072, MWIDE = 8192;  // rows left: one last block up to, blocks of 2 NBO above
 constexpr int PMAX = 128;     // max workgroups cooperating on one panel (512 rows each)
 constexpr int REC = 6 + 2 * PW;   // words of one FP64 exchange record: key lo/hi, row, pad, inverse, data
 constexpr int RECS = 72;          // record stride in the exchange buffer (words)
@@ -37,9 +38,9 @@ struct lsx_lu {
     int64_t* dinfo = nullptr;    // device: [0] info, [1] error flags
     int64_t* hinfo = nullptr;    // pinned host mirror of dinfo
     uint64_t* slots = nullptr;   // panel exchange records
-    int64_t* plist = nullptr;    // permutation lists: inner [0, 4*NBO), outer by block parity
-                                 // [4*NBO, 8*NBO) and [8*NBO, 12*NBO)
-    int* pcount = nullptr;       // [0] inner T, [1], [2] outer T by block parity
+    int64_t* plist = nullptr;    // permutation lists of 4*NBO words: a panel's, then by outer block
+                                 // parity two (one per NBO columns of the block)
+    int* pcount = nullptr;       // their lengths
     int* pinv = nullptr;         // per outer block: inverse of the row map after that block
                                  // (the deferred row interchanges of the L columns)
     uint64_t* tmsg = nullptr;    // triangular-solve block messages (nblk * TMW words)

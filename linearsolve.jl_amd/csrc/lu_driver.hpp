@@ -81,29 +81,46 @@ int getrf_blocked(lsx_lu* lu, T* F, int64_t ld, T* DL, T* DU, GU gemm_upd, GT ge
     int64_t* il = lu->plist;
     int* ic = lu->pcount;
 
+    // The widths of the outer blocks, from the rows m that are left:
+    //   m <= MTAIL: all the columns left are one block, every panel updating all of them (K = PW), on
+    //     every CU.  The trailing matrix is then small enough for its update to take 5 to 20 us a panel,
+    //     and a block of NBO would spend 110 us between its last panel and the next block's first (lists,
+    //     interchanges and TRSM of the next columns, inverses).  n = 500 1044 -> 835 us, 1024 2316 -> 1815,
+    //     3001 10.2 -> 9.2 ms, 16384 (limit 1024 -> 3072) 101.2 -> 100.5; a limit of 4096 gives nothing more;
+    //   m > MWIDE: 2 NBO columns, so that the trailing matrix is read and written half as often, where
+    //     its update and not the panels' chain is the longer of the two: n = 16384 109.8 -> 100.6 ms, 12000
+    //     58.2 -> 55.8, 9000 no change (limits of 7000 to 8192 measure the same, 11000 gives 102.2 and 57.6);
+    //   else NBO.
+    auto width = [&](int64_t jo) -> int {
+        const int64_t m = n - jo;
+        return (int)(m <= MTAIL ? m : m > MWIDE ? 2 * NBO : NBO);
+    };
+    auto plist = [&](int par, int h) { return lu->plist + (1 + 2 * par + h) * 4 * NBO; };
+    auto pcount = [&](int par, int h) { return lu->pcount + 1 + 2 * par + h; };
+    auto build_list = [&](int64_t k0, int kb, int par, int h) {
+        hipLaunchKernelGGL(k_perm_build, dim3(1), dim3(256), 0, lu->cur, lu->ipiv, k0, kb, plist(par, h), pcount(par, h));
+    };
     // factorization of outer block [jo, jo + jbo) (its columns already updated): inner panels,
-    // their interchanges and updates inside the block, diagonal-block inverses, the block's
-    // interchange list (parity par) and the row map
+    // their interchanges (also of the row map) and updates inside the block, the block's interchange
+    // lists (parity par; of a last block only for undeferred interchanges), diagonal-block inverses
     auto panel_block = [&](int64_t jo, int jbo, int par) -> int {
         for (int64_t ji = jo; ji < jo + jbo; ji += PW) {
             const int W = (int)std::min<int64_t>(PW, jo + jbo - ji);
             launch_panel_t<T>(lu, F, ld, ji, W, il, ic);
             const int64_t nleft = ji - jo, nright = jo + jbo - ji - W;
-            if (nleft + nright > 0) {
-                const int pi = lu->prof.begin(lu->cur, PK_LASWP, (double)W * W * nright,
-                                              sizeof(T) * 4.0 * W * (nleft + nright));
-                hipLaunchKernelGGL(k_inner_swap<T>, dim3((unsigned)cdiv(nleft + nright, ICW)), dim3(256), 0, lu->cur, F,
-                                   ld, n, ji, W, il, ic, jo, (int)nleft, ji + W, jo + jbo);
-                lu->prof.end(lu->cur, pi);
-            }
+            const int pi = lu->prof.begin(lu->cur, PK_LASWP, (double)W * W * nright,
+                                          sizeof(T) * 4.0 * W * (nleft + nright));
+            hipLaunchKernelGGL(k_inner_swap<T>, dim3((unsigned)std::max<int64_t>(1, cdiv(nleft + nright, ICW))), dim3(256),
+                               0, lu->cur, F, ld, n, ji, W, il, ic, jo, (int)nleft, ji + W, jo + jbo, lu->perm);
+            lu->prof.end(lu->cur, pi);
             if (nright > 0)
                 gemm_upd(F + ji * ld + (ji + W), ld, F + (ji + W) * ld + ji, ld, F + (ji + W) * ld + (ji + W), ld,
                          n - ji - W, nright, W, 0);
         }
-        // the block's interchange list first: the update stream applies it to the columns right
-        // of the block while the diagonal-block inverses are formed
-        hipLaunchKernelGGL(k_perm_build, dim3(1), dim3(256), 0, lu->cur, lu->ipiv, jo, jbo,
-                           lu->plist + (4 + 4 * par) * NBO, lu->pcount + 1 + par, lu->perm);
+        // the interchange lists first: the update stream applies them to the columns right of the
+        // block while the diagonal-block inverses are formed
+        if (jo + jbo < n)
+            for (int k = 0; k < jbo; k += NBO) build_list(jo + k, std::min(NBO, jbo - k), par, k / NBO);
         LSX_HIP(ctx, hipEventRecord(lu->ev_perm, lu->cur));
         const int64_t b0 = jo / DB, nbk = cdiv(jbo, DB);
         const int pi = lu->prof.begin(lu->cur, PK_OTHER, 0.0, 0.0);
@@ -111,12 +128,17 @@ int getrf_blocked(lsx_lu* lu, T* F, int64_t ld, T* DL, T* DU, GU gemm_upd, GT ge
         lu->prof.end(lu->cur, pi);
         return LSX_OK;
     };
-    // the inverse of the row map after block jo, for the deferred L-column gather; launched after
-    // the block's ev_panel so that the update stream does not wait for it
-    auto inv_perm = [&](int64_t jo) {
-        if (defer)
+    // the inverse of the row map after block [jo, jo + jbo), for the deferred L-column gather; launched
+    // after the block's ev_panel so that the update stream does not wait for it
+    auto inv_perm = [&](int64_t jo, int jbo) {
+        if (defer && jo + jbo < n)
             hipLaunchKernelGGL(k_inv_perm, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, lu->cur, lu->perm,
-                               lu->pinv + (jo / NBO) * n, n);
+                               lu->pinv + (jo / NBO) * n, jbo / NBO, n);
+    };
+    auto interchange = [&](int64_t jo, int jbo, int par, int64_t c0, int64_t c1) {
+        for (int k = 0; k < jbo; k += NBO)
+            launch_laswp_t<T>(lu, F, ld, jo + k, std::min(NBO, jbo - k), plist(par, k / NBO), pcount(par, k / NBO), c0,
+                              c1, 0);
     };
     // interchanges, U12 = L11^{-1} A12 and A22 -= L21 U12 of block [jo, jo + jbo) on columns
     // [c0, c1); wait_inv: the block's diagonal-block inverses may still be in the making on the
@@ -124,41 +146,54 @@ int getrf_blocked(lsx_lu* lu, T* F, int64_t ld, T* DL, T* DU, GU gemm_upd, GT ge
     auto update = [&](int64_t jo, int jbo, int par, int64_t c0, int64_t c1, bool wait_inv) -> int {
         if (c1 <= c0) return LSX_OK;
         const int64_t r1 = jo + jbo, nc = c1 - c0;
-        launch_laswp_t<T>(lu, F, ld, jo, jbo, lu->plist + (4 + 4 * par) * NBO, lu->pcount + 1 + par, c0, c1, 0);
+        interchange(jo, jbo, par, c0, c1);
         if (wait_inv && lu->cur != s1) LSX_HIP(ctx, hipStreamWaitEvent(lu->cur, lu->ev_panel, 0));
-        // L11 = [L1 0; L2 L3] (64-blocks): X1 = L1^{-1} A12[0:64];  A12[64:] -= L2 X1;  X2 = L3^{-1} A12[64:]
-        T* A12 = F + c0 * ld + jo;
-        const int64_t b0 = jo / DB;
-        const int64_t h1 = std::min<int64_t>(DB, jbo), h2 = jbo - h1;
-        gemm_trsm(DL + b0 * DB * DB, DB, A12, ld, A12, ld, h1, nc, h1, 1);
-        if (h2 > 0) {
-            gemm_trsm(F + jo * ld + jo + DB, ld, A12, ld, A12 + DB, ld, h2, nc, DB, 0);
-            gemm_trsm(DL + (b0 + 1) * DB * DB, DB, A12 + DB, ld, A12 + DB, ld, h2, nc, h2, 1);
+        // by 64-blocks of L11: X_i = L_ii^{-1} A12_i, then the rows below it in the block -= L_ki X_i
+        for (int64_t k = 0; k < jbo; k += DB) {
+            T* Ai = F + c0 * ld + jo + k;
+            const int64_t h = std::min<int64_t>(DB, jbo - k), below = jbo - k - h;
+            gemm_trsm(DL + (jo + k) / DB * DB * DB, DB, Ai, ld, Ai, ld, h, nc, h, 1);
+            if (below > 0) gemm_trsm(F + (jo + k) * ld + jo + k + DB, ld, Ai, ld, Ai + DB, ld, below, nc, DB, 0);
         }
-        gemm_upd(F + jo * ld + r1, ld, A12, ld, F + c0 * ld + r1, ld, n - r1, nc, jbo, 0);
+        gemm_upd(F + jo * ld + r1, ld, F + c0 * ld + jo, ld, F + c0 * ld + r1, ld, n - r1, nc, jbo, 0);
         return LSX_OK;
     };
 
-    int rc_ = panel_block(0, (int)std::min<int64_t>(NBO, n), 0);
+    int jbo = width(0);
+    int rc_ = panel_block(0, jbo, 0);
     if (rc_) return rc_;
     LSX_HIP(ctx, hipEventRecord(lu->ev_panel, s0));
-    inv_perm(0);
-    int par = 0;
-    for (int64_t jo = 0; jo < n; jo += NBO, par ^= 1) {
-        const int jbo = (int)std::min<int64_t>(NBO, n - jo);
+    inv_perm(0, jbo);
+    int par = 0, jbn = 0;
+    int64_t deferred = 0;  // columns whose interchanges of later blocks are left to the end
+    for (int64_t jo = 0; jo < n; jo += jbo, jbo = jbn, par ^= 1) {
         const int64_t c1 = jo + jbo;
         lu->cur = s0;
-        if (!defer && jo > 0)
-            launch_laswp_t<T>(lu, F, ld, jo, jbo, lu->plist + (4 + 4 * par) * NBO, lu->pcount + 1 + par, 0, jo, 0);
+        if (!defer && jo > 0) {
+            if (c1 < n) interchange(jo, jbo, par, 0, jo);
+            else
+                for (int64_t k = jo; k < n; k += NBO) {  // the last block made no lists
+                    const int kb = (int)std::min<int64_t>(NBO, n - k);
+                    build_list(k, kb, par, 0);
+                    launch_laswp_t<T>(lu, F, ld, k, kb, plist(par, 0), pcount(par, 0), 0, jo, 0);
+                }
+        }
         if (c1 >= n) break;
-        const int jbn = (int)std::min<int64_t>(NBO, n - c1);
+        deferred = c1;
+        jbn = width(c1);
+        const bool last = c1 + jbn >= n;  // nothing to overlap the last block with: it takes every CU
         if ((rc_ = update(jo, jbo, par, c1, c1 + jbn, true))) return rc_;
-        LSX_HIP(ctx, hipEventRecord(lu->ev_next, s0));
-        LSX_HIP(ctx, hipStreamWaitEvent(s1, lu->ev_next, 0));
-        lu->cur = s1;
+        if (last && s1 != s0) {  // its interchanges move the row map, which the last inv_perm on s1 reads
+            LSX_HIP(ctx, hipEventRecord(lu->ev_next, s1));
+            LSX_HIP(ctx, hipStreamWaitEvent(s0, lu->ev_next, 0));
+        } else if (!last) {
+            LSX_HIP(ctx, hipEventRecord(lu->ev_next, s0));
+            LSX_HIP(ctx, hipStreamWaitEvent(s1, lu->ev_next, 0));
+            lu->cur = s1;
+        }
         if ((rc_ = panel_block(c1, jbn, par ^ 1))) return rc_;
-        LSX_HIP(ctx, hipEventRecord(lu->ev_panel, s1));
-        inv_perm(c1);
+        LSX_HIP(ctx, hipEventRecord(lu->ev_panel, lu->cur));
+        inv_perm(c1, jbn);
         lu->cur = s0;
         if ((rc_ = update(jo, jbo, par, c1 + jbn, n, false))) return rc_;
         // the next block's interchange list (ev_perm) is all the next iteration's first step
@@ -171,11 +206,10 @@ int getrf_blocked(lsx_lu* lu, T* F, int64_t ld, T* DL, T* DU, GU gemm_upd, GT ge
         LSX_HIP(ctx, hipEventRecord(lu->ev_next, s1));
         LSX_HIP(ctx, hipStreamWaitEvent(s0, lu->ev_next, 0));
     }
-    if (defer && n > NBO) {
-        const int64_t ncols = (cdiv(n, NBO) - 1) * NBO;
+    if (defer && deferred > 0) {
         const size_t lds = sizeof(T) * (size_t)(n - NBO);
         const int pi = lu->prof.begin(s0, PK_LASWP, 0.0, 2.0 * sizeof(T) * (double)n * n / 2);
-        hipLaunchKernelGGL(k_left_gather<T>, dim3((unsigned)ncols), dim3(256), lds, s0, F, ld, n,
+        hipLaunchKernelGGL(k_left_gather<T>, dim3((unsigned)deferred), dim3(256), lds, s0, F, ld, n,
                            (const int*)lu->perm, (const int*)lu->pinv);
         lu->prof.end(s0, pi);
     }

@@ -186,15 +186,16 @@ constexpr int ICW = 16;
 template <typename T>
 __global__ __launch_bounds__(256) void k_inner_swap(T* __restrict A, int64_t ld, int64_t n, int64_t j0, int W,
                                                     const int64_t* __restrict list, const int* __restrict count,
-                                                    int64_t c0, int nl, int64_t cr, int64_t cend) {
+                                                    int64_t c0, int nl, int64_t cr, int64_t cend,
+                                                    int* __restrict perm) {
     __shared__ int s_dst[2 * PW], s_src[2 * PW];
     __shared__ T s_buf[2 * PW][ICW + 1];
     __shared__ T s_L[PW][PW + 1];
     const int t = threadIdx.x;
     const int first = (int)blockIdx.x * ICW;
-    const bool right = first >= nl;
-    const int64_t cb = right ? cr + (first - nl) : c0 + first;
-    const int ncol = right ? (int)min((int64_t)ICW, cend - cb) : ICW;
+    const int64_t cb = first >= nl ? cr + (first - nl) : c0 + first;
+    const int ncol = first >= nl ? (int)min((int64_t)ICW, cend - cb) : ICW;
+    const bool right = first >= nl && ncol > 0;
     const int M = min(*count, 2 * PW);
     if (t < M) {
         // rows of [j0, n); clamped, since after a wait that gave up the list may hold anything
@@ -207,6 +208,8 @@ __global__ __launch_bounds__(256) void k_inner_swap(T* __restrict A, int64_t ld,
         for (int u = 0; u < 4; ++u) lv[u] = A[(j0 + (t >> 5) + 8 * u) * ld + j0 + (t & 31)];
     }
     __syncthreads();
+    const bool map = blockIdx.x == 0 && t < M;  // the row map moves as one more column
+    const int pv = map ? perm[s_src[t]] : 0;
     T v[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -220,6 +223,7 @@ __global__ __launch_bounds__(256) void k_inner_swap(T* __restrict A, int64_t ld,
         for (int u = 0; u < 4; ++u) s_L[t & 31][(t >> 5) + 8 * u] = lv[u];
     }
     __syncthreads();  // every source row read before any row is written
+    if (map) perm[s_dst[t]] = pv;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
         const int i = t & 63, cc = (t >> 6) + 4 * u;
@@ -253,7 +257,7 @@ __global__ __launch_bounds__(256) void k_inner_swap(T* __restrict A, int64_t ld,
 // ------------------------------------------------------------------------------------------
 // Row permutation of the LAPACK swap sequence ipiv[k0 .. k0+kb) (ipiv[k] >= k, 1-based) as a
 // list of (destination row, source row) pairs: after the swaps, row dest[i] holds the former
-// row src[i].  Optionally applies the same permutation to perm[] (row i of P*A = row perm[i]).
+// row src[i].
 // One workgroup of 256 threads; kb <= 128.
 // Positions 0..kb-1 stand for rows k0..k0+kb-1, positions kb..T-1 for the distinct pivot rows
 // below the block (first occurrences, in order); swap u exchanges positions u and pos[u] >= u.
@@ -261,15 +265,13 @@ __global__ __launch_bounds__(256) void k_inner_swap(T* __restrict A, int64_t ld,
 // position v held just before swap v, so every final label follows such links backwards in time
 // independently of the others: no sequential replay of the swaps.
 static __global__ __launch_bounds__(256) void k_perm_build(const int64_t* __restrict ipiv, int64_t k0, int kb,
-                                                    int64_t* __restrict list, int* __restrict count,
-                                                    int* __restrict perm) {
+                                                    int64_t* __restrict list, int* __restrict count) {
     __shared__ int64_t s_p[NBO];
     __shared__ int s_first[NBO];
     __shared__ int s_pos[NBO];
     __shared__ int s_prev[NBO];         // last earlier swap with the same target position
     __shared__ int s_last[2 * NBO];     // last swap targeting each position
     __shared__ int64_t s_rows[2 * NBO];
-    __shared__ int s_pv[2 * NBO];
     const int t = threadIdx.x;
     const int64_t top = k0 + kb;
     if (t < kb) s_p[t] = ipiv[k0 + t] - 1;
@@ -325,17 +327,14 @@ static __global__ __launch_bounds__(256) void k_perm_build(const int64_t* __rest
         list[2 * NBO + t] = s_rows[lab];
     }
     if (t == 0) *count = T;
-    if (perm) {
-        if (t < T) s_pv[t] = perm[s_rows[lab]];
-        __syncthreads();
-        if (t < T) perm[s_rows[t]] = s_pv[t];
-    }
 }
 
-// Inverse of a row map: inv[perm[r]] = r.
-static __global__ void k_inv_perm(const int* __restrict perm, int* __restrict inv, int64_t n) {
+// Inverse of a row map, inv[perm[r]] = r, in each of nb consecutive maps of n.
+static __global__ void k_inv_perm(const int* __restrict perm, int* __restrict inv, int nb, int64_t n) {
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < n) inv[perm[r]] = (int)r;
+    if (r >= n) return;
+    const int p = perm[r];
+    for (int b = 0; b < nb; ++b) inv[b * n + p] = (int)r;
 }
 
 // Deferred row interchanges of the L columns.  While the matrix is factored, the interchanges of

@@ -36,7 +36,14 @@ static void launch_panel_t(lsx_lu* lu, T* F, int64_t ld, int64_t j0, int W, int6
     a.P = (int)cdiv(m_rows, 1024);
     if (m_rows <= 256) hipLaunchKernelGGL((k_panel<T, 256, 1>), dim3(1), dim3(256), 0, lu->cur, a);
     else if (m_rows <= 512) hipLaunchKernelGGL((k_panel<T, 512, 1>), dim3(1), dim3(512), 0, lu->cur, a);
-    else hipLaunchKernelGGL((k_panel<T, 512, 2>), dim3(a.P), dim3(512), 0, lu->cur, a);
+    else if (sizeof(T) == 8 || m_rows <= 1024 || m_rows > 2048)
+        hipLaunchKernelGGL((k_panel<T, 512, 2>), dim3(a.P), dim3(512), 0, lu->cur, a);
+    else if constexpr (sizeof(T) == 4) {
+        // FP32 rows leave the registers for 2048 rows in one workgroup: still no exchange (n = 2000 with
+        // its refinement 5.26 -> 4.54 ms); two or more such workgroups are slower than twice as many of 1024
+        a.P = 1;
+        hipLaunchKernelGGL((k_panel<T, 1024, 2>), dim3(1), dim3(1024), 0, lu->cur, a);
+    }
     lu->prof.end(lu->cur, pi);
 }
 

@@ -43,10 +43,10 @@ struct PanelArgs {
 template <typename T, int NT, int RPT>
 __global__ __launch_bounds__(NT) void k_panel(PanelArgs<T> a) {
     constexpr int NW = NT / 64;
-    static_assert(NW <= 8, "the search among the waves takes eight lanes");
     constexpr int WPE = Words<T>::W;
     constexpr int HW = panel_head<T>();
-    constexpr int PR = PMAX / 2;  // workgroups of 1024 rows
+    constexpr int PR = PMAX / 2;                 // workgroups of 1024 rows
+    constexpr bool MULTI = NT * RPT == 1024;     // the shape that several workgroups share a panel in
     const int tid = threadIdx.x, w = blockIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r0 = (int)a.j0 + w * NT * RPT + tid;
     T* col0 = a.A + a.j0 * a.ld;
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(NT) void k_panel(PanelArgs<T> a) {
     // would be waited for by the next global access (or the next wait the compiler places)
     int info = 0;
     __shared__ PanelLds<T, NW> sh;
-    __shared__ PanelRec<T> s_all[RPT > 1 ? PR : 1];
+    __shared__ PanelRec<T> s_all[MULTI ? PR : 1];
     if (w == 0 && tid == 0) {
         __hip_atomic_store(a.count, a.W, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // in memory before any workgroup counts its moved rows (which all have seen a message, or
@@ -74,7 +74,7 @@ __global__ __launch_bounds__(NT) void k_panel(PanelArgs<T> a) {
     }
     const int P = a.P;
     auto exchange = [&](const PanelRec<T>* own, int col, bool sender) -> const PanelRec<T>* {
-        if (RPT == 1 || P == 1) {
+        if (!MULTI || P == 1) {
             __syncthreads();
             return own;
         }

@@ -110,7 +110,7 @@ template <typename T, int NT, int RPT, typename EX>
 __device__ __forceinline__ void panel_columns(T (&v)[RPT][PW], int (&lr)[RPT], bool (&live)[RPT], int W, int j0, int m,
                                               PanelLds<T, NT / 64>& sh, int& info, EX&& exchange) {
     constexpr int NW = NT / 64;
-    static_assert(NW == 2 || NW == 4 || NW == 8, "the search among the waves takes two, four or eight candidates");
+    static_assert(NW == 2 || NW == 4 || NW == 8 || NW == 16, "the search among the waves takes up to sixteen candidates");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 #pragma unroll 1
     for (int g = 0; g < PW / 8; ++g) {

@@ -105,15 +105,16 @@ __device__ __forceinline__ int wave_argmax32(uint64_t u, int lr) {
     }
     return __ffsll((unsigned long long)tie) - 1;
 }
-// The same over N candidates (N = 2, 4 or 8), candidate l & (N - 1) in lane l.
+// The same over N candidates (N = 2, 4, 8 or 16), candidate l & (N - 1) in lane l.
 template <int N>
 __device__ __forceinline__ int wave_argmax_rep(uint64_t u, int lr) {
-    static_assert(N == 2 || N == 4 || N == 8, "two, four or eight candidates");
+    static_assert(N == 2 || N == 4 || N == 8 || N == 16, "up to a row of lanes");
     constexpr uint64_t first = (1ull << N) - 1;
     auto mx = [](uint32_t x) {
         x = dpp_max_u32<0xB1>(x);
         if constexpr (N > 2) x = dpp_max_u32<0x4E>(x);
         if constexpr (N > 4) x = dpp_max_u32<0x141>(x);
+        if constexpr (N > 8) x = dpp_max_u32<0x140>(x);
         return (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
     };
     const uint32_t hi = (uint32_t)(u >> 32);

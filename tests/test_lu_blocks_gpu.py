@@ -1,5 +1,6 @@
 """The blocked LU where its outer blocks change width: one last block of up to 3072 rows, blocks of 128
-columns above, of 256 above 8192 rows; and orders whose L interchanges are not deferred (above 18432)."""
+columns above, of 256 above 8192 rows; orders whose L interchanges are not deferred (above 18432); and FP32 panels of up
+to 2048 rows in one workgroup."""
 import numpy as np
 import pytest
 import scipy.linalg.lapack as lapack
@@ -28,7 +29,7 @@ def test_factors_across_block_widths(lsx, n):
     assert (PA - L @ U).abs().max() <= 4 * n * EPS * (L.abs() @ U.abs()).max()
 
 
-@pytest.mark.parametrize("n,dtype", [(3073, "f32"), (8200, "f32"), (8200, "bf16"), (18560, "f64")])
+@pytest.mark.parametrize("n,dtype", [(1025, "f32"), (2048, "f32"), (2049, "f32"), (3073, "f32"), (8200, "f32"), (8200, "bf16"), (18560, "f64")])
 def test_solves_across_block_widths(lsx, n, dtype):
     print(f"blocks solve n={n} {dtype}", flush=True)
     rng = np.random.default_rng(n)

@@ -2,6 +2,7 @@
 // element type (FP64 for the plain path, FP32 for the mixed path).
 #pragma once
 #include "common.hpp"
+#include "lu.hpp"
 
 namespace lsx {
 
@@ -165,6 +166,88 @@ static void launch_gemm(hipStream_t st, const T* A, int64_t lda, const T* B, int
     const int64_t T_ = cdiv(M, BM) * cdiv(N, BN);
     hipLaunchKernelGGL((k_gemm<T, MODE, BM, BN, NT>), dim3((unsigned)(8 * cdiv(T_, 8))), dim3(NT), 0, st, A, lda, B,
                        ldb, C, ldc, (int)M, (int)N, (int)K);
+}
+
+// C -= A B with K = 32 (A: M x 32, B: 32 x N, C: M x N, one leading dimension): a panel's update inside
+// its outer block, on the chain of the panels, where the time is latency and not rate.  A 64 x 64 tile per
+// workgroup, four waves of 32 x 32, and every load of a tile (A, B and C) issued before the first is
+// waited for; the staged kernel above has three dependent round trips at K = 32.  FP32 products and sums
+// also in the mixed path.  n = 3001 9.07 -> 8.91 ms, 1024 1.80 -> 1.78; mixed, against the split-BF16
+// kernel (128 x 128 tiles, 12 to 15 us), n = 3000 7.87 -> 7.55, 9000 33.7 -> 32.9.
+constexpr int IBK = 32, IBM = 64;
+template <typename T>
+__global__ __launch_bounds__(256) void k_gemm_inner(const T* __restrict Ag, const T* Bg, T* Cg, int64_t ld, int M, int N) {
+    typedef GemmMma<T> G;
+    const int TM = (M + IBM - 1) / IBM, TN = (N + IBM - 1) / IBM, NTL = TM * TN;
+    // a contiguous range of the column-by-column tile order per XCD, as k_gemm
+    const int per = (NTL + 7) / 8, tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || tile >= NTL) return;
+    const int row0 = tile % TM * IBM, col0 = tile / TM * IBM;
+    __shared__ T As[IBK][IBM + 1];
+    __shared__ T Bs[IBK][IBM + 1];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wr = row0 + 32 * (wave & 1) + (lane & 15), wc = col0 + 32 * (wave >> 1);
+    T ra[8], rb[8], cv[2][2][4];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const int r = row0 + (tid & 63), k = (tid >> 6) + 4 * u;
+        ra[u] = r < M ? Ag[(int64_t)k * ld + r] : T(0);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const int k = tid & 31, c = col0 + (tid >> 5) + 8 * u;
+        rb[u] = c < N ? Bg[(int64_t)c * ld + k] : T(0);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int r = wr + 16 * j, c = wc + 16 * i + G::ccol(lane, q);
+                cv[i][j][q] = (r < M && c < N) ? Cg[(int64_t)c * ld + r] : T(0);
+            }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        As[(tid >> 6) + 4 * u][tid & 63] = ra[u];
+        Bs[tid & 31][(tid >> 5) + 8 * u] = rb[u];
+    }
+    __syncthreads();
+    typename G::acc_t acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = typename G::acc_t{T(0), T(0), T(0), T(0)};
+#pragma unroll
+    for (int k4 = 0; k4 < IBK; k4 += 4) {
+        const int kr = k4 + (lane >> 4);
+        T x[2], y[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) x[i] = Bs[kr][32 * (wave >> 1) + 16 * i + (lane & 15)];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) y[j] = As[kr][32 * (wave & 1) + 16 * j + (lane & 15)];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = G::mma(x[i], y[j], acc[i][j]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int r = wr + 16 * j, c = wc + 16 * i + G::ccol(lane, q);
+                if (r < M && c < N) Cg[(int64_t)c * ld + r] = cv[i][j][q] - acc[i][j][q];
+            }
+}
+
+template <typename T>
+static void launch_gemm_inner(lsx_lu* lu, const T* A, const T* B, T* C, int64_t ld, int64_t M, int64_t N) {
+    const int pi = lu->prof.begin(lu->cur, PK_GEMM_SMALL, 2.0 * M * N * IBK, sizeof(T) * 2.0 * M * N);
+    hipLaunchKernelGGL(k_gemm_inner<T>, dim3((unsigned)(8 * cdiv(cdiv(M, IBM) * cdiv(N, IBM), 8))), dim3(256), 0, lu->cur,
+                       A, B, C, ld, (int)M, (int)N);
+    lu->prof.end(lu->cur, pi);
 }
 
 // Threads per tile: eight waves (64 x 32 each on a 128 x 128 tile, 32 x 16 on a 64 x 64 tile),

@@ -7,6 +7,7 @@
 #pragma once
 #include <algorithm>
 
+#include "gemm.hpp"
 #include "lu_kernels.hpp"
 
 namespace lsx {
@@ -60,7 +61,7 @@ static void launch_laswp_t(lsx_lu* lu, T* F, int64_t ld, int64_t k0, int kb, con
 }
 
 // Factors F (n x n, ld) in place; pivots into lu->ipiv, row map into lu->perm, diagonal-block
-// inverses into DL / DU.  gemm_upd does the inner and trailing updates (mode 0: C -= A B),
+// inverses into DL / DU.  gemm_upd does the trailing updates (mode 0: C -= A B),
 // gemm_trsm the products of the blocked TRSM (mode 1: C = A B in place, mode 0); both launch on
 // lu->cur.
 //
@@ -121,8 +122,8 @@ int getrf_blocked(lsx_lu* lu, T* F, int64_t ld, T* DL, T* DU, GU gemm_upd, GT ge
                                0, lu->cur, F, ld, n, ji, W, il, ic, jo, (int)nleft, ji + W, jo + jbo, lu->perm);
             lu->prof.end(lu->cur, pi);
             if (nright > 0)
-                gemm_upd(F + ji * ld + (ji + W), ld, F + (ji + W) * ld + ji, ld, F + (ji + W) * ld + (ji + W), ld,
-                         n - ji - W, nright, W, 0);
+                launch_gemm_inner<T>(lu, F + ji * ld + ji + W, F + (ji + W) * ld + ji, F + (ji + W) * ld + ji + W, ld,
+                                     n - ji - W, nright);
         }
         // the interchange lists first: the update stream applies them to the columns right of the
         // block while the diagonal-block inverses are formed

@@ -77,8 +77,8 @@ int lu64_alloc(lsx_lu* lu) {
     LSX_HIP(ctx, hipMalloc(&lu->dinfo, sizeof(int64_t) * 2));
     LSX_HIP(ctx, hipHostMalloc(&lu->hinfo, sizeof(int64_t) * 2, hipHostMallocDefault));
     LSX_HIP(ctx, hipMalloc(&lu->slots, sizeof(uint64_t) * 2 * (PMAX + 1) * RECS));
-    LSX_HIP(ctx, hipMalloc(&lu->plist, sizeof(int64_t) * 5 * 4 * NBO));
-    LSX_HIP(ctx, hipMalloc(&lu->pcount, sizeof(int) * 5));
+    LSX_HIP(ctx, hipMalloc(&lu->plist, sizeof(int64_t) * 9 * 4 * NBO));
+    LSX_HIP(ctx, hipMalloc(&lu->pcount, sizeof(int) * 9));
     // inverse row maps of the deferred L-column interchanges (used when a column segment of the
     // working type fits in LDS; FP32 is the smaller type)
     if ((n - NBO) * (int64_t)sizeof(float) <= LGMAX_BYTES && n > NBO)

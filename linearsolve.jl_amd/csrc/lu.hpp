@@ -5,7 +5,8 @@
 
 namespace lsx {
 constexpr int NBO = 128;      // outer block: K of the trailing MFMA update
-constexpr int64_t MTAIL = 3072, MWIDE = 8192;  // rows left: one last block up to, blocks of 2 NBO above
+// rows left: one last block up to MTAIL, blocks of 2 NBO above MWIDE, of 4 NBO above MWIDE4 (FP64)
+constexpr int64_t MTAIL = 3072, MWIDE = 8192, MWIDE4 = 10000;
 constexpr int PMAX = 128;     // max workgroups cooperating on one panel (512 rows each)
 constexpr int REC = 6 + 2 * PW;   // words of one FP64 exchange record: key lo/hi, row, pad, inverse, data
 constexpr int RECS = 72;          // record stride in the exchange buffer (words)
@@ -39,7 +40,7 @@ struct lsx_lu {
     int64_t* hinfo = nullptr;    // pinned host mirror of dinfo
     uint64_t* slots = nullptr;   // panel exchange records
     int64_t* plist = nullptr;    // permutation lists of 4*NBO words: a panel's, then by outer block
-                                 // parity two (one per NBO columns of the block)
+                                 // parity four (one per NBO columns of the block)
     int* pcount = nullptr;       // their lengths
     int* pinv = nullptr;         // per outer block: inverse of the row map after that block
                                  // (the deferred row interchanges of the L columns)

@@ -98,13 +98,16 @@ int getrf_blocked(lsx_lu* lu, T* F, int64_t ld, T* DL, T* DU, GU gemm_upd, GT ge
     //   m > MWIDE: 2 NBO columns, so that the trailing matrix is read and written half as often, where
     //     its update and not the panels' chain is the longer of the two: n = 16384 109.8 -> 100.6 ms, 12000
     //     58.2 -> 55.8, 9000 no change (limits of 7000 to 8192 measure the same, 11000 gives 102.2 and 57.6);
+    //     in FP64 4 NBO above MWIDE4 (16384 100.6 -> 98.1 ms, 12000 no change; FP32's shorter updates lose
+    //     to the longer inner ones: mixed 14000 58.1 -> 59.2);
     //   else NBO.
     auto width = [&](int64_t jo) -> int {
         const int64_t m = n - jo;
-        return (int)(m <= MTAIL ? m : m > MWIDE ? 2 * NBO : NBO);
+        if (m <= MTAIL) return (int)m;
+        return m <= MWIDE ? NBO : sizeof(T) == 8 && m > MWIDE4 ? 4 * NBO : 2 * NBO;
     };
-    auto plist = [&](int par, int h) { return lu->plist + (1 + 2 * par + h) * 4 * NBO; };
-    auto pcount = [&](int par, int h) { return lu->pcount + 1 + 2 * par + h; };
+    auto plist = [&](int par, int h) { return lu->plist + (1 + 4 * par + h) * 4 * NBO; };
+    auto pcount = [&](int par, int h) { return lu->pcount + 1 + 4 * par + h; };
     auto build_list = [&](int64_t k0, int kb, int par, int h) {
         hipLaunchKernelGGL(k_perm_build, dim3(1), dim3(256), 0, lu->cur, lu->ipiv, k0, kb, plist(par, h), pcount(par, h));
     };

@@ -1,5 +1,5 @@
 """The blocked LU where its outer blocks change width: one last block of up to 3072 rows, blocks of 128
-columns above, of 256 above 8192 rows; orders whose L interchanges are not deferred (above 18432); and FP32 panels of up
+columns above, of 256 above 8192 rows (512 above 10000, FP64); orders whose L interchanges are not deferred (above 18432); and FP32 panels of up
 to 2048 rows in one workgroup."""
 import numpy as np
 import pytest
@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 EPS = np.finfo(float).eps
 
 
-@pytest.mark.parametrize("n", [3071, 3072, 3073, 3201, 4099, 8193, 8450])
+@pytest.mark.parametrize("n", [3071, 3072, 3073, 3201, 4099, 8193, 8450, 10001])
 def test_factors_across_block_widths(lsx, n):
     print(f"blocks n={n}", flush=True)
     A = np.random.default_rng(n).standard_normal((n, n))

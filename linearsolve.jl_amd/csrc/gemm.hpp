@@ -265,8 +265,7 @@ static bool gemm_dispatch(hipStream_t st, int num_cus, const T* A, int64_t lda, 
         if (big) launch_gemm<T, 0, 128, 128, GEMM_NT>(st, A, lda, B, ldb, C, ldc, M, N, K);
         else launch_gemm<T, 0, 64, 64, GEMM_NT>(st, A, lda, B, ldb, C, ldc, M, N, K);
     } else {
-        if (M <= 64) launch_gemm<T, 1, 64, 64, GEMM_NT>(st, A, lda, B, ldb, C, ldc, M, N, K);
-        else launch_gemm<T, 1, 128, 128>(st, A, lda, B, ldb, C, ldc, M, N, K);
+        launch_gemm<T, 1, 64, 64, GEMM_NT>(st, A, lda, B, ldb, C, ldc, M, N, K);
     }
     return big;
 }

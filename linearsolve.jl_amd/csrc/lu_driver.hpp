@@ -49,14 +49,11 @@ static void launch_panel_t(lsx_lu* lu, T* F, int64_t ld, int64_t j0, int W, int6
 }
 
 template <typename T>
-static void launch_laswp_t(lsx_lu* lu, T* F, int64_t ld, int64_t k0, int kb, const int64_t* list,
-                           const int* count, int64_t c0, int64_t c1, int trsm) {
+static void launch_laswp_t(lsx_lu* lu, T* F, int64_t ld, int kb, const int64_t* list, const int* count, int64_t c0,
+                           int64_t c1) {
     if (c1 <= c0) return;
-    const int64_t nb = cdiv(c1 - c0, LCW);
-    const int pi = lu->prof.begin(lu->cur, PK_LASWP, trsm ? (double)kb * kb * (c1 - c0) : 0.0,
-                                  sizeof(T) * 4.0 * kb * (c1 - c0));
-    hipLaunchKernelGGL(k_laswp_trsm<T>, dim3((unsigned)nb), dim3(256), 0, lu->cur, F, ld, k0, kb, list, count,
-                       c0, c1, trsm);
+    const int pi = lu->prof.begin(lu->cur, PK_LASWP, 0.0, sizeof(T) * 4.0 * kb * (c1 - c0));
+    hipLaunchKernelGGL(k_laswp<T>, dim3((unsigned)cdiv(c1 - c0, LCW)), dim3(256), 0, lu->cur, F, ld, list, count, c0, c1);
     lu->prof.end(lu->cur, pi);
 }
 
@@ -148,8 +145,7 @@ int getrf_blocked(lsx_lu* lu, T* F, int64_t ld, T* DL, T* DU, GU gemm_upd, GT ge
     };
     auto interchange = [&](int64_t jo, int jbo, int par, int64_t c0, int64_t c1) {
         for (int k = 0; k < jbo; k += NBO)
-            launch_laswp_t<T>(lu, F, ld, jo + k, std::min(NBO, jbo - k), plist(par, k / NBO), pcount(par, k / NBO), c0,
-                              c1, 0);
+            launch_laswp_t<T>(lu, F, ld, std::min(NBO, jbo - k), plist(par, k / NBO), pcount(par, k / NBO), c0, c1);
     };
     // interchanges, U12 = L11^{-1} A12 and A22 -= L21 U12 of block [jo, jo + jbo) on columns
     // [c0, c1); wait_inv: the block's diagonal-block inverses may still be in the making on the
@@ -186,7 +182,7 @@ int getrf_blocked(lsx_lu* lu, T* F, int64_t ld, T* DL, T* DU, GU gemm_upd, GT ge
                 for (int64_t k = jo; k < n; k += NBO) {  // the last block made no lists
                     const int kb = (int)std::min<int64_t>(NBO, n - k);
                     build_list(k, kb, par, 0);
-                    launch_laswp_t<T>(lu, F, ld, k, kb, plist(par, 0), pcount(par, 0), 0, jo, 0);
+                    launch_laswp_t<T>(lu, F, ld, kb, plist(par, 0), pcount(par, 0), 0, jo);
                 }
         }
         if (c1 >= n) break;

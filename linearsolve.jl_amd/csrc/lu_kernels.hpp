@@ -383,30 +383,20 @@ static __global__ void k_iota(int* __restrict p, int64_t n) {
 }
 
 // ------------------------------------------------------------------------------------------
-// Applies a permutation list to columns [c0, c1) and, if trsm (kb <= PW), replaces the top kb
-// rows (k0 .. k0+kb) of those columns by L11^{-1} times them, L11 = unit lower of A[k0:, k0:]
-// staged in LDS (blocked_lufact.jl:126-178).  Each workgroup handles LCW columns.
+// Applies a permutation list of rows to columns [c0, c1).  Each workgroup handles LCW columns.
 constexpr int LCW = 32;
 template <typename T>
-__global__ __launch_bounds__(256) void k_laswp_trsm(T* __restrict A, int64_t ld, int64_t k0, int kb,
-                                                    const int64_t* __restrict list,
-                                                    const int* __restrict count, int64_t c0,
-                                                    int64_t c1, int trsm) {
+__global__ __launch_bounds__(256) void k_laswp(T* __restrict A, int64_t ld, const int64_t* __restrict list,
+                                               const int* __restrict count, int64_t c0, int64_t c1) {
     __shared__ int64_t s_dst[2 * NBO];
     __shared__ int64_t s_src[2 * NBO];
     __shared__ T s_buf[2 * NBO][LCW + 1];
-    __shared__ T s_L[PW][PW + 1];
     const int t = threadIdx.x;
     const int NT = *count;
     for (int i = t; i < NT; i += 256) {
         s_dst[i] = list[i];
         s_src[i] = list[2 * NBO + i];
     }
-    if (trsm)
-        for (int idx = t; idx < PW * PW; idx += 256) {
-            const int kk = idx / PW, i = idx - kk * PW;
-            s_L[i][kk] = (i < kb && kk < kb) ? A[(k0 + kk) * ld + k0 + i] : T(0);
-        }
     __syncthreads();
     const int64_t cb = c0 + (int64_t)blockIdx.x * LCW;
     const int ncol = (int)min((int64_t)LCW, c1 - cb);
@@ -427,30 +417,9 @@ __global__ __launch_bounds__(256) void k_laswp_trsm(T* __restrict A, int64_t ld,
         }
     }
     __syncthreads();
-    const int first = trsm ? kb : 0;
-    for (int idx = t; idx < (NT - first) * LCW; idx += 256) {
-        const int cc = idx / (NT - first), i = first + idx - cc * (NT - first);
+    for (int idx = t; idx < NT * LCW; idx += 256) {
+        const int cc = idx / NT, i = idx - cc * NT;
         if (cc < ncol) A[(cb + cc) * ld + s_dst[i]] = s_buf[i][cc];
-    }
-    if (!trsm) return;
-    // forward substitution with the unit-lower kb x kb block (kb <= PW): thread (col, group)
-    // updates rows group + 8j of its column, one barrier per pivot row
-    {
-        const int col = t & (LCW - 1), grp = t >> 5;
-        for (int kk = 0; kk < kb - 1; ++kk) {
-            const T xk = s_buf[kk][col];
-#pragma unroll
-            for (int j = 0; j < PW / 8; ++j) {
-                const int i = grp + 8 * j;
-                if (i > kk && i < kb) s_buf[i][col] = fma(-s_L[i][kk], xk, s_buf[i][col]);
-            }
-            __syncthreads();
-        }
-    }
-    __syncthreads();
-    for (int idx = t; idx < kb * LCW; idx += 256) {
-        const int c2 = idx / kb, i = idx - c2 * kb;
-        if (c2 < ncol) A[(cb + c2) * ld + k0 + i] = s_buf[i][c2];
     }
 }
 

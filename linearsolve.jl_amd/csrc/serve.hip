@@ -837,7 +837,7 @@ int lsx_serve_create(lsx_ctx* ctx, size_t hbm_budget, int32_t nstreams, lsx_serv
     const int lanes = std::max(2, std::min<int>(nstreams, 8));
     const int nd = lanes / 2, ng = lanes - nd;
     if (rc == LSX_OK) rc = lanes_alloc(s, nd, ng);
-    // the GMRES lanes together occupy at most 3/4 of the CUs (one 135 KB-LDS workgroup each), so
+    // the GMRES lanes together occupy at most 3/4 of the CUs (one workgroup per CU, by its LDS), so
     // the dense and batched lanes' kernels always find CUs
     s->gmres_pool = std::max(1, ctx->num_cus * 3 / 4 / ng);
     if (rc) {

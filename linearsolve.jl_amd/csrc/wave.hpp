@@ -23,9 +23,6 @@ __device__ __forceinline__ void static_for(F&& f) {
 template <int CTRL> __device__ __forceinline__ uint32_t dpp32(uint32_t x) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, false);
 }
-template <int CTRL> __device__ __forceinline__ uint64_t dpp64(uint64_t x) {
-    return ((uint64_t)dpp32<CTRL>((uint32_t)(x >> 32)) << 32) | dpp32<CTRL>((uint32_t)x);
-}
 // Value of the lane 16 (32) apart across rows of 16 (halves of 32), by v_permlane16_swap /
 // v_permlane32_swap of x with itself: the swap gives each lane its own value in one result and the
 // partner's in the other.
@@ -37,22 +34,6 @@ __device__ __forceinline__ uint32_t xrow32(uint32_t x) {
     const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
     return ((threadIdx.x >> 5) & 1) ? r[0] : r[1];
 }
-__device__ __forceinline__ uint64_t xrow16_64(uint64_t x) {
-    return ((uint64_t)xrow16((uint32_t)(x >> 32)) << 32) | xrow16((uint32_t)x);
-}
-__device__ __forceinline__ uint64_t xrow32_64(uint64_t x) {
-    return ((uint64_t)xrow32((uint32_t)(x >> 32)) << 32) | xrow32((uint32_t)x);
-}
-__device__ __forceinline__ uint64_t wave_max_u64(uint64_t x) {
-    uint64_t y;
-    y = dpp64<0xB1>(x);  x = y > x ? y : x;   // quad_perm [1,0,3,2]: lane ^ 1
-    y = dpp64<0x4E>(x);  x = y > x ? y : x;   // quad_perm [2,3,0,1]: lane ^ 2
-    y = dpp64<0x141>(x); x = y > x ? y : x;   // row_half_mirror: pairs the two quads of each 8
-    y = dpp64<0x140>(x); x = y > x ? y : x;   // row_mirror: pairs the two halves of each 16
-    y = xrow16_64(x);    x = y > x ? y : x;
-    y = xrow32_64(x);    x = y > x ? y : x;
-    return x;
-}
 __device__ __forceinline__ int wave_min_i32(int x) {
     int y;
     y = (int)dpp32<0xB1>((uint32_t)x);  x = y < x ? y : x;
@@ -62,15 +43,6 @@ __device__ __forceinline__ int wave_min_i32(int x) {
     y = (int)xrow16((uint32_t)x);       x = y < x ? y : x;
     y = (int)xrow32((uint32_t)x);       x = y < x ? y : x;
     return x;
-}
-// Lane holding the best (u, lr) pair of the wave: largest u, then smallest logical row lr.
-// u = 0 marks "no candidate"; the result is uniform across the wave.
-__device__ __forceinline__ int wave_argmax(uint64_t u, int lr) {
-    const uint64_t m = wave_max_u64(u);
-    const uint64_t tie = __ballot(u == m);
-    if (__popcll(tie) == 1 || m == 0) return __ffsll((unsigned long long)tie) - 1;
-    const int mn = wave_min_i32(u == m ? lr : INT_MAX);
-    return __ffsll((unsigned long long)__ballot(u == m && lr == mn)) - 1;
 }
 template <int CTRL> __device__ __forceinline__ uint32_t dpp_max_u32(uint32_t x) {
     const uint32_t y = dpp32<CTRL>(x);
@@ -88,8 +60,9 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
     x = y > x ? y : x;
     return (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
 }
-// Lane holding the best (u, lr) pair, as wave_argmax, in 32-bit steps: the upper halves decide almost
-// always, the lower halves and then the rows are compared only among lanes that tie.
+// Lane holding the best (u, lr) pair of the wave: largest u, then smallest logical row lr; u = 0 marks "no
+// candidate"; the result is uniform.  In 32-bit steps: the upper halves decide almost always, the lower
+// halves and then the rows are compared only among lanes that tie.
 __device__ __forceinline__ int wave_argmax32(uint64_t u, int lr) {
     const uint32_t hi = (uint32_t)(u >> 32);
     uint64_t tie = __ballot(hi == wave_max_u32(hi));

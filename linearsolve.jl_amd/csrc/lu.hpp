@@ -4,7 +4,7 @@
 #include "panel.hpp"
 
 namespace lsx {
-constexpr int NBO = 128;      // outer block: K of the trailing MFMA update
+constexpr int NBO = 128;      // unit of the outer blocks' widths (K of the trailing MFMA update)
 // rows left: one last block up to MTAIL, blocks of 2 NBO above MWIDE, of 4 NBO above MWIDE4 (FP64)
 constexpr int64_t MTAIL = 3072, MWIDE = 8192, MWIDE4 = 10000;
 constexpr int PMAX = 128;     // max workgroups cooperating on one panel (512 rows each)

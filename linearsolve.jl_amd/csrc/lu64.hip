@@ -2,7 +2,8 @@
 //
 // Algorithm: right-looking blocked LU with two block levels, the structure of LAPACK dgetrf
 // and of the reference's own restatement src/blocked_lufact.jl:658-679:
-//   outer block NBO = 128 columns (the K of the trailing MFMA update, which holds ~2/3 n^3 flops);
+//   outer blocks of 128 to 512 columns (the K of the trailing MFMA update, which holds ~2/3 n^3 flops)
+//   and one last block of up to 3072;
 //   inside it, inner panels of PW = 32 columns are factored by a register-resident kernel whose
 //   workgroups each hold up to 1024 rows x 32 columns (k_panel), exchanging, when there are several,
 //   one pivot candidate record per column through flag-in-word messages (no fences, one memory

@@ -3,7 +3,7 @@
 // for the plain path, FP32 or BF16 MFMA for the mixed path).
 //
 // Structure of LAPACK dgetrf and of src/blocked_lufact.jl:658-679, with two block levels:
-// outer blocks of NBO columns (K of the trailing update) split into inner panels of PW columns.
+// outer blocks of NBO to 4 NBO columns (K of the trailing update; the last one wider) split into inner panels of PW columns.
 #pragma once
 #include <algorithm>
 

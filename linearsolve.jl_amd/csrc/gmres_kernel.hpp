@@ -568,16 +568,18 @@ struct GmresWg {
         for (int b0 = 0; b0 < k; b0 += 64) {
             const int nb = min(64, k - b0);
             if (b0 > 0) {
-                constexpr int TR = NT / 64;  // threads per unknown
+                constexpr int TR = NT / 64;  // threads per unknown: 4, 8 or 16 (a row of lanes at most)
+                static_assert(TR == 4 || TR == 8 || TR == 16, "the sum over an unknown's threads");
                 const int j = b0 + tid / TR, sub = tid % TR;
                 double s = 0.0;
                 if (j < k) {
                     const double* Lj = L + (int64_t)j * (j - 1) / 2;
                     for (int i = sub; i < b0; i += TR) s = fma(Lj[i], hs[i], s);
                 }
-                if constexpr (TR > 1) s += dpp_f64<0xB1>(s);
-                if constexpr (TR > 2) s += dpp_f64<0x4E>(s);
-                if constexpr (TR > 4) s += dpp_f64<0x141>(s);
+                s += dpp_f64<0xB1>(s);
+                s += dpp_f64<0x4E>(s);
+                if constexpr (TR > 4) s += dpp_f64<0x141>(s);  // row_half_mirror
+                if constexpr (TR > 8) s += dpp_f64<0x140>(s);  // row_mirror
                 if (sub == 0 && j < k) hs[j] -= s;
                 __syncthreads();
             }

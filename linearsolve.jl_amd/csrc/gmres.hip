@@ -187,7 +187,7 @@ static int grow(lsx_ctx* ctx, void** p, size_t* have, size_t need, const char* w
     return LSX_OK;
 }
 
-int gmres_launch(lsx_csr* A, const GmresParams& p, const double* db, double* dx, const double* dpl,
+int gmres_launch(lsx_csr* A, const GmresParams& p, CoopHold& hold, const double* db, double* dx, const double* dpl,
                  const double* dpr, hipStream_t st) {
     lsx_ctx* ctx = A->ctx;
     const int64_t N = A->N;
@@ -227,6 +227,7 @@ int gmres_launch(lsx_csr* A, const GmresParams& p, const double* db, double* dx,
     g.red = A->red;
     g.out = A->out;
     g.timeout = wait_ticks(ctx, 20.0);
+    hold.take(ctx->device, ctx->num_cus, P);
     auto go = [&](auto lds, auto hbm) {
         if (plan.rglob) hipLaunchKernelGGL(hbm, dim3(P), dim3(plan.nt), plan.dynlds, st, g);
         else hipLaunchKernelGGL(lds, dim3(P), dim3(plan.nt), plan.dynlds, st, g);
@@ -430,7 +431,8 @@ int lsx_gmres_solve(lsx_csr* A, const double* b, double* x, int32_t memory, int3
     if (pl_diag) LSX_HIP(ctx, hipMemcpyAsync(A->dpl, pl_diag, vb, hipMemcpyDefault, A->stream));
     if (pr_diag) LSX_HIP(ctx, hipMemcpyAsync(A->dpr, pr_diag, vb, hipMemcpyDefault, A->stream));
     GmresParams p{memory, restart ? 1 : 0, maxiters, abstol, reltol};
-    int rc = gmres_launch(A, p, A->db, A->dx, pl_diag ? A->dpl : nullptr, pr_diag ? A->dpr : nullptr, A->stream);
+    CoopHold hold;
+    int rc = gmres_launch(A, p, hold, A->db, A->dx, pl_diag ? A->dpl : nullptr, pr_diag ? A->dpr : nullptr, A->stream);
     if (rc) return rc;
     LSX_HIP(ctx, hipMemcpyAsync(x, A->dx, vb, hipMemcpyDefault, A->stream));
     LSX_HIP(ctx, hipMemcpyAsync(A->hout, A->out, sizeof(GmresOut), hipMemcpyDeviceToHost, A->stream));

@@ -1,6 +1,7 @@
 // gmres.hpp — device-resident CSR matrix handle and the SimpleGMRES launcher.
 #pragma once
 #include "common.hpp"
+#include "coop.hpp"
 
 namespace lsx {
 constexpr int PMAX_G = 256;         // max workgroups of one GMRES solve (8192 rows each)
@@ -111,7 +112,8 @@ struct lsx_csr {
 };
 
 namespace lsx {
-int gmres_launch(lsx_csr* A, const GmresParams& p, const double* db, double* dx, const double* dpl,
+// hold: takes the solve's workgroups before the launch; the caller keeps it until the solve has ended.
+int gmres_launch(lsx_csr* A, const GmresParams& p, CoopHold& hold, const double* db, double* dx, const double* dpl,
                  const double* dpr, hipStream_t st);
 // Workgroups, rows per thread and LDS of a solve; LSX_EINVAL (message in ctx) when it does not fit.
 // hbm: the Krylov dimension may exceed what the LDS holds (single solves, gmres_launch); the

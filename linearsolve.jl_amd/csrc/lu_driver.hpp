@@ -7,6 +7,7 @@
 #pragma once
 #include <algorithm>
 
+#include "coop.hpp"
 #include "gemm.hpp"
 #include "lu_kernels.hpp"
 
@@ -71,6 +72,8 @@ int getrf_blocked(lsx_lu* lu, T* F, int64_t ld, T* DL, T* DU, GU gemm_upd, GT ge
     lsx_ctx* ctx = lu->ctx;
     const int64_t n = lu->n;
     const hipStream_t s0 = lu->stream_upd ? lu->stream_upd : lu->stream, s1 = lu->stream2;
+    CoopHold hold;  // (the serving lanes, without lookahead, hold theirs themselves)
+    if (lu->lookahead && cdiv(n, 1024) > COOP_MARGIN) hold.take(ctx->device, ctx->num_cus, (int)cdiv(n, 1024));
     const bool defer = lu->pinv != nullptr && (n - NBO) * (int64_t)sizeof(T) <= LGMAX_BYTES;
     if (s0 != lu->stream) {  // the input (copied on lu->stream) before anything on s0
         LSX_HIP(ctx, hipEventRecord(lu->ev_start, lu->stream));

@@ -21,7 +21,9 @@
 // other solves' ends fill it up); a lane reserves the largest solve's workgroup count and
 // the reservations of all lanes stay below the CU count minus 16.  Then the partly started
 // solves can never hold every CU, and the other kernels always finish, so every solve starts
-// completely in the end.
+// completely in the end.  Solves that the same process runs outside this server (or in another one) are
+// counted beside the lanes' reservations (coop.hpp); a lane takes its workgroups there last and holds
+// nothing that their holders wait for.
 // Lanes run on their own streams and threads, so their work overlaps on the device.  Every
 // kernel is deterministic and a request's arithmetic does not depend on what else is in flight:
 // a result is the same alone and in the mix.  Latency = completion - submission on the serving
@@ -124,7 +126,6 @@ namespace {
 
 enum Lane { LANE_BATCH = 0, LANE_DENSE = 1, LANE_GMRES = 2, NLANES = 3 };
 constexpr int MAXG = 64;           // solves per GMRES launch
-constexpr int COOP_MARGIN = 16;    // CUs never reserved by waiting workgroups
 constexpr size_t HALIGN = 256;     // heap and carve alignment
 
 inline size_t aup(size_t b) { return (b + HALIGN - 1) & ~(HALIGN - 1); }
@@ -459,7 +460,11 @@ void dense_worker(lsx_serve* s, int lane) {
             s->cv.wait(lk, [&] { return s->stop || (j = take_dense(s)) != nullptr; });
             if (!j) return;
         }
-        run_dense(s, L, j);
+        {
+            CoopHold hold;
+            hold.take(s->ctx->device, s->ctx->num_cus, j->coop);
+            run_dense(s, L, j);
+        }
         release_coop(s, j->coop);
         finish(s, j);
     }
@@ -632,7 +637,11 @@ void gmres_worker(lsx_serve* s, int lane) {
             s->cv.wait(lk, [&] { return s->stop || (reserve = take_gmres(s, group)) > 0; });
             if (group.empty()) return;
         }
-        run_gmres_group(s, L, group);
+        {
+            CoopHold hold;
+            hold.take(s->ctx->device, s->ctx->num_cus, reserve);
+            run_gmres_group(s, L, group);
+        }
         release_coop(s, reserve);
         for (Job* j : group) finish(s, j);
     }
@@ -828,7 +837,7 @@ int lsx_serve_create(lsx_ctx* ctx, size_t hbm_budget, int32_t nstreams, lsx_serv
     s->ctx = ctx;
     s->t0 = Clock::now();
     s->budget = hbm_budget;
-    s->coop_total = std::max(64, ctx->num_cus - COOP_MARGIN);
+    s->coop_total = coop_cus(ctx->num_cus);
     const size_t arena_bytes = std::min<size_t>(hbm_budget / 4, (size_t)2 << 30);
     const size_t heap_bytes = (hbm_budget - arena_bytes) & ~(HALIGN - 1);
     int rc = arena_alloc(ctx, s->arena, arena_bytes);

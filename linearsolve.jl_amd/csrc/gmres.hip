@@ -23,8 +23,8 @@ __global__ __launch_bounds__(NT, NT == 1024 ? 4 : (NT == 256 ? 3 : 2)) void k_gm
 // every solve but the one holding the highest number handed out so far has all its ranks
 // running and finishes by itself; with at least as many workgroups as the widest solve, that
 // last one fills up as the others end.
-template <int NT, int RPT>
-__global__ __launch_bounds__(NT, NT == 1024 ? 4 : (NT == 256 ? 3 : 2)) void k_gmres_multi(const GmresArgs* __restrict items,
+template <int NT, int RPT, bool MR = (RPT <= 4)>
+__global__ __launch_bounds__(NT, NT == 256 ? 3 : NT == 1024 || (RPT == 2 && !MR) ? 4 : 2) void k_gmres_multi(const GmresArgs* __restrict items,
                                                                        const int* __restrict first, int nitems,
                                                                        uint32_t* ticket) {
     __shared__ GShared<NT> sh;
@@ -45,7 +45,7 @@ __global__ __launch_bounds__(NT, NT == 1024 ? 4 : (NT == 256 ? 3 : 2)) void k_gm
         }
         const int item = __builtin_amdgcn_readfirstlane(lo);
         const GmresArgs a = items[item];
-        GmresWg<NT, RPT, false> g(a, sh, id - first[item], dyn);
+        GmresWg<NT, RPT, false, MR> g(a, sh, id - first[item], dyn);
         g.run();
     }
 }
@@ -119,8 +119,8 @@ int gmres_cap_limit(int64_t N, bool hbm) {
     return (int)cap;
 }
 
-int gmres_plan(lsx_ctx* ctx, int64_t N, const GmresParams& p, GmresPlan* out, bool hbm, bool one_wg) {
-    pick_shape(N, one_wg, out);
+int gmres_plan(lsx_ctx* ctx, int64_t N, const GmresParams& p, GmresPlan* out, bool hbm, int64_t blocks) {
+    pick_shape(N, blocks > 0, out);
     if (out->P > PMAX_G) return fail(ctx, LSX_EINVAL, "gmres: N = %lld exceeds %d rows", (long long)N, PMAX_G * 8192);
     const int64_t memory = std::max<int64_t>(1, std::min<int64_t>(p.memory, p.maxiters));
     const int64_t cap = p.restart ? memory : std::max<int64_t>(memory, p.maxiters);
@@ -129,10 +129,23 @@ int gmres_plan(lsx_ctx* ctx, int64_t N, const GmresParams& p, GmresPlan* out, bo
         return fail(ctx, LSX_EINVAL, "gmres: Krylov dimension %lld exceeds %d (restart = %d, N = %lld)", (long long)cap,
                     lim, p.restart, (long long)N);
     out->cap = (int)cap;
+    // Solves of one workgroup, more of them than CUs: LDS for as many as the registers let a CU run at
+    // once (they wait on their own barriers and not on each other), if the bookkeeping fits: three of 256
+    // threads for up to 512 rows; two for 513 to 1024 rows, without the rows' entries in registers.  Against
+    // one workgroup to a CU: 2000 blocks of 400 rows, memory 5 / 10 / 20: 8.4 / 5.7 / 5.6 -> 4.9 / 3.3 / 3.2 ms;
+    // of 529 rows 13.8 / 8.6 / 7.8 -> 11.2 / 6.9 / 6.2.  Beyond 1024 rows a second workgroup's registers spill.
+    auto lds_of = [](int64_t share) { return share == 1 ? GMRES_LDS_MAX : 160 * 1024 / (size_t)share - 8 * 1024; };
+    int64_t share = std::max<int64_t>(1, std::min<int64_t>(N <= 512 ? 3 : N <= 1024 ? 2 : 1, cdiv(blocks, ctx->num_cus)));
+    while (share > 1 && sizeof(double) * (size_t)gmres_book_words(cap) > lds_of(share)) --share;
+    out->shared = share > 1;
+    if (out->shared && N > 256 && N <= 512) {
+        out->nt = 256;
+        out->rpt = 2;
+    }
     // LDS: the bookkeeping and the receive buffer first, then the current vector's own rows, then as
     // many basis vectors as fit.  The receive buffer holds the products of a 32-vector group from
     // all workgroups when there is room.
-    const int64_t R = (int64_t)out->nt * out->rpt, words = (int64_t)(GMRES_LDS_MAX / sizeof(double));
+    const int64_t R = (int64_t)out->nt * out->rpt, words = (int64_t)(lds_of(share) / sizeof(double));
     int64_t left = words - gmres_book_words(cap);
     const int64_t rmin = out->P == 1 ? 0 : 512;
     out->rglob = left < rmin;
@@ -167,6 +180,8 @@ int gmres_launch_multi(lsx_ctx* ctx, hipStream_t st, const GmresArgs* items, con
         case 0: go(k_gmres_multi<256, 1>, 256); break;
         case 1: go(k_gmres_multi<512, 1>, 512); break;
         case 2: go(k_gmres_multi<512, 2>, 512); break;
+        case 3: go(k_gmres_multi<256, 2>, 256); break;
+        case 5: go(k_gmres_multi<512, 2, false>, 512); break;
         case 4: go(k_gmres_multi<512, 4>, 512); break;
         case 8: go(k_gmres_multi<512, 8>, 512); break;
         default: go(k_gmres_multi<1024, 8>, 1024); break;
@@ -470,7 +485,7 @@ int lsx_gmres_solve_batched(lsx_csr* A, int64_t blocksize, const double* b, doub
     GmresPlan plan;
     if (blocksize > 8192)
         return fail(ctx, LSX_EINVAL, "lsx_gmres_solve_batched: blocks of more than %d rows are not supported", 8192);
-    int rc = gmres_plan(ctx, blocksize, p, &plan, false, true);
+    int rc = gmres_plan(ctx, blocksize, p, &plan, false, nb);
     if (rc) return rc;
     const hipStream_t st = A->stream;
     // local columns (once per block size), after checking that A is block diagonal

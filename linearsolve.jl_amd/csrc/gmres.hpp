@@ -62,7 +62,10 @@ struct GmresPlan {
     bool rglob;     // the bookkeeping is in HBM (it does not fit the LDS)
     int ncache, own_lds, rbuf_len;  // LDS use (GmresArgs)
     size_t dynlds;  // dynamic LDS bytes per workgroup
-    int cls() const { return nt == 256 ? 0 : nt == 1024 ? 16 : rpt; }  // kernel of a multi-solve launch
+    bool shared;    // several workgroups run on a CU (blocks of a batched solve)
+    int cls() const {  // kernel of a multi-solve launch
+        return nt == 1024 ? 16 : nt == 256 ? (rpt == 1 ? 0 : 3) : shared && rpt == 2 ? 5 : rpt;
+    }
 };
 
 // Doubles of one workgroup's bookkeeping: the packed triangles R and L, the Givens pairs, z, the scales
@@ -118,8 +121,8 @@ int gmres_launch(lsx_csr* A, const GmresParams& p, CoopHold& hold, const double*
 // Workgroups, rows per thread and LDS of a solve; LSX_EINVAL (message in ctx) when it does not fit.
 // hbm: the Krylov dimension may exceed what the LDS holds (single solves, gmres_launch); the
 // multi-solve launches keep the bookkeeping in LDS.
-// one_wg: one workgroup whatever N (at most 8192 rows).
-int gmres_plan(lsx_ctx* ctx, int64_t N, const GmresParams& p, GmresPlan* out, bool hbm = false, bool one_wg = false);
+// blocks > 0: so many solves of one workgroup each, whatever N (at most 8192 rows).
+int gmres_plan(lsx_ctx* ctx, int64_t N, const GmresParams& p, GmresPlan* out, bool hbm = false, int64_t blocks = 0);
 // The fields of a launch that follow from the plan (not the arrays).
 void gmres_plan_args(const GmresPlan& plan, GmresArgs* a);
 // Solves of one kernel class (GmresPlan::cls) in one launch on `pool` workgroups (at least the widest

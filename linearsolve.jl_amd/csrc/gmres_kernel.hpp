@@ -145,14 +145,14 @@ __device__ __forceinline__ void sym_givens(double a, double b, double& c, double
 // The solve on workgroup w of a.P (sh, dyn: the workgroup's static and dynamic LDS).  RG: the
 // bookkeeping is in HBM (a.Rg) instead of LDS; a compile-time choice, so that each pointer below
 // is known to be LDS or global memory and gets that memory's instructions.
-template <int NT, int RPT, bool RG>
+template <int NT, int RPT, bool RG, bool MR = (RPT <= 4)>
 struct GmresWg {
     static constexpr int R = NT * RPT;             // rows of the workgroup
     static constexpr int VW = RPT >= 2 ? 2 : 1;    // neighbouring rows per load
     static constexpr int NP = RPT / VW;            // loads per thread and vector
     static constexpr int NW = NT / 64;
     static constexpr int MAXE = 8;                 // entries of a row held in registers
-    static constexpr bool MREG = RPT <= 4;         // whether they are (else read on each product)
+    static constexpr bool MREG = MR;               // whether they are (else read on each product)
     typedef double dvec __attribute__((ext_vector_type(VW)));
 
     const GmresArgs& a;
@@ -403,54 +403,78 @@ struct GmresWg {
     }
     // Products of vectors c0 .. c1 - 1 with q and u, summed over the wave into sh.part (slots
     // 2 (c - g0) + 0 / 1), CH vectors at a time.  The last group repeats its last vector (read again
-    // from the nearest cache) instead of having a body of its own: more bodies mean more copies of
-    // q and u, which spill.
-    static constexpr int CH = RPT >= 8 ? 4 : 8;
+    // from the nearest cache); with up to two rows per thread the last one to four vectors have a body of
+    // their own (memory 5: blocks of 64 to 529 rows 3 to 5 % faster), beyond that another body means
+    // another copy of q and u, which spill.
+    static constexpr int CH = RPT >= 8 ? 4 : 8, TAIL = 4;
     template <bool LDS>
     __device__ __forceinline__ void dots(int c0, int c1, int g0, const double (&q)[RPT], const double (&u)[RPT]) {
-        for (int c = c0; c < c1; c += CH) {
-            double r[2 * CH];
+        if constexpr (RPT > 2) {
+            dots_by<LDS, CH, false>(c0, c1, g0, q, u);
+        } else {
+            int c = c0;
+            for (; c1 - c > TAIL; c += CH) dots_by<LDS, CH, true>(c, c1, g0, q, u);
+            if (c < c1) dots_by<LDS, TAIL, true>(c, c1, g0, q, u);
+        }
+    }
+    // (ONE: the first group alone)
+    template <bool LDS, int M, bool ONE>
+    __device__ __forceinline__ void dots_by(int c0, int c1, int g0, const double (&q)[RPT], const double (&u)[RPT]) {
+        for (int c = c0; c < c1; c += M) {
+            double r[2 * M];
 #pragma unroll
-            for (int j = 0; j < 2 * CH; ++j) r[j] = 0.0;
+            for (int j = 0; j < 2 * M; ++j) r[j] = 0.0;
 #pragma unroll
             for (int p = 0; p < NP; ++p) {
-                dvec v[CH];
+                dvec v[M];
 #pragma unroll
-                for (int j = 0; j < CH; ++j) v[j] = vload<LDS>(min(c + j, c1 - 1), p);
+                for (int j = 0; j < M; ++j) v[j] = vload<LDS>(min(c + j, c1 - 1), p);
 #pragma unroll
-                for (int j = 0; j < CH; ++j)
+                for (int j = 0; j < M; ++j)
 #pragma unroll
                     for (int t = 0; t < VW; ++t) {
                         r[2 * j] = fma(v[j][t], q[VW * p + t], r[2 * j]);
                         r[2 * j + 1] = fma(v[j][t], u[VW * p + t], r[2 * j + 1]);
                     }
             }
-            constexpr int G = 64 / (2 * CH);  // lanes that hold the same sum
-            const double s = wave_sums<2 * CH>(r);
+            constexpr int G = 64 / (2 * M);  // lanes that hold the same sum
+            const double s = wave_sums<2 * M>(r);
             const int x = lane() / G;
             if ((lane() & (G - 1)) == 0 && c + (x >> 1) < c1) sh.part[wave()][2 * (c - g0) + x] = s;
+            if constexpr (ONE) break;
         }
     }
     // q += sum over vectors c0 .. c1 - 1 of f_c u_c, f_c = sign coef[c] sc[c]
     template <bool LDS>
     __device__ __forceinline__ void axpys(int c0, int c1, double sign, const double* coef, double (&q)[RPT]) const {
-        for (int c = c0; c < c1; c += CH) {
-            double f[CH];
+        if constexpr (RPT > 2) {
+            axpys_by<LDS, CH, false>(c0, c1, sign, coef, q);
+        } else {
+            int c = c0;
+            for (; c1 - c > TAIL; c += CH) axpys_by<LDS, CH, true>(c, c1, sign, coef, q);
+            if (c < c1) axpys_by<LDS, TAIL, true>(c, c1, sign, coef, q);
+        }
+    }
+    template <bool LDS, int M, bool ONE>
+    __device__ __forceinline__ void axpys_by(int c0, int c1, double sign, const double* coef, double (&q)[RPT]) const {
+        for (int c = c0; c < c1; c += M) {
+            double f[M];
 #pragma unroll
-            for (int j = 0; j < CH; ++j) {
+            for (int j = 0; j < M; ++j) {
                 const int cj = min(c + j, c1 - 1);
                 f[j] = c + j < c1 ? sign * (coef[cj] * sc[cj]) : 0.0;
             }
 #pragma unroll
             for (int p = 0; p < NP; ++p) {
-                dvec v[CH];
+                dvec v[M];
 #pragma unroll
-                for (int j = 0; j < CH; ++j) v[j] = vload<LDS>(min(c + j, c1 - 1), p);
+                for (int j = 0; j < M; ++j) v[j] = vload<LDS>(min(c + j, c1 - 1), p);
 #pragma unroll
-                for (int j = 0; j < CH; ++j)
+                for (int j = 0; j < M; ++j)
 #pragma unroll
                     for (int t = 0; t < VW; ++t) q[VW * p + t] = fma(f[j], v[j][t], q[VW * p + t]);
             }
+            if constexpr (ONE) break;
         }
     }
 
@@ -640,7 +664,8 @@ struct GmresWg {
             while (!(solved || tired || breakdown || dead)) {
                 if (!first) {
                     // r0 = Pl \ (b - A x): x complete in every workgroup before the product reads it
-                    (void)allreduce(0.0);
+                    if (a.P > 1) (void)allreduce(0.0);
+                    else __syncthreads();
                     if (dead) break;
                     spmv<true>(a.x, 1.0, q);
                     part = 0.0;
@@ -668,7 +693,7 @@ struct GmresWg {
                     spmv<false>(a.pr ? a.xp : a.V + (int64_t)(k - 1) * ldv, s, q);
                     products(k, q, u);
                     if (dead) break;
-                    subst(k);
+                    if (k > 1) subst(k);
                     refresh();
                     // q -= sum_i h_i v_i
                     {
@@ -722,16 +747,18 @@ struct GmresWg {
                     int inc = 0;
                     for (int i = k; i >= 1; --i) {
                         int64_t pos = nr + i - k;
+                        double y = z[i - 1];
                         for (int j = k; j >= i + 1; --j) {
-                            z[i - 1] = z[i - 1] - Rm[pos - 1] * z[j - 1];
+                            y = y - Rm[pos - 1] * z[j - 1];
                             pos = pos - j + 1;
                         }
                         if (fabs(Rm[pos - 1]) <= btol) {
-                            z[i - 1] = 0.0;
+                            y = 0.0;
                             inc = 1;
                         } else {
-                            z[i - 1] = z[i - 1] / Rm[pos - 1];
+                            y = y / Rm[pos - 1];
                         }
+                        z[i - 1] = y;
                     }
                     sh.inc = inc;
                 }

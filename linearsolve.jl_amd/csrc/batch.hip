@@ -88,6 +88,7 @@ struct BatchShared {
                                    // during the factorization, L11 of a panel without held L21
     };
     double red[2][BT / 64];
+    int info;                  // 1 + the first column whose pivot is zero
     int chg[SW];               // rows below the panel(s) that the interchanges move
     int nchg;
     double xs[BNMAX];          // solve vector
@@ -102,6 +103,13 @@ __device__ __forceinline__ int64_t uniform64(int64_t x) {
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x);
     const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)x >> 32));
     return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
+// Entry i of a system's matrix (at most 2 MB): a 32-bit byte offset from a uniform base, one register per
+// address (and no scalar pair per column, which spill).
+template <typename T> __device__ __forceinline__ T& el(T* A, int i) {
+    typedef typename std::conditional<std::is_const<T>::value, const char, char>::type C;
+    return *reinterpret_cast<T*>(reinterpret_cast<C*>(A) + (uint32_t)i * (uint32_t)sizeof(T));
 }
 
 // MFMA of the factor type: the transposed 16 x 16 tile D = X Y (X(i, k) = -U12(k, col i),
@@ -161,7 +169,7 @@ __device__ __forceinline__ void gather_left(BatchShared<T>& sh, T* A, int n) {
                     const int r = tid + k * BT;
 #pragma unroll
                     for (int c = 0; c < GC; ++c)
-                        g[k][c] = (r < m2 && cg + c < jb) ? A[(j0 + cg + c) * n + sh.perm[c1 + r]] : T(0);
+                        g[k][c] = (r < m2 && cg + c < jb) ? el(A, (j0 + cg + c) * n + sh.perm[c1 + r]) : T(0);
                 }
                 __syncthreads();
 #pragma unroll
@@ -169,7 +177,7 @@ __device__ __forceinline__ void gather_left(BatchShared<T>& sh, T* A, int n) {
                     const int r = tid + k * BT;
 #pragma unroll
                     for (int c = 0; c < GC; ++c)
-                        if (r < m2 && cg + c < jb) A[(j0 + cg + c) * n + c1 + r] = g[k][c];
+                        if (r < m2 && cg + c < jb) el(A, (j0 + cg + c) * n + c1 + r) = g[k][c];
                 }
             }
         }
@@ -203,7 +211,7 @@ __device__ __forceinline__ void tile_load(typename BMma<T>::acc_t (&c)[R][C], co
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const int lr = rb + 16 * a2 + (lane & 15), lc = cb + 16 * b2 + BMma<T>::ccol(lane, q);
-                    c[a2][b2][q] = (lr < mr && lc < nc) ? (T)S[lc * ld + sr[a2]] : T(0);
+                    c[a2][b2][q] = (lr < mr && lc < nc) ? (T)el(S, lc * ld + sr[a2]) : T(0);
                 }
         return;
     }
@@ -214,7 +222,7 @@ __device__ __forceinline__ void tile_load(typename BMma<T>::acc_t (&c)[R][C], co
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int lr = rb + 16 * a2 + (lane & 15), lc = cb + 16 * b2 + BMma<T>::ccol(lane, q);
-                c[a2][b2][q] = (lr < mr && lc < nc) ? A[lc * ld + lr] : T(0);
+                c[a2][b2][q] = (lr < mr && lc < nc) ? el(A, lc * ld + lr) : T(0);
             }
 }
 template <typename T, int R, int C>
@@ -226,7 +234,7 @@ __device__ __forceinline__ void tile_store(const typename BMma<T>::acc_t (&c)[R]
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int lr = rb + 16 * a2 + (lane & 15), lc = cb + 16 * b2 + BMma<T>::ccol(lane, q);
-                if (lr < mr && lc < nc) A[lc * ld + lr] = c[a2][b2][q];
+                if (lr < mr && lc < nc) el(A, lc * ld + lr) = c[a2][b2][q];
             }
 }
 // C (mr x nc at A22) -= L21 U12 for KB columns of L21 (at L21), U12 staged negated in LDS (column c's KB
@@ -258,7 +266,7 @@ __device__ __forceinline__ void tiles_update(T* A22, const double* S, const int*
         for (int a2 = 0; a2 < R2; ++a2) {
             const int lr = rb + 16 * a2 + (lane & 15);
 #pragma unroll
-            for (int k4 = 0; k4 < KS; ++k4) yl[a2][k4] = lr < mr ? L21[(k4 * 4 + (lane >> 4)) * ld + lr] : T(0);
+            for (int k4 = 0; k4 < KS; ++k4) yl[a2][k4] = lr < mr ? el(L21, (k4 * 4 + (lane >> 4)) * ld + lr) : T(0);
         }
         for (int cbi = cbs; cbi < cbe; ++cbi) {
             const int cb = cbi * (16 * C2);
@@ -307,13 +315,13 @@ __device__ __forceinline__ void swap_solve(BatchShared<T>& sh, T* A, const doubl
             const int c = b + u * CP + grp, co = c * n;
             if (S) {
 #pragma unroll
-                for (int t = 0; t < NR; ++t) x[u][t] = c < c1 ? (T)S[co + sh.perm[j0 + l16 + 16 * t]] : T(0);
+                for (int t = 0; t < NR; ++t) x[u][t] = c < c1 ? (T)el(S, co + sh.perm[j0 + l16 + 16 * t]) : T(0);
             } else {
 #pragma unroll
                 for (int t = 0; t < NR; ++t) {
-                    x[u][t] = c < c1 ? A[co + sh.perm[j0 + l16 + 16 * t]] : T(0);
+                    x[u][t] = c < c1 ? el(A, co + sh.perm[j0 + l16 + 16 * t]) : T(0);
                     const int i = l16 + 16 * t;
-                    w[u][t] = (c < c1 && i < nchg) ? A[co + sh.perm[sh.chg[i]]] : T(0);
+                    w[u][t] = (c < c1 && i < nchg) ? el(A, co + sh.perm[sh.chg[i]]) : T(0);
                 }
             }
         }
@@ -323,7 +331,7 @@ __device__ __forceinline__ void swap_solve(BatchShared<T>& sh, T* A, const doubl
 #pragma unroll
             for (int t = 0; t < NR; ++t) {
                 const int i = l16 + 16 * t;
-                if (c < c1 && i < nchg) A[co + sh.chg[i]] = w[u][t];
+                if (c < c1 && i < nchg) el(A, co + sh.chg[i]) = w[u][t];
             }
         }
         static_for<0, 16 * NR>([&](auto kc) {
@@ -348,7 +356,7 @@ __device__ __forceinline__ void swap_solve(BatchShared<T>& sh, T* A, const doubl
 #pragma unroll
             for (int t = 0; t < NR; ++t)
                 if (c < c1) {
-                    A[c * n + j0 + l16 + 16 * t] = x[u][t];
+                    el(A, c * n + j0 + l16 + 16 * t) = x[u][t];
                     if (neg) neg[(c - c0) * ns + l16 + 16 * t] = -x[u][t];
                 }
         }
@@ -364,10 +372,16 @@ __device__ __forceinline__ void swap_solve(BatchShared<T>& sh, T* A, const doubl
 // or 16 columns below n = 192), panels with two barriers and two rows through LDS per column, and a
 // copy of the matrices first; of the time 31 % is the panels', 28 % the trailing updates', 13 % the
 // solves', 12 % U12's.  3,000 systems, FP32 factors: 11.2 -> 8.9 ms.
+// Small systems leave most of a panel's waves without rows, and a branch per column between the loads of
+// a panel (with a spilled address each) made every load wait for the one before it.  With those waves
+// waiting at the barriers only, no barriers in panels of one wave, and branch-free loads by 32-bit offsets
+// (el): 20,000 FP64 systems of n = 1 0.65 -> 0.45 ms, of 8 to 16 1.25 -> 0.83; FP32 of 33 to 64 5.3 -> 3.3,
+// 3,000 FP32 systems of 8 to 512 8.9 -> 6.7, 20,000 50.6 -> 36.8; FP64 of 8 to 512 39.2 -> 38.8.
 template <typename T>
 __device__ __forceinline__ void factor_sys(BatchShared<T>& sh, T* A, const double* src, int n, int64_t vo, int64_t* ipiv,
                                            int64_t& info) {
     int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     PanelLds<T, BT / 64>& pl = *reinterpret_cast<PanelLds<T, BT / 64>*>(sh.wide);
     constexpr int POFF = (int)((sizeof(PanelLds<T, BT / 64>) + 15) / 16 * 16 / sizeof(T));  // LDS after the panel's
     constexpr int BST = PW + 2;                                                          // stride of panel B's U12 there
@@ -395,41 +409,54 @@ __device__ __forceinline__ void factor_sys(BatchShared<T>& sh, T* A, const doubl
                     live[t] = r < n;
                     lr[t] = r;
                     old[t] = r < n ? sh.perm[r] : 0;
-                    if (S && j == 0) {
+                    // (eight columns at a time without branches: rows past the end take the last one's
+                    // values, which nothing uses, columns past the end zeros)
+                    const int rc = min(r, n - 1);
+                    const bool none = j + 64 * wave + t * BT >= n;  // a wave without such rows
 #pragma unroll
-                        for (int q = 0; q < PW; ++q) v[t][q] = (r < n && q < w) ? (T)S[q * n + r] : T(0);
-                    } else {
+                    for (int q0 = 0; q0 < PW; q0 += 8) {
+                        if (none || q0 >= w) {
 #pragma unroll
-                        for (int q = 0; q < PW; ++q) v[t][q] = (r < n && q < w) ? A[(j + q) * n + r] : T(0);
+                            for (int q = q0; q < q0 + 8; ++q) v[t][q] = T(0);
+                        } else if (S && j == 0) {
+#pragma unroll
+                            for (int q = q0; q < q0 + 8; ++q) v[t][q] = (T)el(S, min(q, w - 1) * n + rc);
+                        } else {
+#pragma unroll
+                            for (int q = q0; q < q0 + 8; ++q) v[t][q] = el(A, (j + min(q, w - 1)) * n + rc);
+                        }
+                    }
+                    if (w < PW) {
+#pragma unroll
+                        for (int q = 0; q < PW; ++q) v[t][q] = q < w ? v[t][q] : T(0);
                     }
                 }
-                panel_columns<T, BT, RPT>(v, lr, live, w, j, n, pl, zero, [](const PanelRec<T>* r, int, bool) {
+                panel_columns<T, BT, RPT, true>(v, lr, live, w, j, n, pl, zero, [](const PanelRec<T>* r, int, bool) {
                     __syncthreads();
                     return r;
                 });
+                if (tid == 0) sh.info = zero;
                 __syncthreads();
+                zero = sh.info;
                 if (tid == 0) sh.nchg = 0;
                 if (tid < w) {
                     sh.piv[j + tid] = pl.piv[tid];
                     if (ipiv) ipiv[vo + j + tid] = (int64_t)pl.piv[tid] + 1;
                 }
-                const int rot = 8 * ((w + 7) / 8);
 #pragma unroll
                 for (int t = 0; t < RPT; ++t) {
                     if (j + tid + t * BT >= n) continue;
                     const int top = lr[t] - j;
                     sh.perm[lr[t]] = old[t];
-                    T* dst = A + j * n + lr[t];
-                    if (top < w) {
+                    const int dst = j * n + lr[t];
+                    if (top >= w) {  // a whole panel: after its four rotations slot q holds column q again
 #pragma unroll
-                        for (int q = 0; q < PW; ++q)
-                            if (q < w) dst[q * n] = pl.fin[top].v[q];
+                        for (int q = 0; q < PW; ++q) el(A, dst + q * n) = v[t][q];
+                    } else if (w == PW) {
+#pragma unroll
+                        for (int q = 0; q < PW; ++q) el(A, dst + q * n) = pl.fin[top].v[q];
                     } else {
-#pragma unroll
-                        for (int p = 0; p < PW; ++p) {
-                            const int q = (p + rot) & (PW - 1);
-                            if (q < w) dst[q * n] = v[t][p];
-                        }
+                        for (int q = 0; q < w; ++q) el(A, dst + q * n) = pl.fin[top].v[q];
                     }
                 }
             }
@@ -440,7 +467,7 @@ __device__ __forceinline__ void factor_sys(BatchShared<T>& sh, T* A, const doubl
                     const int r = j + tid + t * BT;
                     if (r < n && lr[t] != r) {
 #pragma unroll
-                        for (int q = 0; q < PW; ++q) g[t][q] = A[(j0 + q) * n + r];
+                        for (int q = 0; q < PW; ++q) g[t][q] = el(A, (j0 + q) * n + r);
                     }
                 }
                 __syncthreads();
@@ -449,11 +476,12 @@ __device__ __forceinline__ void factor_sys(BatchShared<T>& sh, T* A, const doubl
                     const int r = j + tid + t * BT;
                     if (r < n && lr[t] != r) {
 #pragma unroll
-                        for (int q = 0; q < PW; ++q) A[(j0 + q) * n + lr[t]] = g[t][q];
+                        for (int q = 0; q < PW; ++q) el(A, (j0 + q) * n + lr[t]) = g[t][q];
                     }
                 }
             }
             __syncthreads();
+            if (j + w >= n) continue;  // the last panel
             // the rows below the panel that are not in their places of the step's start
             for (int i = j + w + tid; i < n; i += BT)
                 if (sh.perm[i] != i) sh.chg[atomicAdd(&sh.nchg, 1)] = i;
@@ -471,7 +499,7 @@ __device__ __forceinline__ void factor_sys(BatchShared<T>& sh, T* A, const doubl
         T* L11 = sh.wide;  // L11[i (SW + 1) + k]
         for (int i = tid; i < SW * SW; i += BT) {
             const int r = i & (SW - 1), k = i / SW;
-            L11[r * (SW + 1) + k] = A[(j0 + k) * n + j0 + r];
+            L11[r * (SW + 1) + k] = el(A, (j0 + k) * n + j0 + r);
         }
         __syncthreads();
         swap_solve<T, 2>(sh, A, S, n, j0, c2, n, [&](int i, int k) { return L11[i * (SW + 1) + k]; }, (T*)nullptr, 0);
@@ -483,7 +511,7 @@ __device__ __forceinline__ void factor_sys(BatchShared<T>& sh, T* A, const doubl
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
                     const int i = b0 + u * BT;
-                    t8[u] = i < nc * SW ? A[(cc + i / SW) * n + j0 + (i & (SW - 1))] : T(0);
+                    t8[u] = i < nc * SW ? el(A, (cc + i / SW) * n + j0 + (i & (SW - 1))) : T(0);
                 }
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
@@ -497,7 +525,7 @@ __device__ __forceinline__ void factor_sys(BatchShared<T>& sh, T* A, const doubl
         __syncthreads();
     }
     info = zero;
-    gather_left<T, SW>(sh, A, n);
+    if (n > SW) gather_left<T, SW>(sh, A, n);  // (one step: nothing to its left, and sh.perm is its interchanges)
 }
 
 // s - sum_{k0 <= k < k1} a[k * n] x[k] in the order of k (FP64), sixteen loads in flight; ABS: ra += the
@@ -612,8 +640,6 @@ __global__ __launch_bounds__(BT, BatchCfg<T>::WG * BT / 256) void k_batch_lu(Bat
         int64_t info = 0;
         const double* src = a.src ? *a.src : nullptr;
         if (src) src += ao;
-        for (int i = tid; i < n; i += BT) sh.perm[i] = i;
-        __syncthreads();
         factor_sys<T>(sh, A, src, n, vo, a.ipiv, info);
         // solve: x = U^{-1} L^{-1} P b
         for (int i = tid; i < n; i += BT) sh.xs[i] = a.b[vo + sh.perm[i]];

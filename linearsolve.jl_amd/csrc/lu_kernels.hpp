@@ -141,7 +141,7 @@ __global__ __launch_bounds__(NT) void k_panel(PanelArgs<T> a) {
                                                lane < P ? s_all[lane & (PR - 1)].row : INT_MAX);
         return &s_all[wlane];
     };
-    panel_columns<T, NT, RPT>(v, lr, live, a.W, (int)a.j0, (int)a.m, sh, info, exchange);
+    panel_columns<T, NT, RPT, false>(v, lr, live, a.W, (int)a.j0, (int)a.m, sh, info, exchange);
     __syncthreads();
     if (w == 0) {
         if (tid < a.W) a.ipiv[a.j0 + tid] = (int64_t)sh.piv[tid] + 1;

@@ -106,16 +106,31 @@ struct PanelLds {
 // piv[c] (LDS): the logical row interchanged with row j0 + c; info: 1 + the first column (from 0, in the
 // matrix) whose pivot is zero, if it was 0.  On return row lr is row j0 + i (i < W): its columns are
 // fin[i] (LDS, after a barrier); of the other rows slot q holds column (q + 8 ceil(W / 8)) mod PW.
-template <typename T, int NT, int RPT, typename EX>
+// FEW (one workgroup): panels may have far fewer rows than NT RPT and fewer than PW columns, and other
+// workgroups of the CU use what the waves without rows leave: those only take part in the barriers, a
+// thread's second row and the groups of slots past the last column are skipped where there are none, and a
+// panel of one wave needs no barriers.  info is then valid in the waves with rows (the first among them).
+template <typename T, int NT, int RPT, bool FEW, typename EX>
 __device__ __forceinline__ void panel_columns(T (&v)[RPT][PW], int (&lr)[RPT], bool (&live)[RPT], int W, int j0, int m,
                                               PanelLds<T, NT / 64>& sh, int& info, EX&& exchange) {
     constexpr int NW = NT / 64;
     static_assert(NW == 2 || NW == 4 || NW == 8 || NW == 16, "the search among the waves takes up to sixteen candidates");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool one = FEW && m - j0 <= 64;                           // one wave has all the rows
+    const bool two = RPT > 1 && (!FEW || j0 + NT + 64 * wave < m);  // this wave has second rows
+    if (FEW && j0 + 64 * wave >= m) {
+        if (one) return;
+        if (lane == 0) {
+            sh.cand[wave].key = 0;
+            sh.cand[wave].row = INT_MAX;
+        }
+        for (int c = 0; c < 2 * W; ++c) __syncthreads();  // two per column
+        return;
+    }
 #pragma unroll 1
     for (int g = 0; g < PW / 8; ++g) {
         if (8 * g >= W) break;
-        const int nb = 4 - g;  // groups of eight slots that hold columns not yet finished
+        const int nb = (FEW ? (W + 7) / 8 : 4) - g;  // groups of eight slots that hold columns not yet finished
         // columns of slots lane & 15 and 16 + (lane & 15)
         const int ca = ((lane & 15) + 8 * g) & (PW - 1), cb = ca ^ 16;
         static_for<0, 8>([&](auto cc) {
@@ -128,22 +143,25 @@ __device__ __forceinline__ void panel_columns(T (&v)[RPT][PW], int (&lr)[RPT], b
             int krow = lr[0];
             T best = v[0][c];
             bool second = false;
-            if constexpr (RPT > 1) {
-                const uint64_t k1 = live[1] ? pivot_key(v[1][c]) : 0;
-                second = k1 > key || (k1 == key && lr[1] < krow);
+            if (RPT > 1 && two) {
+                const uint64_t k1 = live[RPT - 1] ? pivot_key(v[RPT - 1][c]) : 0;
+                second = k1 > key || (k1 == key && lr[RPT - 1] < krow);
                 key = second ? k1 : key;
-                krow = second ? lr[1] : krow;
-                best = second ? v[1][c] : best;
+                krow = second ? lr[RPT - 1] : krow;
+                best = second ? v[RPT - 1][c] : best;
             }
             const T binv = T(1) / best;  // formed in the shadow of the search
             const int wl = wave_argmax32(key, krow);
-            if (lane == wl) {
-                sh.cand[wave].key = key;
-                sh.cand[wave].row = krow;
+            int wi = 0;
+            if (!one) {
+                if (lane == wl) {
+                    sh.cand[wave].key = key;
+                    sh.cand[wave].row = krow;
+                }
+                __syncthreads();
+                const PanelCand cd = sh.cand[lane & (NW - 1)];
+                wi = wave_argmax_rep<NW>(cd.key, cd.row);
             }
-            __syncthreads();
-            const PanelCand cd = sh.cand[lane & (NW - 1)];
-            const int wi = wave_argmax_rep<NW>(cd.key, cd.row);
             PanelRec<T>& rec = sh.fin[col];
             if (wave == wi && lane == wl) {
                 rec.key = key;
@@ -166,7 +184,9 @@ __device__ __forceinline__ void panel_columns(T (&v)[RPT][PW], int (&lr)[RPT], b
                     asm volatile("; first row" ::: "memory");
                 }
             }
-            const PanelRec<T>* win = exchange(&rec, col, wave == wi);
+            const PanelRec<T>* win = &rec;
+            if (one) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            else win = exchange(&rec, col, wave == wi);
             int grow = win->row;
             const T pv = win->v[col], inv = win->inv;
             const T pa = win->v[ca], pb = win->v[cb];
@@ -181,6 +201,7 @@ __device__ __forceinline__ void panel_columns(T (&v)[RPT][PW], int (&lr)[RPT], b
             T nl[RPT];
 #pragma unroll
             for (int t = 0; t < RPT; ++t) {
+                if (t > 0 && !two) continue;
                 live[t] = live[t] && lr[t] != grow;
                 lr[t] = lr[t] == grow ? k : (lr[t] == k ? grow : lr[t]);
                 T l = v[t][c] * inv;
@@ -189,12 +210,14 @@ __device__ __forceinline__ void panel_columns(T (&v)[RPT][PW], int (&lr)[RPT], b
                 nl[t] = live[t] ? -l : T(0);  // a finished row's registers do not matter any more
             }
 #pragma unroll
-            for (int t = 0; t < RPT; ++t) fmac_row<0, c + 1>(v[t], pa, nl[t]);
+            for (int t = 0; t < RPT; ++t)
+                if (t == 0 || two) fmac_row<0, c + 1>(v[t], pa, nl[t]);
 #pragma unroll
             for (int b = 1; b < 4; ++b)
                 if (b < nb) {
 #pragma unroll
                     for (int t = 0; t < RPT; ++t) {
+                        if (t > 0 && !two) continue;
                         if (b == 1) fmac_row<8, 0>(v[t], pa, nl[t]);
                         else if (b == 2) fmac_row<16, 0>(v[t], pb, nl[t]);
                         else fmac_row<24, 0>(v[t], pb, nl[t]);
@@ -204,6 +227,7 @@ __device__ __forceinline__ void panel_columns(T (&v)[RPT][PW], int (&lr)[RPT], b
         // the next group's columns to slots 0 .. 7
 #pragma unroll
         for (int t = 0; t < RPT; ++t) {
+            if (t > 0 && !two) continue;
             T done[8];
 #pragma unroll
             for (int q = 0; q < 8; ++q) done[q] = v[t][q];

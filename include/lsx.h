@@ -180,9 +180,9 @@ int lsx_batch_destroy(lsx_batch* batch);
  * receives the pivots packed like b.  Returns the number of systems with info > 0. */
 int lsx_batch_factor_solve(lsx_batch* batch, const double* A, const double* b, double* x,
                            int64_t* info, int64_t* ipiv);
-/* Size-binned tile table: a hint that a system of size n might take panels of bw[k] (8, 16 or 32)
- * columns, for the first bin with n <= upper[k].  The table is checked; every system takes 32-column
- * panels, the fastest at every size.  No reference counterpart. */
+/* Size-binned tile table: kept for callers of earlier versions, in which a system of size n took panels of
+ * bw[k] (8, 16 or 32) columns for the first bin with n <= upper[k].  The table is checked and otherwise
+ * has no effect: every system takes 32-column panels.  No reference counterpart. */
 int lsx_batch_set_tiles(lsx_batch* batch, int32_t nbins, const int32_t* upper, const int32_t* bw);
 /* LSX_F32 batches: refinement target (normwise backward error, default 1e-14) and step limit
  * (default 10).  No reference counterpart. */

@@ -521,9 +521,10 @@ TILE_TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tile_tabl
 
 
 def load_tile_table(path=TILE_TABLE, dtype=LSX_F64):
-    """Size-binned panel widths written by autotune.py for the factor type dtype:
+    """A size-binned panel-width table of a JSON file for the factor type dtype:
     {"bins": [[upper, bw], ...] (FP64 factors), "bins_fp32": [...] (FP32 factors)} (None if absent;
-    FP32 batches fall back to the FP64 table when the file has none of their own)."""
+    FP32 batches fall back to the FP64 table when the file has none of their own).  Reads tables made for
+    earlier versions of the library; the widths no longer choose anything (_BatchHandle.set_tiles)."""
     if not os.path.exists(path):
         return None
     with open(path) as f:
@@ -540,9 +541,8 @@ class _BatchHandle:
         ctx.check(_abi.lib().lsx_batch_create(ctx.handle, len(self.sizes), self.sizes.ctypes.data, dtype,
                                               ctypes.byref(h)), "lsx_batch_create")
         self.h = h
-        table = load_tile_table(dtype=dtype) if tiles == "auto" else tiles
-        if table:
-            self.set_tiles(table)
+        if tiles and tiles != "auto":
+            self.set_tiles(tiles)
 
     def __del__(self):
         h = getattr(self, "h", None)
@@ -551,6 +551,7 @@ class _BatchHandle:
             self.h = None
 
     def set_tiles(self, table):
+        """Checks a table of [(upper, panel width), ...]; no effect: every system takes 32-column panels."""
         up = np.ascontiguousarray([u for u, _ in table], dtype=np.int32)
         bw = np.ascontiguousarray([w for _, w in table], dtype=np.int32)
         self.ctx.check(_abi.lib().lsx_batch_set_tiles(self.h, len(up), up.ctypes.data, bw.ctypes.data),

@@ -894,6 +894,7 @@ int lsx_batch_destroy(lsx_batch* B) {
     return LSX_OK;
 }
 
+// (for callers of earlier versions: checks the table, which chooses nothing any more)
 int lsx_batch_set_tiles(lsx_batch* B, int32_t nbins, const int32_t* upper, const int32_t* bw) {
     if (!B || nbins < 0 || (nbins > 0 && (!upper || !bw))) return LSX_EINVAL;
     lsx_ctx* ctx = B->ctx;

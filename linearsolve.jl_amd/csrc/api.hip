@@ -36,14 +36,14 @@ int lu64_alloc(lsx_lu* lu) {
     const int nblk = (int)cdiv(n, DB);
     LSX_HIP(ctx, hipStreamCreateWithFlags(&lu->stream, hipStreamNonBlocking));
     // getrf lookahead streams.  The panel workgroups wait on each other, so they get CUs of their
-    // own: 4 per XCD (32 in all, enough for the 512-row workgroups of n <= 16384) and the
-    // trailing updates the rest.  The CU set {per*x + (x + 8j) mod per} puts 4 CUs on every XCD
+    // own: 4 per XCD (32 in all, for at most 16 workgroups of 1024 rows at n <= 16384 and the updates
+    // inside a block) and the trailing updates the rest.  The CU set {per*x + (x + 8j) mod per} puts 4 CUs on every XCD
     // whether CU mask bits are numbered XCD by XCD or round-robin over the XCDs.
     // (only for n >= 2048: below that the lookahead gains nothing, and a CU-masked stream takes a
     // hardware queue of its own, of which a process has few)
     const int per = ctx->num_cus / 8;
     bool masked = false;
-    if (lu->lookahead && n >= 2048 && ctx->num_cus % 8 == 0 && per % 8 == 0 && per >= 32 && cdiv(n, 512) <= 32) {
+    if (lu->lookahead && n >= 2048 && ctx->num_cus % 8 == 0 && per % 8 == 0 && per >= 32 && n <= 16 * PROWS) {
         const int words = (ctx->num_cus + 31) / 32;
         std::vector<uint32_t> ms(words, 0u), mc(words, 0u);
         for (int x = 0; x < 8; ++x)
@@ -211,8 +211,8 @@ int lsx_synchronize(lsx_ctx* ctx) {
 int lsx_lu_create(lsx_ctx* ctx, int64_t n, int dtype, lsx_lu** out) {
     if (!ctx || !out) return LSX_EINVAL;
     *out = nullptr;
-    if (n < 1 || n > (int64_t)PMAX * 512)
-        return fail(ctx, LSX_EINVAL, "lsx_lu_create: n = %lld outside [1, %d]", (long long)n, PMAX * 512);
+    if (n < 1 || n > (int64_t)PMAX * PROWS)
+        return fail(ctx, LSX_EINVAL, "lsx_lu_create: n = %lld outside [1, %d]", (long long)n, PMAX * PROWS);
     if (dtype != LSX_F64 && dtype != LSX_F32 && dtype != LSX_BF16)
         return fail(ctx, LSX_EINVAL, "lsx_lu_create: unknown dtype %d", dtype);
     DeviceGuard g(ctx);

@@ -7,9 +7,9 @@ namespace lsx {
 constexpr int NBO = 128;      // unit of the outer blocks' widths (K of the trailing MFMA update)
 // rows left: one last block up to MTAIL, blocks of 2 NBO above MWIDE, of 4 NBO above MWIDE4 (FP64)
 constexpr int64_t MTAIL = 3072, MWIDE = 8192, MWIDE4 = 10000;
-constexpr int PMAX = 128;     // max workgroups cooperating on one panel (512 rows each)
-constexpr int REC = 6 + 2 * PW;   // words of one FP64 exchange record: key lo/hi, row, pad, inverse, data
-constexpr int RECS = 72;          // record stride in the exchange buffer (words)
+constexpr int PROWS = 1024;   // rows of a workgroup when several share a panel
+constexpr int PMAX = 64;      // most workgroups of one panel (one lane of a wave for each one's record)
+constexpr int RECS = 72;      // record stride in the exchange buffer (words; FP64: 6 + 2 PW of them used)
 constexpr int DB = 64;            // diagonal block of the explicit inverses and triangular solves
 constexpr int TRHS = 16;          // right-hand sides per triangular-solve launch
 constexpr int64_t LGMAX_BYTES = 144 * 1024;  // LDS of the deferred L-interchange pass

@@ -35,7 +35,7 @@ static void launch_panel_t(lsx_lu* lu, T* F, int64_t ld, int64_t j0, int W, int6
     // one row per thread while 512 threads cover the panel, then two: the fewest entries to update per
     // column (256 rows 32 us, 512 rows 38 us per panel), and no exchange between workgroups up to 1024
     // rows (47 us; two workgroups of 512 rows took 105)
-    a.P = (int)cdiv(m_rows, 1024);
+    a.P = (int)cdiv(m_rows, PROWS);
     if (m_rows <= 256) hipLaunchKernelGGL((k_panel<T, 256, 1>), dim3(1), dim3(256), 0, lu->cur, a);
     else if (m_rows <= 512) hipLaunchKernelGGL((k_panel<T, 512, 1>), dim3(1), dim3(512), 0, lu->cur, a);
     else if (sizeof(T) == 8 || m_rows <= 1024 || m_rows > 2048)
@@ -73,7 +73,7 @@ int getrf_blocked(lsx_lu* lu, T* F, int64_t ld, T* DL, T* DU, GU gemm_upd, GT ge
     const int64_t n = lu->n;
     const hipStream_t s0 = lu->stream_upd ? lu->stream_upd : lu->stream, s1 = lu->stream2;
     CoopHold hold;  // (the serving lanes, without lookahead, hold theirs themselves)
-    if (lu->lookahead && cdiv(n, 1024) > COOP_MARGIN) hold.take(ctx->device, ctx->num_cus, (int)cdiv(n, 1024));
+    if (lu->lookahead && cdiv(n, PROWS) > COOP_MARGIN) hold.take(ctx->device, ctx->num_cus, (int)cdiv(n, PROWS));
     const bool defer = lu->pinv != nullptr && (n - NBO) * (int64_t)sizeof(T) <= LGMAX_BYTES;
     if (s0 != lu->stream) {  // the input (copied on lu->stream) before anything on s0
         LSX_HIP(ctx, hipEventRecord(lu->ev_start, lu->stream));

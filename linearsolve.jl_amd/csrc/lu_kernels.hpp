@@ -45,8 +45,7 @@ __global__ __launch_bounds__(NT) void k_panel(PanelArgs<T> a) {
     constexpr int NW = NT / 64;
     constexpr int WPE = Words<T>::W;
     constexpr int HW = panel_head<T>();
-    constexpr int PR = PMAX / 2;                 // workgroups of 1024 rows
-    constexpr bool MULTI = NT * RPT == 1024;     // the shape that several workgroups share a panel in
+    constexpr bool MULTI = NT * RPT == PROWS;    // the shape that several workgroups share a panel in
     const int tid = threadIdx.x, w = blockIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r0 = (int)a.j0 + w * NT * RPT + tid;
     T* col0 = a.A + a.j0 * a.ld;
@@ -65,7 +64,7 @@ __global__ __launch_bounds__(NT) void k_panel(PanelArgs<T> a) {
     // would be waited for by the next global access (or the next wait the compiler places)
     int info = 0;
     __shared__ PanelLds<T, NW> sh;
-    __shared__ PanelRec<T> s_all[MULTI ? PR : 1];
+    __shared__ PanelRec<T> s_all[MULTI ? PMAX : 1];
     if (w == 0 && tid == 0) {
         __hip_atomic_store(a.count, a.W, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // in memory before any workgroup counts its moved rows (which all have seen a message, or
@@ -137,8 +136,8 @@ __global__ __launch_bounds__(NT) void k_panel(PanelArgs<T> a) {
             }
         }
         __syncthreads();
-        const int wlane = wave_argmax32(lane < P ? s_all[lane & (PR - 1)].key : 0,
-                                               lane < P ? s_all[lane & (PR - 1)].row : INT_MAX);
+        const int wlane = wave_argmax32(lane < P ? s_all[lane & (PMAX - 1)].key : 0,
+                                               lane < P ? s_all[lane & (PMAX - 1)].row : INT_MAX);
         return &s_all[wlane];
     };
     panel_columns<T, NT, RPT, false>(v, lr, live, a.W, (int)a.j0, (int)a.m, sh, info, exchange);

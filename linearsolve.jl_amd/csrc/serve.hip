@@ -323,11 +323,11 @@ int classify(lsx_serve* s, Job* j) {
             j->footprint = (size_t)(8 * n * n + 64 * n);
             return LSX_OK;
         }
-        if (n > (int64_t)PMAX * 512)
-            return fail(s->ctx, LSX_EINVAL, "lsx_serve_submit: dense n = %lld exceeds %d", (long long)n, PMAX * 512);
+        if (n > (int64_t)PMAX * PROWS)
+            return fail(s->ctx, LSX_EINVAL, "lsx_serve_submit: dense n = %lld exceeds %d", (long long)n, PMAX * PROWS);
         j->lane = LANE_DENSE;
         j->footprint = dense_block(0, n).bytes;
-        j->coop = (int)cdiv(n, 512) + 1;  // panel workgroups, plus the chained solve's running one
+        j->coop = (int)cdiv(n, PROWS) + 1;  // panel workgroups, plus the chained solve's running one
         return LSX_OK;
     }
     j->lane = LANE_GMRES;

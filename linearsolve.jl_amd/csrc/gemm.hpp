@@ -171,8 +171,8 @@ static void launch_gemm(hipStream_t st, const T* A, int64_t lda, const T* B, int
 // C -= A B with K = 32 (A: M x 32, B: 32 x N, C: M x N, one leading dimension): a panel's update inside
 // its outer block, on the chain of the panels, where the time is latency and not rate.  A 64 x 64 tile per
 // workgroup, four waves of 32 x 32, and every load of a tile (A, B and C) issued before the first is
-// waited for; the staged kernel above has three dependent round trips at K = 32.  FP32 products and sums
-// also in the mixed path.  n = 3001 9.07 -> 8.91 ms, 1024 1.80 -> 1.78; mixed, against the split-BF16
+// waited for; the staged kernel above has three dependent round trips at K = 32.  FP32 factors take FP32
+// products and sums here too (BF16 factors: k_gemm_inner_split).  n = 3001 9.07 -> 8.91 ms, 1024 1.80 -> 1.78; mixed, against the split-BF16
 // kernel (128 x 128 tiles, 12 to 15 us), n = 3000 7.87 -> 7.55, 9000 33.7 -> 32.9.
 constexpr int IBK = 32, IBM = 64;
 template <typename T>

@@ -189,6 +189,114 @@ __global__ __launch_bounds__(512, 1) void k_gemm_split(const float* __restrict A
     }
 }
 
+// C -= A B with K = 32, one leading dimension and S BF16 pieces per operand: the BF16 factors' update of a
+// panel inside its outer block, as k_gemm_inner (gemm.hpp) is the FP32 factors'.  64 x 64 tiles, four
+// waves of 32 x 32, every load of a tile issued before the first is waited for; one MFMA per term covers all
+// of K.
+template <int S>
+__global__ __launch_bounds__(256) void k_gemm_inner_split(const float* __restrict Ag, const float* Bg, float* Cg,
+                                                          int64_t ld, int M, int N) {
+    constexpr int TB_ = 64;
+    const int TM = (M + TB_ - 1) / TB_, TN = (N + TB_ - 1) / TB_, NTL = TM * TN;
+    const int per = (NTL + 7) / 8, tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || tile >= NTL) return;
+    const int row0 = tile % TM * TB_, col0 = tile / TM * TB_;
+    __shared__ __align__(16) __bf16 As[S][TB_][SBK + SPAD];
+    __shared__ __align__(16) __bf16 Bs[S][TB_][SBK + SPAD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave & 1, wn = wave >> 1;
+    const int ar = tid & 63, akg = tid >> 6, bkb = tid & 3, bc = tid >> 2;  // as in k_gemm_split
+    const bool bvec = ((ld & 3) == 0) && ((reinterpret_cast<uintptr_t>(Bg) & 15) == 0);
+    const bool vec = ((ld & 3) == 0) && ((reinterpret_cast<uintptr_t>(Cg) & 15) == 0);
+    float ra[8], rb[8];
+    sv4f cv[2][2];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ra[e] = row0 + ar < M ? Ag[(int64_t)(akg * 8 + e) * ld + row0 + ar] : 0.f;
+    {
+        const float* bp = Bg + (int64_t)(col0 + bc) * ld + bkb * 8;
+        if (bvec && col0 + bc < N) {
+            const sv4f u0 = *reinterpret_cast<const sv4f*>(bp), u1 = *reinterpret_cast<const sv4f*>(bp + 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                rb[e] = u0[e];
+                rb[e + 4] = u1[e];
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) rb[e] = col0 + bc < N ? bp[e] : 0.f;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int col = col0 + wn * 32 + j * 16 + (lane & 15), row = row0 + wm * 32 + i * 16 + 4 * (lane >> 4);
+            const float* cp = Cg + (int64_t)col * ld + row;
+            if (col < N && vec && row + 3 < M) {
+                cv[i][j] = *reinterpret_cast<const sv4f*>(cp);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) cv[i][j][q] = (col < N && row + q < M) ? cp[q] : 0.f;
+            }
+        }
+    {
+        sv8bf pa[S], pb[S];
+        split8<S>(ra, pa);
+        split8<S>(rb, pb);
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            *reinterpret_cast<sv8bf*>(&As[s][ar][akg * 8]) = pa[s];
+            *reinterpret_cast<sv8bf*>(&Bs[s][bc][bkb * 8]) = pb[s];
+        }
+    }
+    __syncthreads();
+    const int kq = 8 * (lane >> 4);
+    sv8bf x[2][S], y[2][S];
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            x[i][s] = *reinterpret_cast<const sv8bf*>(&As[s][wm * 32 + i * 16 + (lane & 15)][kq]);
+            y[i][s] = *reinterpret_cast<const sv8bf*>(&Bs[s][wn * 32 + i * 16 + (lane & 15)][kq]);
+        }
+    sv4f acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = sv4f{0.f, 0.f, 0.f, 0.f};
+    // the small terms first (k_gemm_split)
+    constexpr int NTERM = S == 1 ? 1 : (S == 2 ? 3 : 6);
+    constexpr int TA[6] = {2, 1, 0, 1, 0, 0}, TB[6] = {0, 1, 2, 0, 1, 0};
+#pragma unroll
+    for (int t = 6 - NTERM; t < 6; ++t)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[i][TA[t]], y[j][TB[t]], acc[i][j], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int col = col0 + wn * 32 + j * 16 + (lane & 15), row = row0 + wm * 32 + i * 16 + 4 * (lane >> 4);
+            float* cp = Cg + (int64_t)col * ld + row;
+            sv4f nv;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) nv[q] = cv[i][j][q] - acc[i][j][q];
+            if (col < N && vec && row + 3 < M) {
+                *reinterpret_cast<sv4f*>(cp) = nv;
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (col < N && row + q < M) cp[q] = nv[q];
+            }
+        }
+}
+template <int S>
+static void launch_gemm_inner_split(hipStream_t st, const float* A, const float* B, float* C, int64_t ld, int64_t M, int64_t N) {
+    hipLaunchKernelGGL(k_gemm_inner_split<S>, dim3((unsigned)(8 * cdiv(cdiv(M, 64) * cdiv(N, 64), 8))), dim3(256), 0, st, A, B,
+                       C, ld, (int)M, (int)N);
+}
+
 // C -= A B with S BF16 pieces per operand on stream st.
 template <int S>
 static void launch_gemm_split(hipStream_t st, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,

@@ -36,7 +36,10 @@ static void gemm_f64(lsx_lu* lu, const double* A, int64_t lda, const double* B, 
 int lu64_getrf(lsx_lu* lu) {
     auto g = [lu](const double* A, int64_t lda, const double* B, int64_t ldb, double* C, int64_t ldc, int64_t M,
                   int64_t N, int64_t K, int mode) { gemm_f64(lu, A, lda, B, ldb, C, ldc, M, N, K, mode); };
-    return getrf_blocked<double>(lu, lu->F, lu->ld, lu->DL, lu->DU, g, g);
+    auto gi = [lu](const double* A, const double* B, double* C, int64_t ld, int64_t M, int64_t N) {
+        launch_gemm_inner<double>(lu, A, B, C, ld, M, N);
+    };
+    return getrf_blocked<double>(lu, lu->F, lu->ld, lu->DL, lu->DU, g, g, gi);
 }
 
 int lu_ensure_work(lsx_lu* lu, int64_t nrhs) {

@@ -60,15 +60,15 @@ static void launch_laswp_t(lsx_lu* lu, T* F, int64_t ld, int kb, const int64_t* 
 
 // Factors F (n x n, ld) in place; pivots into lu->ipiv, row map into lu->perm, diagonal-block
 // inverses into DL / DU.  gemm_upd does the trailing updates (mode 0: C -= A B),
-// gemm_trsm the products of the blocked TRSM (mode 1: C = A B in place, mode 0); both launch on
-// lu->cur.
+// gemm_trsm the products of the blocked TRSM (mode 1: C = A B in place, mode 0), gemm_in a panel's update
+// inside its block (C -= A B, K = PW); all launch on lu->cur.
 //
 // Lookahead: the trailing update of outer block b first updates the columns of block b + 1 on
 // lu->stream, then block b + 1 is factored on lu->stream2 while lu->stream updates the remaining
 // columns.  The row interchanges of a block are applied right of it at once and, when a column
 // segment fits in LDS, left of it (the L columns) in one pass at the end.
-template <typename T, typename GU, typename GT>
-int getrf_blocked(lsx_lu* lu, T* F, int64_t ld, T* DL, T* DU, GU gemm_upd, GT gemm_trsm) {
+template <typename T, typename GU, typename GT, typename GI>
+int getrf_blocked(lsx_lu* lu, T* F, int64_t ld, T* DL, T* DU, GU gemm_upd, GT gemm_trsm, GI gemm_in) {
     lsx_ctx* ctx = lu->ctx;
     const int64_t n = lu->n;
     const hipStream_t s0 = lu->stream_upd ? lu->stream_upd : lu->stream, s1 = lu->stream2;
@@ -125,8 +125,7 @@ int getrf_blocked(lsx_lu* lu, T* F, int64_t ld, T* DL, T* DU, GU gemm_upd, GT ge
                                0, lu->cur, F, ld, n, ji, W, il, ic, jo, (int)nleft, ji + W, jo + jbo, lu->perm);
             lu->prof.end(lu->cur, pi);
             if (nright > 0)
-                launch_gemm_inner<T>(lu, F + ji * ld + ji + W, F + (ji + W) * ld + ji, F + (ji + W) * ld + ji + W, ld,
-                                     n - ji - W, nright);
+                gemm_in(F + ji * ld + ji + W, F + (ji + W) * ld + ji, F + (ji + W) * ld + ji + W, ld, n - ji - W, nright);
         }
         // the interchange lists first: the update stream applies them to the columns right of the
         // block while the diagonal-block inverses are formed

@@ -176,7 +176,15 @@ int mixed_getrf(lsx_lu* lu) {
                    int64_t N, int64_t K, int mode) { gemm_f32(lu, A, lda, B, ldb, C, ldc, M, N, K, mode); };
     auto gu = [lu](const float* A, int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc, int64_t M,
                    int64_t N, int64_t K, int) { gemm_lowp(lu, A, lda, B, ldb, C, ldc, M, N, K); };
-    const int rc = getrf_blocked<float>(lu, lu->F32, lu->ld32, m->DL, m->DU, gu, gt);
+    // updates inside a block: FP32 products for FP32 factors; two BF16 pieces for BF16 factors, as their
+    // other trailing updates (an order up to MTAIL has no others, and would get FP32 factors)
+    auto gi = [lu](const float* A, const float* B, float* C, int64_t ld, int64_t M, int64_t N) {
+        if (lu->dtype != LSX_BF16) return launch_gemm_inner<float>(lu, A, B, C, ld, M, N);
+        const int pi = lu->prof.begin(lu->cur, PK_GEMM_SMALL, 2.0 * M * N * PW, sizeof(float) * 2.0 * M * N);
+        launch_gemm_inner_split<2>(lu->cur, A, B, C, ld, M, N);
+        lu->prof.end(lu->cur, pi);
+    };
+    const int rc = getrf_blocked<float>(lu, lu->F32, lu->ld32, m->DL, m->DU, gu, gt, gi);
     double an = 0.0;
     for (int64_t i = 0; i < nb; ++i) an = nanmax(an, m->hpart[i]);
     m->anorm_h = an;

@@ -82,10 +82,9 @@ struct BatchShared {
     static constexpr int SB = BatchCfg<T>::SB;
     static_assert(BNMAX <= SB * (SB + 1), "the FP32 residual is kept in the solve staging block");
     union {
-        // factor_sys: the panel's LDS and the second panel's U12 / L11 of both panels / staged U12
+        // factor_sys: the panel's LDS and, behind it, the second panel's U12 / L11 of both panels / staged U12
         __align__(16) T wide[UCH * ust<T>()];
-        double dblk[SB][SB + 1];   // staged diagonal block of the solves / FP32 path: the residual /
-                                   // during the factorization, L11 of a panel without held L21
+        double dblk[SB][SB + 1];   // staged diagonal block of the solves / FP32 path: the residual
     };
     double red[2][BT / 64];
     int info;                  // 1 + the first column whose pivot is zero

@@ -172,8 +172,9 @@ static void launch_gemm(hipStream_t st, const T* A, int64_t lda, const T* B, int
 // its outer block, on the chain of the panels, where the time is latency and not rate.  A 64 x 64 tile per
 // workgroup, four waves of 32 x 32, and every load of a tile (A, B and C) issued before the first is
 // waited for; the staged kernel above has three dependent round trips at K = 32.  FP32 factors take FP32
-// products and sums here too (BF16 factors: k_gemm_inner_split).  n = 3001 9.07 -> 8.91 ms, 1024 1.80 -> 1.78; mixed, against the split-BF16
-// kernel (128 x 128 tiles, 12 to 15 us), n = 3000 7.87 -> 7.55, 9000 33.7 -> 32.9.
+// products and sums here too (BF16 factors: k_gemm_inner_split).  Factor + one solve against that kernel:
+// n = 1024 1.82 -> 1.78 ms, 3001 9.37 -> 9.21; mixed, against the split-BF16 kernel (128 x 128 tiles, 12 to
+// 15 us), n = 2000 4.27 -> 4.10, 3000 7.95 -> 7.62, 9000 34.2 -> 33.2.
 constexpr int IBK = 32, IBM = 64;
 template <typename T>
 __global__ __launch_bounds__(256) void k_gemm_inner(const T* __restrict Ag, const T* Bg, T* Cg, int64_t ld, int M, int N) {

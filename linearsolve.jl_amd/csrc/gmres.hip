@@ -81,8 +81,11 @@ __global__ void k_spmv(int64_t N, const int32_t* __restrict rowptr, const int32_
 // the same from a few workgroups to GMRES_WIDE of them, while everything else shrinks with the rows
 // of a workgroup, so a solve takes the fewest rows per thread that keep it within a bound of
 // workgroups.  The bounds grow with the rows: up to GALL workgroups the products take one message
-// round instead of two.  GMRES_WIDE keeps every solve inside the serving lanes' share of the CUs, so
-// a solve has the same shape, and the same bits, in every launch form.
+// round instead of two.  GMRES(30), us a step: with 16 for the first bound 110^2 14.8 instead of 13.0;
+// with 32 for the second 230^2 20.1 instead of 17.1; with 64 for the third 512^2 44.4 instead of 23.7, for
+// the fourth 600^2 80.6 instead of 46.7.  Wider ones: 64 first 160^2 14.8 instead of 15.4 (and twice the CUs),
+// 128 second 300^2 17.6 instead of 21.3.  GMRES_WIDE keeps every solve inside the serving lanes' share of
+// the CUs, so a solve has the same shape, and the same bits, in every launch form.
 constexpr int GMRES_WIDE = 128;
 static void pick_shape(int64_t N, bool one_wg, GmresPlan* out) {
     out->nt = N <= 256 ? 256 : 1024;
@@ -106,11 +109,12 @@ int csr_spmv_dev(lsx_csr* A, const double* dx, double* dy, hipStream_t st) {
 constexpr size_t GMRES_LDS_MAX = 149 * 1024;  // dynamic LDS of a workgroup (160 KB less the static part)
 
 // The largest Krylov dimension of one solve: GMRES_MAX_CAP_G (bookkeeping in HBM where the LDS does
-// not hold it); with hbm false (the multi-solve launches) 128, and less for matrices whose
-// workgroups have many rows.
+// not hold it); with hbm false (the multi-solve launches) GMRES_MAX_CAP, and less above 2048 rows of a
+// workgroup.  That second limit is what the entry points have always accepted; gmres_plan holds every
+// dimension up to GMRES_MAX_CAP in LDS.
 int gmres_cap_limit(int64_t N, bool hbm) {
     if (hbm) return GMRES_MAX_CAP_G;
-    int64_t rows = 8192;  // LDS rows (two doubles each) set aside beside R, the Givens pairs and z
+    int64_t rows = 8192;  // rows of a workgroup, at two doubles each beside cap (cap + 1) / 2 + 3 cap + 1
     if (N <= 512) rows = 512;
     else if (N <= 2048 || (N > 8192 && cdiv(N, 2048) <= GMRES_WIDE)) rows = 2048;
     else if (N > 8192 && cdiv(N, 4096) <= GMRES_WIDE) rows = 4096;

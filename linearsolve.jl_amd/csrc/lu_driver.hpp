@@ -3,7 +3,8 @@
 // for the plain path, FP32 or BF16 MFMA for the mixed path).
 //
 // Structure of LAPACK dgetrf and of src/blocked_lufact.jl:658-679, with two block levels:
-// outer blocks of NBO to 4 NBO columns (K of the trailing update; the last one wider) split into inner panels of PW columns.
+// outer blocks of NBO to 4 NBO columns (K of the trailing update; the last one wider) split into inner
+// panels of PW columns.
 #pragma once
 #include <algorithm>
 
@@ -41,8 +42,8 @@ static void launch_panel_t(lsx_lu* lu, T* F, int64_t ld, int64_t j0, int W, int6
     else if (sizeof(T) == 8 || m_rows <= 1024 || m_rows > 2048)
         hipLaunchKernelGGL((k_panel<T, 512, 2>), dim3(a.P), dim3(512), 0, lu->cur, a);
     else if constexpr (sizeof(T) == 4) {
-        // FP32 rows leave the registers for 2048 rows in one workgroup: still no exchange (n = 2000 with
-        // its refinement 5.26 -> 4.54 ms); two or more such workgroups are slower than twice as many of 1024
+        // FP32 rows leave the registers for 2048 rows in one workgroup: still no exchange (with refinement,
+        // n = 2000 5.08 -> 4.10 ms, 9000 34.4 -> 33.2); two or more such workgroups are slower than twice as many of 1024
         a.P = 1;
         hipLaunchKernelGGL((k_panel<T, 1024, 2>), dim3(1), dim3(1024), 0, lu->cur, a);
     }
@@ -93,13 +94,15 @@ int getrf_blocked(lsx_lu* lu, T* F, int64_t ld, T* DL, T* DU, GU gemm_upd, GT ge
     //   m <= MTAIL: all the columns left are one block, every panel updating all of them (K = PW), on
     //     every CU.  The trailing matrix is then small enough for its update to take 5 to 20 us a panel,
     //     and a block of NBO would spend 110 us between its last panel and the next block's first (lists,
-    //     interchanges and TRSM of the next columns, inverses).  n = 500 1044 -> 835 us, 1024 2316 -> 1815,
-    //     3001 10.2 -> 9.2 ms, 16384 (limit 1024 -> 3072) 101.2 -> 100.5; a limit of 4096 gives nothing more;
+    //     interchanges and TRSM of the next columns, inverses).  Factor + one solve without and with it:
+    //     n = 500 1.12 -> 0.82 ms, 1024 2.39 -> 1.78, 3001 10.3 -> 9.2, 16384 99.8 -> 98.5; a limit of 1024
+    //     gives 9.7 at 3001, one of 4096 22.3 against 21.8 at 6000;
     //   m > MWIDE: 2 NBO columns, so that the trailing matrix is read and written half as often, where
-    //     its update and not the panels' chain is the longer of the two: n = 16384 109.8 -> 100.6 ms, 12000
-    //     58.2 -> 55.8, 9000 no change (limits of 7000 to 8192 measure the same, 11000 gives 102.2 and 57.6);
-    //     in FP64 4 NBO above MWIDE4 (16384 100.6 -> 98.1 ms, 12000 no change; FP32's shorter updates lose
-    //     to the longer inner ones: mixed 14000 58.1 -> 59.2);
+    //     its update and not the panels' chain is the longer of the two: n = 16384 110.0 -> 100.6 ms, 12000
+    //     58.4 -> 55.5, 9000 no change; in FP64 4 NBO above MWIDE4: 13000 64.8 -> 64.6, 14000 73.6 -> 72.7,
+    //     15000 83.6 -> 82.1, 16384 100.6 -> 98.3 (10300 to 11000 lose 1.3 %; limits of 11000, 12000 and 13500
+    //     take 0.3 to 2 % back from 13000 to 16384; FP32's shorter updates lose to the longer inner ones:
+    //     mixed 14000 58.1 -> 59.2);
     //   else NBO.
     auto width = [&](int64_t jo) -> int {
         const int64_t m = n - jo;

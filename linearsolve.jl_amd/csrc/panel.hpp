@@ -101,8 +101,8 @@ struct PanelLds {
 };
 
 // v: the rows (panel column q in slot q); lr, live: their labels (logical rows, j0 ..) and whether they
-// may still become a pivot; W columns; labels lie in [j0, m).  exchange(win, column, parity, groups of
-// live slots) turns the workgroup's winning record into the panel's (itself with one workgroup).
+// may still become a pivot; W columns; labels lie in [j0, m).  exchange(rec, column, sender) turns the
+// workgroup's winning record (written by the wave whose sender is true) into the panel's, past a barrier.
 // piv[c] (LDS): the logical row interchanged with row j0 + c; info: 1 + the first column (from 0, in the
 // matrix) whose pivot is zero, if it was 0.  On return row lr is row j0 + i (i < W): its columns are
 // fin[i] (LDS, after a barrier); of the other rows slot q holds column (q + 8 ceil(W / 8)) mod PW.

@@ -88,7 +88,8 @@ int lsx_lu_destroy(lsx_lu* lu);
 
 /* getrf: copies A (host or device, lda >= n) into the handle and factors it.
  * Replaces lu(A, check=false) / LAPACK.getrf!(factors, ipiv) at src/factorization.jl:689-697
- * (ccall path src/openblas.jl:144-151).  Returns info (> 0: first zero pivot, as LAPACK). */
+ * (ccall path src/openblas.jl:144-151).  Returns info (> 0: first zero pivot, as LAPACK;
+ * LSX_F32 / LSX_BF16: first pivot that is zero, NaN or without an FP32 reciprocal). */
 int lsx_lu_factor(lsx_lu* lu, const double* A, int64_t lda);
 
 /* Copies the resident factors (L unit-lower below the diagonal, U on and above) and the

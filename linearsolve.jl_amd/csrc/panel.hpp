@@ -104,7 +104,7 @@ struct PanelLds {
 // may still become a pivot; W columns; labels lie in [j0, m).  exchange(rec, column, sender) turns the
 // workgroup's winning record (written by the wave whose sender is true) into the panel's, past a barrier.
 // piv[c] (LDS): the logical row interchanged with row j0 + c; info: 1 + the first column (from 0, in the
-// matrix) whose pivot is zero, if it was 0.  On return row lr is row j0 + i (i < W): its columns are
+// matrix) whose pivot is zero (FP32 without FEW: zero, NaN or without a reciprocal), if it was 0.  On return row lr is row j0 + i (i < W): its columns are
 // fin[i] (LDS, after a barrier); of the other rows slot q holds column (q + 8 ceil(W / 8)) mod PW.
 // FEW (one workgroup): panels may have far fewer rows than NT RPT and fewer than PW columns, and other
 // workgroups of the CU use what the waves without rows leave: those only take part in the barriers, a
@@ -196,7 +196,10 @@ __device__ __forceinline__ void panel_columns(T (&v)[RPT][PW], int (&lr)[RPT], b
             // it is replaced by k so that every later row index stays inside the matrix.
             if (grow < k || grow >= m) grow = k;
             if (tid == 0) sh.piv[col] = grow;
-            if (pv == T(0) && info == 0) info = k + 1;
+            // FP32 factors to be refined (not FEW): neither a NaN pivot nor one without an FP32 reciprocal
+            // (the matrix is not finite, or out of FP32's range) gives factors to refine with
+            const bool bad = sizeof(T) == 4 && !FEW ? !(fabs(inv) <= std::numeric_limits<T>::max()) : pv == T(0);
+            if (bad && info == 0) info = k + 1;
             const bool normal = fabs(pv) >= std::numeric_limits<T>::min();
             T nl[RPT];
 #pragma unroll

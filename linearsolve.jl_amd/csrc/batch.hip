@@ -369,13 +369,14 @@ __device__ __forceinline__ void swap_solve(BatchShared<T>& sh, T* A, const doubl
 // src: the matrix where the caller has it, read by the first step (so no copy is made first).
 // 20,000 systems of n in [8, 512], FP64: 58.2 -> 39.1 ms against one update per 32-column panel (8
 // or 16 columns below n = 192), panels with two barriers and two rows through LDS per column, and a
-// copy of the matrices first; of the time 31 % is the panels', 28 % the trailing updates', 13 % the
-// solves', 12 % U12's.  3,000 systems, FP32 factors: 11.2 -> 8.9 ms.
+// copy of the matrices first.  3,000 systems, FP32 factors: 11.2 -> 8.9 ms.
 // Small systems leave most of a panel's waves without rows, and a branch per column between the loads of
 // a panel (with a spilled address each) made every load wait for the one before it.  With those waves
 // waiting at the barriers only, no barriers in panels of one wave, and branch-free loads by 32-bit offsets
 // (el): 20,000 FP64 systems of n = 1 0.65 -> 0.45 ms, of 8 to 16 1.25 -> 0.83; FP32 of 33 to 64 5.3 -> 3.3,
-// 3,000 FP32 systems of 8 to 512 8.9 -> 6.7, 20,000 50.6 -> 36.8; FP64 of 8 to 512 39.2 -> 38.8.
+// 3,000 FP32 systems of 8 to 512 8.9 -> 6.7, 20,000 50.6 -> 36.8; FP64 of 8 to 512 39.2 -> 38.8.  Of the
+// time of 20,000 systems, FP64 (FP32): panels 30 (23) %, trailing updates 29 (27), solves 21 (9), U12 16
+// (11), the L columns' gather 3 (2), FP32's refinement 28.
 template <typename T>
 __device__ __forceinline__ void factor_sys(BatchShared<T>& sh, T* A, const double* src, int n, int64_t vo, int64_t* ipiv,
                                            int64_t& info) {
